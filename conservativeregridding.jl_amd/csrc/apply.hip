@@ -13,12 +13,13 @@
 //   k_apply_rows<T,FB>  one thread per row; blockIdx.y = block of FB fields,
 //                       the slowest launch dimension; XCD-contiguous row tiles
 //   k_apply_long<T,FB>  rows with more than kLongRow non-zeros, one wave each
-//   k_apply_fieldsfast  FP32 fields with field stride 1: one wave per row,
-//                       lanes across fields, fully coalesced
+//   k_levels<T,V>       (levels.hip) fields with field stride 1: a row's fields
+//                       across neighbouring lanes, coalesced without staging
 // FP64 fields accumulate in FP64 (fused multiply-add) and divide by the area
-// like finalize_regridding!.  FP32 fields use the FP64 A rounded to FP32 once
-// per non-zero and field block, FP32 products, FP32 Kahan-compensated row
-// sums, and a final scale by the FP64 reciprocal area.
+// like finalize_regridding!.  FP32 fields in the row kernels use the FP64 A
+// rounded to FP32 once per non-zero and field block, FP32 products, FP32
+// Kahan-compensated row sums, and a final scale by the FP64 reciprocal area;
+// levels.hip and the default tile kernel multiply and sum in FP64.
 #include <algorithm>
 #include <vector>
 
@@ -154,42 +155,23 @@ __global__ void __launch_bounds__(64) k_apply_long(
     }
 }
 
-// ---- FP32, fields fastest (field stride 1) ----------------------------------------
-// One wave per row; lane l owns fields l, l+64, ... (up to kFieldRegs per lane).
-constexpr int kFieldRegs = 4;
-
-__global__ void __launch_bounds__(256) k_apply_fieldsfast(
-    const int64_t *__restrict__ rowptr, const int32_t *__restrict__ col,
-    const double *__restrict__ val, int64_t nrows, const float *__restrict__ x, int64_t xc,
-    float *__restrict__ y, int64_t yc, int64_t nfields, const double *__restrict__ inv_area) {
-    int64_t row = (int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
-    int lane = threadIdx.x & 63;
-    if (row >= nrows) return;
-    int64_t k0 = rowptr[row], k1 = rowptr[row + 1];
-    for (int64_t f0 = 0; f0 < nfields; f0 += 64 * kFieldRegs) {
-        Acc<float> acc[kFieldRegs];
-#pragma unroll
-        for (int j = 0; j < kFieldRegs; ++j) acc[j].init();
-        for (int64_t k = k0; k < k1; ++k) {
-            const float *xr = x + (int64_t)col[k] * xc;
-            float v = (float)val[k];
-#pragma unroll
-            for (int j = 0; j < kFieldRegs; ++j) {
-                int64_t f = f0 + lane + 64 * j;
-                if (f < nfields) acc[j].add(v, xr[f]);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < kFieldRegs; ++j) {
-            int64_t f = f0 + lane + 64 * j;
-            if (f < nfields) y[row * yc + f] = acc[j].finish(nullptr, inv_area, row);
-        }
-    }
-}
-
-__global__ void k_inv(const double *__restrict__ a, int64_t n, double *__restrict__ inv) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) inv[i] = 1.0 / a[i];
+// Reciprocal areas and the list of wide rows of both directions; thread i takes
+// row i of A, then of A^T.
+struct FinishDir {
+    const double *area;
+    double *inv;
+    const int64_t *rowptr;
+    int64_t n;
+    int32_t *wide, *nwide;
+};
+__global__ void k_zero_counts(int32_t *n) { n[threadIdx.x] = 0; }
+__global__ void k_finish(FinishDir f, FinishDir b) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const FinishDir &d = t < f.n ? f : b;
+    const int64_t i = t < f.n ? t : t - f.n;
+    if (i >= d.n) return;
+    d.inv[i] = 1.0 / d.area[i];
+    if (d.rowptr[i + 1] - d.rowptr[i] > kWideRow) d.wide[atomicAdd(d.nwide, 1)] = (int32_t)i;
 }
 
 // Rows with more than kLongRow non-zeros, appended in any order (each long row
@@ -227,12 +209,26 @@ static void ensure_long_rows(const Csr &A, hipStream_t s) {
 }
 
 void finalize_regridder(cr_regridder *R, hipStream_t s) {
-    R->fwd.inv_area.alloc_kept(R->fwd.nrows, s);
-    R->bwd.inv_area.alloc_kept(R->bwd.nrows, s);
-    hipLaunchKernelGGL(k_inv, dim3(grid_for(R->fwd.nrows, 256)), dim3(256), 0, s, R->a_dst.p,
-                       R->fwd.nrows, R->fwd.inv_area.p);
-    hipLaunchKernelGGL(k_inv, dim3(grid_for(R->bwd.nrows, 256)), dim3(256), 0, s, R->a_src.p,
-                       R->bwd.nrows, R->bwd.inv_area.p);
+    // one buffer: both directions' reciprocal areas, the two counters, the two lists
+    int64_t n[2], cap[2];
+    for (int t = 0; t < 2; ++t) {
+        Csr &A = t ? R->bwd : R->fwd;
+        n[t] = A.nrows;
+        cap[t] = A.wide_cap = std::min<int64_t>(A.nrows, A.nnz / (kWideRow + 1));
+    }
+    R->finish.alloc_kept(n[0] + n[1] + 1 + (cap[0] + cap[1] + 1) / 2, s);
+    int32_t *count = (int32_t *)(R->finish.p + n[0] + n[1]);
+    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(2), 0, s, count);
+    FinishDir dir[2];
+    for (int t = 0; t < 2; ++t) {
+        Csr &A = t ? R->bwd : R->fwd;
+        dir[t] = {t ? R->a_src.p : R->a_dst.p, R->finish.p + (t ? n[0] : 0), A.rowptr.p, n[t],
+                  count + 2 + (t ? cap[0] : 0), count + t};
+        A.inv_area = dir[t].inv;
+        A.wide = dir[t].wide;
+        A.nwide = dir[t].nwide;
+    }
+    hipLaunchKernelGGL(k_finish, dim3(grid_for(n[0] + n[1], 256)), dim3(256), 0, s, dir[0], dir[1]);
     CR_HIP(hipGetLastError());
 }
 
@@ -261,6 +257,23 @@ void launch_tiles(const TilePlan &P, int F, int acc, int nchunks, int chunk_majo
                   int64_t sf, T *y, int64_t dc, int64_t df, int64_t nf, const double *scale, int64_t nrows,
                   int64_t ncols, hipStream_t s);
 
+// Fields stored side by side per cell (levels.hip).
+void launch_levels(const Csr &A, const float *x, int64_t xc, float *y, int64_t yc, int64_t nf, const double *scale,
+                   hipStream_t s);
+void launch_levels(const Csr &A, const TilePlan &P, const double *x, int64_t xc, double *y, int64_t yc, int64_t nf,
+                   const double *scale, hipStream_t s);
+
+template <class T>
+static void launch_huge(const Csr &A, const TilePlan &P, const T *x, int64_t sc, int64_t sf, T *y, int64_t dc,
+                        int64_t df, int64_t nf, const double *area, const double *inv, hipStream_t s) {
+    if (!P.nhuge) return;
+    constexpr int FB = sizeof(T) == 4 ? 8 : 1;
+    const int64_t gy = (nf + FB - 1) / FB;
+    CR_REQUIRE(gy <= 65535, CR_UNSUPPORTED, "too many fields for one launch");
+    hipLaunchKernelGGL((k_apply_long<T, FB>), dim3((unsigned)P.nhuge, (unsigned)gy), dim3(64), 0, s, P.huge.p,
+                       A.rowptr.p, A.col.p, A.val.p, x, sc, sf, y, dc, df, nf, area, inv);
+}
+
 template <class T>
 static void launch_tiled(const Csr &A, int geom, int F, int acc, int nchunks, int chunk_major, const T *x,
                          int64_t sc, int64_t sf, T *y, int64_t dc, int64_t df, int64_t nf, const double *area,
@@ -269,13 +282,7 @@ static void launch_tiled(const Csr &A, int geom, int F, int acc, int nchunks, in
     const TilePlan &P = tile_plan(A, f32 ? kRounds : kEven, geom, s, blocks);
     launch_tiles<T>(P, F, acc, nchunks, chunk_major, x, sc, sf, y, dc, df, nf, f32 ? inv : area, A.nrows,
                     A.ncols, s);
-    if (P.nhuge) {
-        constexpr int FB = f32 ? 8 : 1;
-        const int64_t gy = (nf + FB - 1) / FB;
-        CR_REQUIRE(gy <= 65535, CR_UNSUPPORTED, "too many fields for one launch");
-        hipLaunchKernelGGL((k_apply_long<T, FB>), dim3((unsigned)P.nhuge, (unsigned)gy), dim3(64), 0, s,
-                           P.huge.p, A.rowptr.p, A.col.p, A.val.p, x, sc, sf, y, dc, df, nf, area, inv);
-    }
+    launch_huge<T>(A, P, x, sc, sf, y, dc, df, nf, area, inv, s);
 }
 
 // FP32 kernel variants the autotuner tries (index = variant): the row kernel
@@ -345,10 +352,23 @@ static void launch_f32_variant(int v, const Csr &A, const float *x, int64_t sc, 
 constexpr int kNumF64Variants = 2;  // 0 row kernel, 1 tile kernel
 constexpr int kDefaultF64Variant = 1;
 
-// Kernel choice: FP64 -> the tile kernel (1 or 2 fields per stage) unless the
-// row kernel is pinned; FP32 with unit field strides and many fields ->
-// fields-fastest kernel; other FP32 layouts -> the autotuned (or pinned, or
-// default: 1024-row tiles, 4 fields per stage, FP64 sums) variant.
+// Whether a call goes to the kernel for fields side by side: field stride 1 on
+// both sides and enough fields for the matrix's rows.  Measured against the
+// tile kernel, which gathers one field at a time (us, this kernel / tile):
+// 5.5 non-zeros a row, FP32 k = 4: 42 / 29, 6: 39 / 52, 50: 136 / 1638; FP64
+// k = 4: 50 / 48, 6: 56 / 101.  43 a row, FP32 k = 12: 42 / 35, 16: 28 / 56;
+// FP64 k = 6: 41 / 28, 11: 46 / 68.  26 a row, FP32 k = 12: 44 / 38, 16: 24 / 65.
+static bool levels_layout(const Csr &A, int dtype, int64_t nf, int64_t sf, int64_t df) {
+    if (sf != 1 || df != 1) return false;
+    const int64_t mean = A.nnz / std::max<int64_t>(1, A.nrows);
+    if (dtype == CR_F64) return A.f64_variant < 0 && nf >= std::max<int64_t>(6, std::min<int64_t>(16, mean / 4));
+    return nf >= 64 || (A.tuned_variant < 0 && nf >= (mean <= 8 ? 6 : 16));
+}
+
+// Kernel choice: fields side by side -> levels.hip; other FP64 layouts -> the
+// tile kernel (1 or 2 fields per stage) unless the row kernel is pinned; other
+// FP32 layouts -> the autotuned (or pinned, or default: 1024-row tiles, 4
+// fields per stage, FP64 sums) variant.
 void apply(const cr_regridder *R, bool transpose, int dtype, int64_t nf, const void *src,
            int64_t sc, int64_t sf, void *dst, int64_t dc, int64_t df, bool normalize, hipStream_t s,
            int force_variant = -1) {
@@ -360,20 +380,22 @@ void apply(const cr_regridder *R, bool transpose, int dtype, int64_t nf, const v
         double *y = (double *)dst;
         const double *ar = normalize ? area : nullptr;
         const int v = A.f64_variant >= 0 ? A.f64_variant : kDefaultF64Variant;
-        if (v == 1)
+        if (levels_layout(A, dtype, nf, sf, df)) {
+            const TilePlan &P = tile_plan(A, kEven, kGeomS, s, false);
+            launch_levels(A, P, x, sc, y, dc, nf, ar, s);
+            launch_huge<double>(A, P, x, sc, sf, y, dc, df, nf, ar, nullptr, s);
+        } else if (v == 1)
             launch_tiled<double>(A, kGeomS, nf >= 2 ? 2 : 1, false, 0, 0, x, sc, sf, y, dc, df, nf, ar, nullptr,
                                  s);
         else if (nf == 1) launch_rows<double, 1>(A, x, sc, sf, y, dc, df, nf, ar, nullptr, s);
         else launch_rows<double, 8>(A, x, sc, sf, y, dc, df, nf, ar, nullptr, s);
-    } else if (sf == 1 && df == 1 && nf >= 64 && force_variant < 0) {
-        hipLaunchKernelGGL(k_apply_fieldsfast, dim3(grid_for(A.nrows, 4)), dim3(256), 0, s, A.rowptr.p,
-                           A.col.p, A.val.p, A.nrows, (const float *)src, sc, (float *)dst, dc, nf,
-                           normalize ? A.inv_area.p : nullptr);
+    } else if (force_variant < 0 && levels_layout(A, dtype, nf, sf, df)) {
+        launch_levels(A, (const float *)src, sc, (float *)dst, dc, nf, normalize ? A.inv_area : nullptr, s);
     } else {
         int v = force_variant >= 0 ? force_variant : A.tuned_variant;
         if (v < 0 || v >= kNumVariants) v = default_f32_variant(A, s);
         launch_f32_variant(v, A, (const float *)src, sc, sf, (float *)dst, dc, df, nf,
-                           normalize ? A.inv_area.p : nullptr, s);
+                           normalize ? A.inv_area : nullptr, s);
     }
     CR_HIP(hipGetLastError());
 }
@@ -391,7 +413,7 @@ bool apply_ready(const cr_regridder *R, bool transpose, int dtype, int64_t nf, i
         const int v = A.f64_variant >= 0 ? A.f64_variant : kDefaultF64Variant;
         return v == 1 ? plan_ready(A, kEven, kGeomS, false) : long_rows_ready();
     }
-    if (sf == 1 && df == 1 && nf >= 64) return true;
+    if (levels_layout(A, dtype, nf, sf, df)) return true;
     int v = A.tuned_variant;
     if (v < 0 || v >= kNumVariants) {
         v = A.default_variant.load();
@@ -417,7 +439,7 @@ void prepare(const cr_regridder *R, bool transpose, int dtype, int64_t nf, int64
         } else {
             ensure_long_rows(A, s);
         }
-    } else if (!(sf == 1 && df == 1 && nf >= 64)) {
+    } else if (!levels_layout(A, dtype, nf, sf, df)) {
         int v = A.tuned_variant;
         if (v < 0 || v >= kNumVariants) v = default_f32_variant(A, s);
         const F32Variant &V = kF32Variants[v];

@@ -40,12 +40,18 @@ struct TilePlan {
     int64_t tile_cols = 0, tile_lines = 0;
 };
 
+constexpr int kWideRow = 32;
+
 struct Csr {
     int64_t nrows = 0, ncols = 0, nnz = 0;
     DevBuf<int64_t> rowptr;
     DevBuf<int32_t> col;
     DevBuf<double> val;
-    DevBuf<double> inv_area;   // 1 / area of the row cells (FP32 batched path)
+    // in the regridder's `finish` buffer: 1 / area of the row cells (FP32 fields);
+    // the rows with more than kWideRow non-zeros, in any order, and their number
+    const double *inv_area = nullptr;
+    const int32_t *wide = nullptr, *nwide = nullptr;
+    int64_t wide_cap = 0;  // places in the list
     int tuned_variant = -1;    // FP32 kernel variant (cr_regrid_tune / set_variant); -1: default
     mutable std::atomic<int> default_variant{-1};  // the default FP32 variant chosen for this matrix; -1: not yet
     int f64_variant = -1;      // FP64 kernel variant; -1: default
@@ -73,6 +79,7 @@ struct cr_regridder {
     cr::Csr fwd;  // A:   n_dst x n_src
     cr::Csr bwd;  // A^T: n_src x n_dst
     cr::DevBuf<double> a_dst, a_src;
+    cr::DevBuf<double> finish;  // what finalize_regridder derives from the CSR arrays and the areas
     cr_build_stats stats{};
     // stored areas = area_scale * unit-sphere areas (radius^2, divided by max(A)
     // after normalize!); 0 when built from arrays (no geometry: no vertex gradients)

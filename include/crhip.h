@@ -375,9 +375,13 @@ cr_status cr_regrid_tune(cr_regridder *R, int32_t transpose, int64_t nfields, co
  *           bytes.  The default is 15 (A used in FP64), or 28 when 15's tiles
  *           fetch over 3 source lines per 32 distinct source cells and 28's
  *           fetch fewer (decided once per direction at its first default
- *           apply).  FP32 fields with unit field strides and >= 64 fields
- *           always use the fields-fastest kernel.
- *   CR_F64: 0 row kernel, 1 staged tile kernel (default).
+ *           apply).  Fields side by side (unit field strides) have a kernel
+ *           of their own: FP32 with >= 64 fields always, with fewer (>= 6, or
+ *           16 where rows have more than 8 non-zeros on average) unless a
+ *           variant is pinned or tuned; FP64 sums of the FP64 A, no plan.
+ *   CR_F64: 0 row kernel, 1 staged tile kernel (default; unit field strides
+ *           and >= 6 fields, more for long rows: the side-by-side kernel, with
+ *           the tile kernel's plan and results).
  */
 int32_t cr_regrid_variant_count(int32_t dtype);
 cr_status cr_regrid_set_variant(cr_regridder *R, int32_t transpose, int32_t dtype, int32_t variant);
