@@ -69,65 +69,57 @@ inline bool stream_capturing(hipStream_t s) {
                std::string(what) + " is not made yet and cannot be made during stream capture: call "   \
                                    "cr_regrid_prepare (or one cr_regrid) with the same arguments first")
 
-// Device memory.  DevBuf(n) uses hipMalloc (long-lived buffers owned by a
-// handle); DevBuf(n, stream) takes stream-ordered memory from the device's
-// default pool (build temporaries), which keeps freed blocks for the next
-// build instead of returning them to the driver.
-void configure_pool();
+// Device memory (memory.hip keeps freed blocks for the next allocation).
+// device_alloc: first used in order on stream s, or (ordered false) on any
+// stream; device_free: every use in order on stream s, or unknown.
+void *device_alloc(size_t bytes, bool ordered, hipStream_t s);
+void device_free(void *p, bool ordered, hipStream_t s);
 
+// DevBuf(n): memory for any stream (buffers of grids); DevBuf(n, stream): a
+// temporary, used and freed in order on its stream; alloc_kept(n, stream):
+// owned by a handle, filled on `stream`, afterwards used on any stream.
 template <class T>
 struct DevBuf {
     T *p = nullptr;
     size_t n = 0;
     hipStream_t st = nullptr;
-    bool pooled = false;
+    bool ordered = false;  // freed in order on st
     DevBuf() = default;
     explicit DevBuf(size_t count) { alloc(count); }
     DevBuf(size_t count, hipStream_t s) { alloc_async(count, s); }
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    DevBuf(DevBuf &&o) noexcept : p(o.p), n(o.n), st(o.st), pooled(o.pooled) {
+    DevBuf(DevBuf &&o) noexcept : p(o.p), n(o.n), st(o.st), ordered(o.ordered) {
         o.p = nullptr;
         o.n = 0;
     }
     DevBuf &operator=(DevBuf &&o) noexcept {
         if (this != &o) {
             release();
-            p = o.p; n = o.n; st = o.st; pooled = o.pooled;
+            p = o.p; n = o.n; st = o.st; ordered = o.ordered;
             o.p = nullptr; o.n = 0;
         }
         return *this;
     }
     ~DevBuf() { release(); }
-    void alloc(size_t count) {
-        release();
-        n = count;
-        pooled = false;
-        if (count) CR_HIP(hipMalloc(&p, count * sizeof(T)));
-    }
-    void alloc_async(size_t count, hipStream_t s) {
-        release();
-        n = count;
-        st = s;
-        pooled = true;
-        configure_pool();
-        if (count) CR_HIP(hipMallocAsync((void **)&p, count * sizeof(T), s));
-    }
-    // Pool memory that outlives the call that allocated it (owned by a handle):
-    // allocated in order on `s`, released on the null stream.
-    void alloc_kept(size_t count, hipStream_t s) {
-        alloc_async(count, s);
-        st = nullptr;
-    }
+    void alloc(size_t count) { get(count, false, false, nullptr); }
+    void alloc_async(size_t count, hipStream_t s) { get(count, true, true, s); }
+    void alloc_kept(size_t count, hipStream_t s) { get(count, true, false, s); }
     void release() {
-        if (p) {
-            if (pooled) (void)hipFreeAsync(p, st);
-            else (void)hipFree(p);
-        }
+        device_free(p, ordered, st);
         p = nullptr;
         n = 0;
     }
     size_t bytes() const { return n * sizeof(T); }
+
+  private:
+    void get(size_t count, bool first_on_s, bool freed_on_s, hipStream_t s) {
+        release();
+        st = s;
+        ordered = freed_on_s;
+        if (count) p = (T *)device_alloc(count * sizeof(T), first_on_s, s);
+        n = count;
+    }
 };
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
