@@ -7,14 +7,18 @@
 //      a stable radix sort of the non-zeros by column.  A tile that starts at
 //      row s counts, for each row, the non-zeros with prev[k] < s as new
 //      distinct columns, which is the greedy column budget's count.
-//   2. k_plan_table: for every start row s on the kRowAlign grid, the tile a
-//      greedy pass from s makes (one workgroup per start: per-row counts, a
-//      block scan, the first row that breaks a budget): end, column capacity,
-//      slots per thread.
-//   3. k_plan_walk: one workgroup follows the chain 0 -> end(0) -> ... through
-//      that table (held in LDS in chunks).  A start off the grid (after a tile
-//      shorter than kRowAlign rows) is evaluated in place.  Running sums give
-//      every tile its first slot and first column.
+//   2. k_plan_table: for every start row s on the kRowAlign grid, the tiles a
+//      greedy pass makes from s to the next row on the grid where a tile ends:
+//      one tile, or up to kRowAlign where rows are so long that tiles end
+//      between grid rows (one workgroup per start: per-row counts, a block scan,
+//      the first row that breaks a budget).
+//   3. the chain 0 -> end(0) -> ... through that table, in chunks of kChunk
+//      starts: k_plan_chunk gives every start the row where the chain leaves its
+//      chunk and the tiles, slots and columns on the way (pointer doubling in
+//      LDS); k_plan_emit, a workgroup per chunk, follows the chunk exits from
+//      row 0 to its own chunk and writes the records of the tiles there.  (One
+//      workgroup chasing the whole chain, tiles off the grid evaluated in place,
+//      took 1480 us of the quarter-degree forward plan, 300 us transposed.)
 //   4. one readback of the totals, the plan's buffers allocated;
 //   5. k_plan_fill: one workgroup per tile: the distinct columns (block radix
 //      sort of the tile's column indices), the pieces and their rounds
@@ -24,6 +28,8 @@
 //
 // The huge rows (more than kCols non-zeros) are listed by a flag scan.  The
 // device-wide sort and scan come from build.hip (sort_pairs, exclusive_sum).
+#include <climits>
+
 #include <rocprim/block/block_radix_sort.hpp>
 
 #include "regridder.hpp"
@@ -32,8 +38,9 @@ namespace cr {
 
 namespace {
 
-constexpr int kPlanThreads = 256;  // workgroup of the table and walk kernels
-constexpr int kWalkChunk = 8192;   // table entries the walk holds in LDS
+constexpr int kPlanThreads = 256;  // workgroup of the table and chain kernels
+constexpr int kChunk = 1024;       // start rows on the grid per chunk of the chain
+constexpr int kShortRow = 32;      // longer rows are counted by a whole wave
 
 struct TileRec {  // a tile found by the walk
     int64_t row0, ent_off, col_off;
@@ -115,31 +122,57 @@ __device__ WindowTile window_tile(int64_t s, int64_t nrows, const int64_t *__res
     uint32_t tot[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) tot[c] = 0u;
+    const int64_t kfirst = rp[s];
+    int off[RPT], len[RPT];  // first non-zero from kfirst, non-zeros
+    uint32_t nu[RPT];        // new columns
+    bool any_huge = false;
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
         const int64_t r = s + tid * RPT + i;
+        off[i] = len[i] = 0;
+        nu[i] = 0u;
+        live[i] = false;
+        if (r < nrows) {
+            const int64_t k0 = rp[r], n = rp[r + 1] - k0;
+            live[i] = n <= G::kCols;
+            any_huge |= !live[i];
+            off[i] = (int)(k0 - kfirst);
+            len[i] = live[i] ? (int)n : 0;
+        }
+    }
+    // rows past the slots' budget fail whatever their columns: not counted
+    const int most = __syncthreads_or(any_huge) ? INT_MAX : G::kThreads * G::kEnt;
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+        const int32_t *pk = prev + kfirst + off[i];
+        if (off[i] <= most && len[i] <= kShortRow)
+            for (int k = 0; k < len[i]; ++k) nu[i] += pk[k] < s ? 1u : 0u;
+        // a long row: its wave counts it, 64 non-zeros at a time
+        for (uint64_t m = __ballot(off[i] <= most && len[i] > kShortRow); m; m &= m - 1) {
+            const int lane = __ffsll((unsigned long long)m) - 1;
+            const int o = __shfl(off[i], lane, 64), n = __shfl(len[i], lane, 64);
+            uint32_t c = 0;
+            for (int k = tid & 63; k < n; k += 64) c += prev[kfirst + o + k] < s ? 1u : 0u;
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d, 64);
+            if ((tid & 63) == lane) nu[i] = c;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
         uint32_t v[K];
 #pragma unroll
         for (int c = 0; c < K; ++c) v[c] = 0u;
-        live[i] = false;
-        if (r < nrows) {
-            const int64_t k0 = rp[r], k1 = rp[r + 1], n = k1 - k0;
-            if (n <= G::kCols) {
-                live[i] = true;
-                uint32_t nu = 0;
-                for (int64_t k = k0; k < k1; ++k) nu += prev[k] < s ? 1u : 0u;
-                v[1] = nu;
-                if constexpr (STYLE == kRounds) {
-                    if (n > 0) {
-                        const int p = piece_count(n), q = (int)(n / p), x = (int)(n % p);
-                        v[0] = (uint32_t)p;
-                        hist_add(v + 2, q, (uint32_t)(p - x));
-                        if (x) hist_add(v + 2, q + 1, (uint32_t)x);
-                    }
-                } else {
-                    v[0] = (uint32_t)n;
-                }
+        v[1] = nu[i];
+        if constexpr (STYLE == kRounds) {
+            if (len[i] > 0) {
+                const int p = piece_count(len[i]), q = len[i] / p, x = len[i] % p;
+                v[0] = (uint32_t)p;
+                hist_add(v + 2, q, (uint32_t)(p - x));
+                if (x) hist_add(v + 2, q + 1, (uint32_t)x);
             }
+        } else {
+            v[0] = (uint32_t)len[i];
         }
 #pragma unroll
         for (int c = 0; c < K; ++c) {
@@ -236,76 +269,111 @@ __global__ void k_plan_prev(int64_t nnz, const int32_t *__restrict__ scol, const
     prev[k] = found;
 }
 
+// One entry per start row on the grid: the next row on the grid where a tile
+// ends, the tiles up to there, their slots per thread and columns (summed).
+// sub[s + i]: end row and capacity | slots per thread << 16 of the i-th of them
+// (at most kRowAlign: a tile that ends between grid rows is shorter than that).
 template <class G, int STYLE>
 __global__ void __launch_bounds__(kPlanThreads) k_plan_table(int64_t nrows, const int64_t *__restrict__ rp,
                                                              const int32_t *__restrict__ prev,
-                                                             int2 *__restrict__ table) {
+                                                             int4 *__restrict__ table, int2 *__restrict__ sub) {
     __shared__ uint32_t scan_lds[6 * kPlanThreads / 64];
     __shared__ int sh[4];
     const int64_t s = (int64_t)blockIdx.x * kRowAlign;
-    const WindowTile w = window_tile<G, STYLE>(s, nrows, rp, prev, scan_lds, sh);
-    if (threadIdx.x == 0) table[blockIdx.x] = make_int2((int)w.end, w.cap | (w.ent << 16));
+    int64_t at = s;
+    int4 sum = make_int4(0, 0, 0, 0);
+    do {
+        const WindowTile w = window_tile<G, STYLE>(at, nrows, rp, prev, scan_lds, sh);
+        if (threadIdx.x == 0) sub[s + sum.y] = make_int2((int)w.end, w.cap | (w.ent << 16));
+        sum.y += 1;
+        sum.z += w.ent;
+        sum.w += w.cap;
+        at = w.end;
+    } while (at < nrows && at % kRowAlign != 0 && sum.y < kRowAlign);
+    sum.x = (int)at;
+    if (threadIdx.x == 0) table[blockIdx.x] = sum;
 }
 
-template <class G, int STYLE>
-__global__ void __launch_bounds__(kPlanThreads) k_plan_walk(int64_t nrows, const int64_t *__restrict__ rp,
-                                                            const int32_t *__restrict__ prev,
-                                                            const int2 *__restrict__ table, TileRec *__restrict__ recs,
-                                                            int64_t *__restrict__ totals) {
-    __shared__ uint32_t scan_lds[6 * kPlanThreads / 64];
-    __shared__ int sh[4];
-    __shared__ int2 chunk[kWalkChunk];
-    __shared__ int64_t bc[4];
-    const int tid = threadIdx.x;
-    const int64_t nA = (nrows + kRowAlign - 1) / kRowAlign;
-    int64_t s = 0, t = 0, ent_total = 0, col_total = 0, cbase = -1;
-    auto emit = [&](int64_t end, int cap, int ent) {
-        TileRec rec;
-        rec.row0 = s;
-        rec.ent_off = ent_total;
-        rec.col_off = col_total;
-        rec.nrows = (int32_t)(end - s);
-        rec.ent = ent;
-        rec.cap = cap;
-        rec.pad = 0;
-        recs[t] = rec;
-        ++t;
-        ent_total += (int64_t)ent * G::kThreads;
-        col_total += cap;
-        s = end;
-    };
-    while (s < nrows) {
-        if (s % kRowAlign == 0) {
-            const int64_t a = s / kRowAlign;
-            if (cbase < 0 || a < cbase || a >= cbase + kWalkChunk) {
-                cbase = a;
-                for (int i = tid; i < kWalkChunk && cbase + i < nA; i += kPlanThreads) chunk[i] = table[cbase + i];
-                __syncthreads();
-            }
-            if (tid == 0) {
-                while (s < nrows && s % kRowAlign == 0 && s / kRowAlign < cbase + kWalkChunk) {
-                    const int2 e = chunk[s / kRowAlign - cbase];
-                    emit(e.x, e.y & 0xffff, e.y >> 16);
-                }
-            }
-        } else {
-            const WindowTile w = window_tile<G, STYLE>(s, nrows, rp, prev, scan_lds, sh);
-            if (tid == 0) emit(w.end, w.cap, w.ent);
-        }
-        if (tid == 0) {
-            bc[0] = s;
-            bc[1] = t;
-            bc[2] = ent_total;
-            bc[3] = col_total;
-        }
-        __syncthreads();
-        s = bc[0];
-        t = bc[1];
-        ent_total = bc[2];
-        col_total = bc[3];
-        __syncthreads();
+// For every start of a chunk: the first row of the chain from it that lies past
+// the chunk, and the sums on the way (each jump is at least one start, so the
+// doubling ends within log2(kChunk) rounds).
+__global__ void __launch_bounds__(kPlanThreads) k_plan_chunk(int64_t nrows, const int4 *__restrict__ table,
+                                                             int4 *__restrict__ exits) {
+    constexpr int IPT = kChunk / kPlanThreads;
+    __shared__ int4 e[kChunk];
+    const int64_t nA = (nrows + kRowAlign - 1) / kRowAlign, base = (int64_t)blockIdx.x * kChunk;
+    const int64_t past = min(nrows, (base + kChunk) * kRowAlign);
+    int4 v[IPT];
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        const int i = threadIdx.x + j * kPlanThreads;
+        v[j] = base + i < nA ? table[base + i] : make_int4((int)nrows, 0, 0, 0);
+        e[i] = v[j];
     }
-    if (tid == 0) {
+    __syncthreads();
+    for (int round = 1; round < kChunk; round *= 2) {
+        bool more = false;
+#pragma unroll
+        for (int j = 0; j < IPT; ++j)
+            if (v[j].x < past) {
+                const int4 n = e[v[j].x / kRowAlign - (int)base];
+                v[j] = make_int4(n.x, v[j].y + n.y, v[j].z + n.z, v[j].w + n.w);
+                more = true;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < IPT; ++j) e[threadIdx.x + j * kPlanThreads] = v[j];
+        if (!__syncthreads_or(more)) break;
+    }
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        const int64_t a = base + threadIdx.x + j * kPlanThreads;
+        if (a < nA) exits[a] = v[j];
+    }
+}
+
+// The records of the tiles that start in the workgroup's chunk.
+template <class G>
+__global__ void __launch_bounds__(kPlanThreads) k_plan_emit(int64_t nrows, const int4 *__restrict__ table,
+                                                            const int4 *__restrict__ exits,
+                                                            const int2 *__restrict__ sub, TileRec *__restrict__ recs,
+                                                            int64_t *__restrict__ totals) {
+    __shared__ int4 e[kChunk];
+    const int64_t nA = (nrows + kRowAlign - 1) / kRowAlign, base = (int64_t)blockIdx.x * kChunk;
+    for (int i = threadIdx.x; i < kChunk && base + i < nA; i += kPlanThreads) e[i] = table[base + i];
+    __syncthreads();
+    if (threadIdx.x) return;
+    int64_t s = 0, t = 0, ent_total = 0, col_total = 0;
+    while (s < min(nrows, base * kRowAlign)) {
+        const int4 x = exits[s / kRowAlign];
+        t += x.y;
+        ent_total += (int64_t)x.z * G::kThreads;
+        col_total += x.w;
+        s = x.x;
+    }
+    const int64_t past = min(nrows, (base + kChunk) * kRowAlign);
+    while (s < past) {
+        const int4 x = e[s / kRowAlign - base];
+        int64_t at = s;
+        for (int i = 0; i < x.y; ++i) {
+            int2 q = make_int2(x.x, x.w | (x.z << 16));  // the one tile of the entry
+            if (x.y > 1) q = sub[s + i];
+            TileRec rec;
+            rec.row0 = at;
+            rec.ent_off = ent_total;
+            rec.col_off = col_total;
+            rec.nrows = (int32_t)(q.x - at);
+            rec.ent = q.y >> 16;
+            rec.cap = q.y & 0xffff;
+            rec.pad = 0;
+            recs[t++] = rec;
+            ent_total += (int64_t)rec.ent * G::kThreads;
+            col_total += rec.cap;
+            at = q.x;
+        }
+        s = x.x;
+    }
+    if (blockIdx.x == gridDim.x - 1) {
         totals[0] = t;
         totals[1] = ent_total;
         totals[2] = col_total;
@@ -682,14 +750,17 @@ void make_plan(const Csr &A, TilePlan &P, hipStream_t s) {
         hipLaunchKernelGGL(k_plan_prev, dim3(grid_for(nnz, 256)), dim3(256), 0, s, nnz, scol.p, sk.p, row.p,
                            A.rowptr.p, (int64_t)G::kCols, (int64_t)G::kRows, prev.p);
     }
-    DevBuf<int2> table(nA > 0 ? nA : 1, s);
+    const int64_t nC = (nA + kChunk - 1) / kChunk;
+    DevBuf<int4> table(nA, s), exits(nA, s);
+    DevBuf<int2> sub(nA * kRowAlign, s);
     DevBuf<TileRec> recs(nrows > 0 ? nrows : 1, s);
     DevBuf<int64_t> totals(3, s);
     DevBuf<int64_t> hflag(nrows + 1, s), hpos(nrows + 1, s);
     hipLaunchKernelGGL((k_plan_table<G, STYLE>), dim3((unsigned)nA), dim3(kPlanThreads), 0, s, nrows, A.rowptr.p,
-                       prev.p, table.p);
-    hipLaunchKernelGGL((k_plan_walk<G, STYLE>), dim3(1), dim3(kPlanThreads), 0, s, nrows, A.rowptr.p, prev.p,
-                       table.p, recs.p, totals.p);
+                       prev.p, table.p, sub.p);
+    hipLaunchKernelGGL(k_plan_chunk, dim3((unsigned)nC), dim3(kPlanThreads), 0, s, nrows, table.p, exits.p);
+    hipLaunchKernelGGL(k_plan_emit<G>, dim3((unsigned)nC), dim3(kPlanThreads), 0, s, nrows, table.p, exits.p, sub.p,
+                       recs.p, totals.p);
     CR_HIP(hipMemsetAsync(hflag.p + nrows, 0, sizeof(int64_t), s));
     hipLaunchKernelGGL(k_huge_flags, dim3(grid_for(nrows, 256)), dim3(256), 0, s, nrows, A.rowptr.p,
                        (int64_t)G::kCols, hflag.p);
