@@ -12,8 +12,10 @@
 // per-vertex gradients with FP64 atomics (order-nondeterministic in the last
 // bits).  Gradients are tangential: the areas depend on the vertices through
 // v/|v|.  Areas here are on the unit sphere; `area_scale` converts.
+#include <algorithm>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "regridder.hpp"
 #include "sphgeom.hpp"
@@ -58,7 +60,6 @@ struct VertexSink {
     double *lacc_subj, *lacc_clip;     // LDS accumulators of one side's slots, or null
     double *own_clip;                  // the pair's own 4 x 3 clip-slot sums in LDS, or null
     double *own_subj;                  // the pair's own 4 x 3 subject-slot sums in LDS, or null
-    bool own_atomic = false;           // other lanes add to the own sums too (LDS atomics)
 
     // slot e of the subject, 0 <= e <= ns (an edge's end vertex e + 1 wraps)
     __device__ int wrap(int e) const { return e >= ns ? e - ns : e; }
@@ -84,13 +85,9 @@ struct VertexSink {
             add_local(lacc_subj, e, tangential(g, sv(e)));
         } else if (own_subj) {  // this pair's own sums
             const d3 t = tangential(g, sv(e));
-            if (own_atomic) {
-                add_local(own_subj, e, t);
-            } else {
-                own_subj[3 * e] += t.x;
-                own_subj[3 * e + 1] += t.y;
-                own_subj[3 * e + 2] += t.z;
-            }
+            own_subj[3 * e] += t.x;
+            own_subj[3 * e + 1] += t.y;
+            own_subj[3 * e + 2] += t.z;
         } else {
             add(g_subj, subj_vi[e], tangential(g, sv(e)));
         }
@@ -102,13 +99,9 @@ struct VertexSink {
         if (lacc_clip) {
             add_local(lacc_clip, kk, t);
         } else if (own_clip) {  // this pair's own sums
-            if (own_atomic) {
-                add_local(own_clip, kk, t);
-            } else {
-                own_clip[3 * kk] += t.x;
-                own_clip[3 * kk + 1] += t.y;
-                own_clip[3 * kk + 2] += t.z;
-            }
+            own_clip[3 * kk] += t.x;
+            own_clip[3 * kk + 1] += t.y;
+            own_clip[3 * kk + 2] += t.z;
         } else {
             add(g_clip, clip_vi[kk], t);
         }
@@ -186,131 +179,229 @@ __device__ __forceinline__ void flush_rows(const double *lacc, int64_t r0, int64
     }
 }
 
-// Crossing work of the boundary decomposition, queued per wave in LDS: a
-// crossing's gradient (tangential at it) with its label and its pair's lane,
-// done 64 at a time by the whole wave at the points where every lane's pass 2
-// is in step.  A flush leaves fewer than 64; a lane adds at most 2 between
-// flushes.
-constexpr int kXQueue = 64 + 2 * 64;
+// Gradients of one line's two vertices into caller vertices.
+__device__ __forceinline__ void add_line(double *g, const int32_t *vi, int j, int j1, const d3 &p, const d3 &q,
+                                         double w, const LineSum &S) {
+    if (!g) return;
+    d3 gp, gq;
+    line_grad(p, q, LineSum{w * S.p, w * S.q}, gp, gq);
+    atomicAdd(g + 3 * (int64_t)vi[j], gp.x);
+    atomicAdd(g + 3 * (int64_t)vi[j] + 1, gp.y);
+    atomicAdd(g + 3 * (int64_t)vi[j] + 2, gp.z);
+    atomicAdd(g + 3 * (int64_t)vi[j1], gq.x);
+    atomicAdd(g + 3 * (int64_t)vi[j1] + 1, gq.y);
+    atomicAdd(g + 3 * (int64_t)vi[j1] + 2, gq.z);
+}
 
-struct XQueue {
-    int32_t lab[kXQueue], lane[kXQueue];
-    double g[3 * kXQueue];
-    int32_t pd[64], ps[64];  // each lane's pair (destination, source cell)
-    int n;
-};
+// Destination rows of a wave summed in LDS: at most 256 lines of three doubles.
+inline int arc_rows(int dst_nv) { return std::max(1, std::min(64, 256 / dst_nv)); }
 
+// The vertex pass by boundary arcs (edges_plan + edges_arcs), one wave per 64
+// consecutive non-zeros, a lane each.  Nothing but two numbers per line is summed
+// per pair: a destination cell's lines are summed in LDS over the wave's pairs (an
+// edge wholly inside the other cell adds its coefficient alone) and turned into
+// vertex gradients once per wave and row; a source cell's lines once per pair, in
+// registers (it clips) or in LDS (it is clipped, at most 4 vertices).  A pair
+// near a degenerate configuration is appended to `list` (wave by wave, in order)
+// for k_clip_grad_list.
+//
+// Bound: FP64 VALU of the plan (side values of every subject vertex against the
+// clip lines, then the few edges that cross) and the gradients' own traffic.
+// Differentiating every crossing and fan triangle instead, with the crossings
+// queued in LDS, took 15 600 VALU instructions a wave against 5 500 here: quarter
+// degree -> HEALPix 256 (16-gons, nnz 4.35 M) 3.62 -> 1.49 ms, C96 -> 1 degree
+// 200 -> 95 us.  The lane-to-double mapping of the atomics matters as much: with
+// a lane per pair and vertex the same arithmetic ran 2.55 ms.
 template <int NC>
-struct QueueEmit {
-    VertexSink<NC> *sink;
-    XQueue *q;
-    bool live;
-    // the decomposition emits subject vertices, clip vertices and
-    // subject x clip crossings (no clip x clip crossings)
-    __device__ __forceinline__ void operator()(int32_t l, const d3 &x, const d3 &g) {
-        if (!live) return;
-        const int32_t t = lab_type(l);
-        if (t == kLabXF) {
-            const d3 gt = tangential(g, x);
-            const int e = atomicAdd(&q->n, 1);
-            q->lab[e] = l;
-            q->lane[e] = threadIdx.x;
-            q->g[3 * e] = gt.x;
-            q->g[3 * e + 1] = gt.y;
-            q->g[3 * e + 2] = gt.z;
-        } else if (t == kLabS) {
-            sink->add_subj(l & kLabIndexMask, g);
-        } else {
-            sink->add_clip(lab_lo(l), g);
-        }
-    }
-};
-
-// The vertex pass by boundary decomposition (edges_plan + edges_emit), one
-// wave per 64 consecutive non-zeros: flat loops over the subject edges and
-// the clip edges (no clip stages), every lane through the same iterations
-// (a declined or empty lane emits nothing), crossings through the queue.  A
-// pair the decomposition declines (near a degenerate configuration, or a
-// degenerate clip edge) is appended to `list` (wave by wave, in order) for
-// k_clip_grad_list.
-template <int NC>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_clip_grad_edges(
+__global__ void __launch_bounds__(64) k_clip_grad_arcs(
     const int32_t *__restrict__ rowid, const int32_t *__restrict__ col, const double *__restrict__ coef,
     int64_t nnz, const double *__restrict__ dst_cells, int dst_nv, const int32_t *__restrict__ dst_vi,
-    const double *__restrict__ src_cells, int src_nv, const int32_t *__restrict__ src_vi, int clip_is_dst,
-    double *__restrict__ g_dst, double *__restrict__ g_src, int32_t *__restrict__ list,
+    const double *__restrict__ src_cells, int src_nv, const int32_t *__restrict__ src_vi, int clip_is_dst, int window,
+    int private_v, double *__restrict__ g_dst, double *__restrict__ g_src, int32_t *__restrict__ list,
     uint32_t *__restrict__ count) {
-    extern __shared__ double lacc[];  // kGradRows * dst_nv * 3
-    __shared__ double own[64 * 12];
-    __shared__ XQueue q;
+    extern __shared__ double lds[];
     const int lane = threadIdx.x;
+    double *rows = lds;  // window x dst_nv x (M_p, M_q, coefficient of whole edges)
+    const int nrow = window * dst_nv * 3;
+    // a source cell of at most 4 vertices: the sums of its lines (it is clipped),
+    // then its vertices' gradients, 12 a pair
+    double *own = rows + nrow;
+    const bool use_own = src_nv <= 4;
+    uint8_t *codes = (uint8_t *)(own + (use_own ? 64 * 12 : 0));  // [subject edge][lane]: k_in + 1 | k_out + 1 << 4
     const int64_t k0 = (int64_t)blockIdx.x * 64, k = k0 + lane;
     const int64_t r0 = rowid[k0];
-    const int nacc = kGradRows * dst_nv * 3;
-    for (int i = lane; i < nacc; i += 64) lacc[i] = 0.0;
-    double *my_own = own + 12 * lane;
-#pragma unroll
-    for (int i = 0; i < 12; ++i) my_own[i] = 0.0;
-    const bool real = k < nnz;
-    const int64_t kk = real ? k : k0;  // lanes past the end run the loops on a valid pair
-    const int32_t d = rowid[kk], s = col[kk];
-    q.pd[lane] = d;
-    q.ps[lane] = s;
-    if (lane == 0) q.n = 0;
+    for (int i = lane; i < nrow; i += 64) rows[i] = 0.0;
+    double *mine = own + 12 * lane;
+    if (use_own)
+        for (int i = 0; i < 12; ++i) mine[i] = 0.0;
     __syncthreads();
-    const double c = real ? coef[kk] : 0.0;
-    VertexSink<NC> sink = pair_sink<NC>(d, s, r0, lacc, my_own, dst_cells, dst_nv, dst_vi, src_cells, src_nv, src_vi,
-                                clip_is_dst, g_dst, g_src);
-    EdgesPlan<NC> P;
-    const bool planned = edges_plan<NC>(sink.clip, sink.nc, sink.subj, sink.ns, P);
-    const bool live = c != 0.0 && planned;
-    // declined pairs to the list: one atomic per wave, lanes in order
-    {
-        const bool fb = c != 0.0 && !planned;
-        const uint64_t m = __ballot(fb);
-        if (m) {
-            uint32_t base = 0;
-            if (lane == 0) base = atomicAdd(count, (uint32_t)__popcll(m));
-            base = __shfl(base, 0);
-            if (fb) list[base + __popcll(m & ((1ull << lane) - 1ull))] = (int32_t)k;
+    const double w = k < nnz ? coef[k] : 0.0;
+    bool planned = true;
+    if (w != 0.0) {
+        const int64_t d = rowid[k], s = col[k];
+        const double *dp = dst_cells + 3 * (int64_t)dst_nv * d, *sp = src_cells + 3 * (int64_t)src_nv * s;
+        const double *clip = clip_is_dst ? dp : sp, *subj = clip_is_dst ? sp : dp;
+        const int nc = clip_is_dst ? dst_nv : src_nv, ns = clip_is_dst ? src_nv : dst_nv;
+        const int32_t *dvi = dst_vi + (int64_t)dst_nv * d, *svi = src_vi + (int64_t)src_nv * s;
+        double *row = d - r0 < window ? rows + (d - r0) * dst_nv * 3 : nullptr;
+        uint8_t *code = codes + lane;
+        EdgesPlan P;
+        planned = edges_plan<NC>(clip, nc, subj, ns, P, [&](int j, int k_in, int k_out) {
+            code[64 * j] = (uint8_t)((k_in + 1) | (k_out + 1) << 4);
+        });
+        if (planned) {
+            auto subject_line = [&](int j, const LineSum &S) {
+                if (clip_is_dst && use_own) {
+                    mine[2 * j] = S.p;
+                    mine[2 * j + 1] = S.q;
+                } else if (!clip_is_dst && row) {
+                    atomicAdd(row + 3 * j, w * S.p);
+                    atomicAdd(row + 3 * j + 1, w * S.q);
+                } else {
+                    const int j1 = j + 1 == ns ? 0 : j + 1;
+                    add_line(clip_is_dst ? g_src : g_dst, clip_is_dst ? svi : dvi, j, j1, load3(subj + 3 * j),
+                             load3(subj + 3 * j1), w, S);
+                }
+            };
+            for (uint64_t m = P.full; m; m &= m - 1) {
+                const int j = __builtin_ctzll(m);
+                if (!clip_is_dst && row) {
+                    atomicAdd(row + 3 * j + 2, w);
+                } else {
+                    const double h = whole_sum(load3(subj + 3 * j), load3(subj + 3 * (j + 1 == ns ? 0 : j + 1)));
+                    subject_line(j, LineSum{h, h});
+                }
+            }
+            LineSum S[NC];
+            edges_arcs<NC>(
+                clip, nc, subj, ns, P,
+                [&](int j, int &k_in, int &k_out) {
+                    const int c = code[64 * j];
+                    k_in = (c & 15) - 1;
+                    k_out = (c >> 4) - 1;
+                },
+                subject_line, S);
+            if (clip_is_dst) {
+#pragma unroll
+                for (int m = 0; m < NC; ++m) {
+                    if (row) {
+                        atomicAdd(row + 3 * m, w * S[m].p);
+                        atomicAdd(row + 3 * m + 1, w * S[m].q);
+                    } else {
+                        const int m1 = (m + 1) % NC;
+                        add_line(g_dst, dvi, m, m1, load3(clip + 3 * m), load3(clip + 3 * m1), w, S[m]);
+                    }
+                }
+            } else {
+                // vertex m: its parts from the lines before and after it
+                d3 g[NC];
+#pragma unroll
+                for (int m = 0; m < NC; ++m) g[m] = mk3(0.0, 0.0, 0.0);
+#pragma unroll
+                for (int m = 0; m < NC; ++m) {
+                    d3 gp, gq;
+                    line_grad(load3(clip + 3 * m), load3(clip + 3 * ((m + 1) % NC)), LineSum{w * S[m].p, w * S[m].q}, gp,
+                              gq);
+                    g[m] = g[m] + gp;
+                    g[(m + 1) % NC] = g[(m + 1) % NC] + gq;
+                }
+#pragma unroll
+                for (int m = 0; m < NC; ++m) {
+                    if (m < 4 && use_own) {
+                        mine[3 * m] = g[m].x;
+                        mine[3 * m + 1] = g[m].y;
+                        mine[3 * m + 2] = g[m].z;
+                    } else {
+                        VertexSink<NC>::add(g_src, svi[m], g[m]);
+                    }
+                }
+            }
+            if (clip_is_dst && use_own) {
+                d3 g[4];
+                LineSum L[4];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    g[m] = mk3(0.0, 0.0, 0.0);
+                    L[m] = LineSum{w * mine[2 * m], w * mine[2 * m + 1]};
+                }
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    if (m >= src_nv) continue;
+                    const int m1 = m + 1 == src_nv ? 0 : m + 1;
+                    d3 gp, gq;
+                    line_grad(load3(subj + 3 * m), load3(subj + 3 * m1), L[m], gp, gq);
+                    g[m] = g[m] + gp;
+                    if (m1 == 0) g[0] = g[0] + gq;
+                    else g[(m + 1) % 4] = g[(m + 1) % 4] + gq;
+                }
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    mine[3 * m] = g[m].x;
+                    mine[3 * m + 1] = g[m].y;
+                    mine[3 * m + 2] = g[m].z;
+                }
+            }
         }
     }
-    auto work = [&](int e) {
-        const int L = q.lane[e];
-        const int32_t l = q.lab[e];
-        const d3 gt = mk3(q.g[3 * e], q.g[3 * e + 1], q.g[3 * e + 2]);
-        VertexSink<NC> sk = pair_sink<NC>(q.pd[L], q.ps[L], r0, lacc, own + 12 * L, dst_cells, dst_nv, dst_vi, src_cells,
-                                  src_nv, src_vi, clip_is_dst, g_dst, g_src);
-        sk.own_atomic = true;
-        const int a = lab_hi(l), b = lab_lo(l);
-        d3 gp1, gq1, gp2, gq2;
-        if (crossing_backward_arc(gt, sk.sv(a), sk.sv(a + 1), sk.cv(b), sk.cv(b + 1), gp1, gq1, gp2, gq2)) {
-            sk.add_subj(a, gp1);
-            sk.add_subj(a + 1, gq1);
-            sk.add_clip(b, gp2);
-            sk.add_clip(b + 1, gq2);
-        }
-    };
-    auto flush = [&](bool drain) {
-        __syncthreads();
-        int n = q.n;
-        while (n >= 64) {
-            work(n - 64 + lane);
-            n -= 64;
-        }
-        if (drain && lane < n) work(lane);
-        __syncthreads();
-        if (lane == 0) q.n = drain ? 0 : n;
-        __syncthreads();
-    };
-    QueueEmit<NC> em{&sink, &q, live};
-    edges_emit<NC>(P, sink.subj, sink.ns, c, em, [&] { flush(false); });
-    flush(true);
-    if (live) flush_own(sink, src_nv, my_own, g_src);
+    // declined pairs to the list: one atomic per wave, lanes in order
+    const uint64_t m = __ballot(!planned);
+    if (m) {
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(count, (uint32_t)__popcll(m));
+        base = __shfl(base, 0);
+        if (!planned) list[base + __popcll(m & ((1ull << lane) - 1ull))] = (int32_t)k;
+    }
     __syncthreads();
+    // the pairs' source vertices, neighbouring lanes on neighbouring doubles (a
+    // quad's 12 are two runs of 48 bytes: an atomic of 64 lanes then touches about
+    // 11 lines; a lane per pair touched 64)
+    if (use_own && g_src) {
+        const int32_t s = k < nnz ? col[k] : 0;
+        for (int i = lane; i < 64 * 12; i += 64) {
+            const int pair = i / 12, e = i - 12 * pair;
+            const int64_t sp = __shfl(s, pair, 64);
+            const double v = own[i];
+            if (v != 0.0) atomicAdd(g_src + 3 * (int64_t)src_vi[sp * src_nv + e / 3] + e % 3, v);
+        }
+    }
     if (!g_dst) return;
-    const int64_t klast = min(nnz, k0 + 64) - 1;
-    flush_rows(lacc, r0, min((int64_t)kGradRows, (int64_t)rowid[klast] - r0 + 1), dst_nv, dst_vi, g_dst);
+    // the wave's destination rows: a lane per vertex, from the lines before and
+    // after it, then a lane per double
+    const int64_t last = rowid[min(nnz, k0 + 64) - 1] - r0 + 1;
+    const int n = (int)min((int64_t)window, last) * dst_nv;
+    d3 g[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int i = lane + 64 * t;
+        g[t] = mk3(0.0, 0.0, 0.0);
+        if (i >= n) continue;
+        const int r = i / dst_nv, v = i - r * dst_nv, u = v == 0 ? dst_nv - 1 : v - 1, v1 = v + 1 == dst_nv ? 0 : v + 1;
+        const double *cell = dst_cells + 3 * (int64_t)dst_nv * (r0 + r), *line = rows + 3 * dst_nv * r;
+        const d3 pu = load3(cell + 3 * u), pv = load3(cell + 3 * v), pn = load3(cell + 3 * v1);
+        d3 gp, gq, unused;
+        line_grad(pu, pv, LineSum{0.0, line[3 * u + 1] + line[3 * u + 2] * whole_sum(pu, pv)}, unused, gq);
+        line_grad(pv, pn, LineSum{line[3 * v] + line[3 * v + 2] * whole_sum(pv, pn), 0.0}, gp, unused);
+        g[t] = gq + gp;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int i = lane + 64 * t;
+        if (i >= n) continue;
+        rows[3 * i] = g[t].x;
+        rows[3 * i + 1] = g[t].y;
+        rows[3 * i + 2] = g[t].z;
+    }
+    __syncthreads();
+    // cells that own their vertices: only the first and last row can be another wave's too
+    const int lo = private_v ? dst_nv * 3 : 3 * n, hi = private_v ? (int)(last - 1) * dst_nv * 3 : 0;
+    for (int i = lane; i < 3 * n; i += 64) {
+        const double v = rows[i];
+        if (v == 0.0) continue;
+        double *to = g_dst + 3 * (int64_t)dst_vi[r0 * dst_nv + i / 3] + i % 3;
+        if (i >= lo && i < hi) *to += v;
+        else atomicAdd(to, v);
+    }
 }
 
 // The vertex pass through the clip pipeline (clip_area_backward) for the
@@ -615,23 +706,22 @@ static void backward(const cr_regridder *R, const cr_grid *dst, const cr_grid *s
         }
         hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, count);  // a kernel: no memset node in a graph
         const size_t lds = (size_t)kGradRows * dst->nv * 3 * sizeof(double);
-        if (clip_nv <= 4) {
-            hipLaunchKernelGGL(k_clip_grad_edges<4>, dim3(grid_for(F.nnz, 64)), dim3(64), lds, s, rowid, F.col.p,
+        const bool cd = R->stats.clip_with_dst != 0;
+        const int window = arc_rows(dst->nv);
+        const size_t arcs_lds = ((size_t)window * dst->nv * 3 + (src->nv <= 4 ? 64 * 12 : 0)) * sizeof(double) +
+                                64 * (size_t)(cd ? src->nv : dst->nv);
+        auto vertex_pass = [&](auto nc) {
+            constexpr int NC = decltype(nc)::value;
+            hipLaunchKernelGGL(k_clip_grad_arcs<NC>, dim3(grid_for(F.nnz, 64)), dim3(64), arcs_lds, s, rowid, F.col.p,
                                coef, F.nnz, dst->cells.p, dst->nv, dst->vidx.p, src->cells.p, src->nv, src->vidx.p,
-                               R->stats.clip_with_dst, g_dst_verts, g_src_verts, list, count);
-            hipLaunchKernelGGL(k_clip_grad_list<4>, dim3(kListBlocks), dim3(64), lds, s, rowid, F.col.p, coef,
+                               (int)cd, window, dst->private_vertices, g_dst_verts, g_src_verts, list, count);
+            hipLaunchKernelGGL(k_clip_grad_list<NC>, dim3(kListBlocks), dim3(64), lds, s, rowid, F.col.p, coef,
                                dst->cells.p, dst->nv, dst->vidx.p, src->cells.p, src->nv, src->vidx.p,
                                R->stats.clip_with_dst, g_dst_verts, g_src_verts, (const int32_t *)list,
                                (const uint32_t *)count, F.nrows);
-        } else {
-            hipLaunchKernelGGL(k_clip_grad_edges<8>, dim3(grid_for(F.nnz, 64)), dim3(64), lds, s, rowid, F.col.p,
-                               coef, F.nnz, dst->cells.p, dst->nv, dst->vidx.p, src->cells.p, src->nv, src->vidx.p,
-                               R->stats.clip_with_dst, g_dst_verts, g_src_verts, list, count);
-            hipLaunchKernelGGL(k_clip_grad_list<8>, dim3(kListBlocks), dim3(64), lds, s, rowid, F.col.p, coef,
-                               dst->cells.p, dst->nv, dst->vidx.p, src->cells.p, src->nv, src->vidx.p,
-                               R->stats.clip_with_dst, g_dst_verts, g_src_verts, (const int32_t *)list,
-                               (const uint32_t *)count, F.nrows);
-        }
+        };
+        if (clip_nv <= 4) vertex_pass(std::integral_constant<int, 4>());
+        else vertex_pass(std::integral_constant<int, 8>());
         CR_HIP(hipGetLastError());
     }
     double *g_to = transpose ? g_src_verts : g_dst_verts;

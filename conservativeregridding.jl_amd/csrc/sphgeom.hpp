@@ -455,25 +455,6 @@ CR_HD void clip_area_backward(const double *clip, int nc, const double *subj, in
     P.area_close();
 }
 
-// crossing_backward for a crossing that lies on the arc p1 -> q1, with the
-// gradient already made tangential at the crossing: the sign of y is that of
-// y.(p1 + q1).
-CR_HD bool crossing_backward_arc(const d3 &gt, const d3 &p1, const d3 &q1, const d3 &p2, const d3 &q2, d3 &gp1,
-                                 d3 &gq1, d3 &gp2, d3 &gq2) {
-    d3 n1 = cross(p1, q1), n2 = cross(p2, q2);
-    d3 y = cross(n1, n2);
-    double L = sqrt(dot(y, y));
-    if (!(L > 1e-300)) return false;
-    double sigma = dot(y, p1 + q1) >= 0.0 ? 1.0 : -1.0;
-    d3 yb = (sigma / L) * gt;
-    d3 n1b = cross(n2, yb), n2b = cross(yb, n1);
-    gp1 = cross(q1, n1b);
-    gq1 = cross(n1b, p1);
-    gp2 = cross(q2, n2b);
-    gq2 = cross(n2b, p2);
-    return true;
-}
-
 // Gradient w.r.t. the great-circle crossing x = y/|y| (y = +-(n1 x n2),
 // n1 = p1 x q1, n2 = p2 x q2) pushed back to p1, q1, p2, q2.
 CR_HD bool crossing_backward(const d3 &x, const d3 &g, const d3 &p1, const d3 &q1, const d3 &p2,
@@ -493,390 +474,295 @@ CR_HD bool crossing_backward(const d3 &x, const d3 &g, const d3 &p1, const d3 &q
 }
 
 // ============================================================================
-// Backward by boundary decomposition (no clip pipeline): edges_plan, then
-// edges_emit.
+// Backward by boundary arcs (no clip pipeline): edges_plan, then edges_arcs and
+// line_grad.
 //
-// area(P), P = subject ∩ clip, is the sum over P's boundary arcs a -> b of the
-// fan triangle E(O, a, b) for any fixed point O (the area does not depend on
-// it; O is taken on P's boundary so that every triangle is as small as P).
-// The arcs are (i) the part of each subject edge inside the convex clip
-// polygon -- one interval, from the edge's side values against every clip
-// line: the latest entry and the earliest exit (Liang-Barsky on the chord
-// parameter; the crossings are the forward's crossing() of the edge's own end
-// points) -- and (ii) the parts of the clip edges inside the subject, which
-// begin where a subject edge leaves the clip polygon through that edge's line
-// or at a clip vertex inside the subject, and end where a subject edge enters
-// or at the next clip vertex.  A clip edge carries at most two such points
-// here.  Each arc's two end points take their derivatives: a subject vertex
-// or clip vertex directly, a crossing through crossing_backward (labels as in
-// clip_area_backward, g not yet tangential, coef applied).  Every loop runs
-// over the ring sizes: no clip stages, no recursion.
+// To first order the area of P = subject ∩ clip changes only by the motion of
+// the great circles that carry its boundary (the motion of a corner along them
+// is of second order), so no crossing point is differentiated.  When vertex p of
+// the line p -> q (inside on its left, n = p x q) moves by d along n / |n|, a
+// point x of the line moves inward by d sin(xq) / sin(pq) (angles to q), so an arc
+// a -> b on it loses the area d / |n| (cos(bq) - cos(aq)), that is
+//   dA/dp = -n / |n|^2 M_p,   M_p = (|a - q|^2 - |b - q|^2) / 2,
+//   dA/dq = -n / |n|^2 M_q,   M_q = (|b - p|^2 - |a - p|^2) / 2
+// (tangential by themselves).  M_p and M_q are sums over the line's arcs: all
+// arcs of one line (of one pair, or of all pairs that share the cell) are summed
+// first, and line_grad runs once per line.  An edge's squared lengths are taken
+// from differences, so nothing of the order of the sphere is cancelled (the same
+// sums kept as vectors b - a, with q x ((b - a) x n) / n.n at the end, lost three
+// digits on quarter-degree cells).
 //
-// edges_plan returns false (and edges_emit then emits nothing for the pair)
-// when the pair is near a configuration where the area is not differentiable
-// or where the decisions above could differ from the forward clip's by
-// rounding -- a subject vertex within ~1e-10 of a clip edge's length from
-// that edge (on its line between the lines through its corners), a crossing
-// within that distance of a clip corner or of another crossing on its clip
-// edge, an edge entering and leaving through neighbouring lines at one point
-// -- when a clip edge meets the subject's boundary more than twice, or when a
-// clip edge is degenerate.  The caller then uses clip_area_backward.
+// The arcs: (i) the part of each subject edge inside the convex clip polygon --
+// one interval, from the edge's side values against every clip line: the latest
+// entry and the earliest exit (Liang-Barsky on the chord parameter; the
+// crossings are the forward's crossing() of the edge's own end points); (ii) the
+// parts of the clip edges inside the subject: they begin where a subject edge
+// leaves the clip polygon through that edge's line or at a clip vertex inside
+// the subject, and end where a subject edge enters or at the next clip vertex,
+// so their sums are signed sums over those points.
+//
+// edges_plan returns false when the pair is near a configuration where the area
+// is not differentiable or where the decisions above could differ from the
+// forward clip's by rounding -- a subject vertex within ~1e-10 of a clip edge's
+// length from that edge (on its line between the lines through its corners), a
+// crossing within that distance of a clip corner or of another crossing on its
+// clip edge, an edge entering and leaving through neighbouring lines at one
+// point -- when a clip edge meets the subject's boundary more than twice, or
+// when a clip edge is degenerate (the forward's corner there is the crossing of
+// the neighbouring lines).  The caller then uses clip_area_backward.
 // ============================================================================
 constexpr double kEdgeTol = 1e-10;
 
-// d E(O, a, b) / da and / db for the fan triangle O -> a -> b (O fixed).
-CR_HD void fan_grad(const d3 &O, const d3 &a, const d3 &b, double coef, d3 &ga, d3 &gb) {
-    const double T = dot(O, cross(a, b));
-    const double D = 1.0 + dot(O, a) + dot(a, b) + dot(b, O);
-    const double f = coef * 2.0 / (T * T + D * D);
-    ga = f * (D * cross(b, O) - T * (O + b));
-    gb = f * (D * cross(O, a) - T * (O + a));
-}
-
 // The crossings of one subject edge with the clip lines: the latest entry
-// (k_in, t_in) and the earliest exit (k_out, t_out); empty when an end point
-// pair lies outside one line.
-// The winners' side values (and, with corners, their clip edge's end points)
-// are carried out of the unrolled loop, so no array is indexed by a run-time
-// line number (which would put it in scratch memory).
+// (k_in, t_in) and the earliest exit (k_out, t_out); empty when its end points
+// lie outside one line.  The winners' neighbours' side values (against the lines
+// through their clip edge's first and last corner) are carried out of the
+// unrolled loop, so no array is indexed by a run-time line number (which would
+// put it in scratch memory).
 template <int NC>
 struct EdgeCut {
-    double t_in, t_out, ap_in, aq_in, ap_out, aq_out;
-    // POS: the end points' side values against the lines before and after
-    // the winning line (through its clip edge's first and last corner), and
-    // their tolerances: at the crossing they place it along the clip edge
+    double t_in, t_out;
     double bp_in, bq_in, fp_in, fq_in, btol_in, ftol_in;
     double bp_out, bq_out, fp_out, fq_out, btol_out, ftol_out;
     int k_in, k_out;
-    bool empty;
-    template <bool POS>
     CR_HD void make(const double (&ap)[NC], const double (&aq)[NC], const double (&tol)[NC]) {
         t_in = 0.0;
         t_out = 1.0;
-        ap_in = aq_in = ap_out = aq_out = 0.0;
         k_in = -1;
         k_out = -1;
-        empty = false;
+        bp_in = bq_in = fp_in = fq_in = btol_in = ftol_in = 0.0;
+        bp_out = bq_out = fp_out = fq_out = btol_out = ftol_out = 0.0;
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
             const bool pin = ap[k] >= 0.0, qin = aq[k] >= 0.0;
-            if (pin && qin) continue;
-            if (!pin && !qin) {
-                empty = true;
-                continue;
-            }
+            if (pin == qin) continue;
             const double t = fabs(ap[k]) / (fabs(ap[k]) + fabs(aq[k]));
             const int b = (k + NC - 1) % NC, f = (k + 1) % NC;
             if (!pin && t > t_in) {
                 t_in = t;
                 k_in = k;
-                ap_in = ap[k];
-                aq_in = aq[k];
-                if (POS) {
-                    bp_in = ap[b];
-                    bq_in = aq[b];
-                    fp_in = ap[f];
-                    fq_in = aq[f];
-                    btol_in = tol[b];
-                    ftol_in = tol[f];
-                }
+                bp_in = ap[b];
+                bq_in = aq[b];
+                fp_in = ap[f];
+                fq_in = aq[f];
+                btol_in = tol[b];
+                ftol_in = tol[f];
             }
             if (pin && t < t_out) {
                 t_out = t;
                 k_out = k;
-                ap_out = ap[k];
-                aq_out = aq[k];
-                if (POS) {
-                    bp_out = ap[b];
-                    bq_out = aq[b];
-                    fp_out = ap[f];
-                    fq_out = aq[f];
-                    btol_out = tol[b];
-                    ftol_out = tol[f];
-                }
+                bp_out = ap[b];
+                bq_out = aq[b];
+                fp_out = ap[f];
+                fq_out = aq[f];
+                btol_out = tol[b];
+                ftol_out = tol[f];
             }
         }
     }
-    CR_HD bool inside() const { return !empty && t_in < t_out; }
 };
 
-// The crossing of subject edge j with the clip line through ck with normal
-// nk: the forward's crossing() of the edge's own end points.
-CR_HD d3 edge_cut_point(const double *subj, int ns, int j, const d3 &ck, const d3 &nk) {
-    const d3 p = load3(subj + 3 * j), q = load3(subj + 3 * (j + 1 == ns ? 0 : j + 1));
-    return crossing(p, dot(nk, p - ck), q, dot(nk, q - ck));
-}
-
-// What pass 1 leaves for pass 2: the clip ring and its lines, the crossings
-// on every clip edge (at most two, in order along the edge; kind 1 = a
-// clip-edge arc begins there), and O.
-template <int NC>
 struct EdgesPlan {
-    d3 c[NC], n[NC], O;
-    int32_t lab_lo[NC], lab_hi[NC];
-    int kind_lo[NC], kind_hi[NC], cnt[NC];
-    bool any_out;
+    uint64_t full, part;  // subject edges inside the clip polygon as a whole, in part
+    unsigned corners;     // bit k: clip vertex k lies inside the subject
 };
 
-// Pass 1: the checks (false: use clip_area_backward) and the plan.
-template <int NC>
-CR_HD bool edges_plan_(const double *clip, int nc, const double *subj, int ns, EdgesPlan<NC> &P) {
+// The checks (false: use clip_area_backward) and the plan.  code(j, k_in,
+// k_out): the lines (or -1) through which edge j, a bit of `part`, enters and
+// leaves.  At most 64 subject vertices.
+template <int NC, class Code>
+CR_HD bool edges_plan(const double *clip, int nc, const double *subj, int ns, EdgesPlan &P, Code &&code) {
+    P.full = P.part = 0;
+    P.corners = 0;
+    d3 c[NC], n[NC];
     double tol[NC];
-    // a declined plan still drives edges_emit in step with the other lanes
-    // (emitting nothing): it reads no crossing labels (no counts) and finite lines
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) c[k] = load3(clip + 3 * (k < nc ? k : nc - 1));
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-        P.c[k] = load3(clip + 3 * (k < nc ? k : nc - 1));
-        P.n[k] = mk3(0.0, 0.0, 0.0);
-        P.lab_lo[k] = P.lab_hi[k] = -1;
-        P.kind_lo[k] = P.kind_hi[k] = 0;
-        P.cnt[k] = 0;
-    }
-    P.any_out = false;
-    P.O = load3(subj);
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-        const d3 e = P.c[(k + 1) % NC] - P.c[k];
-        const d3 nk = cross(P.c[k], e);
-        const double nn = dot(nk, nk);
-        // a degenerate clip edge (a polar cell's coincident corners, a padded
-        // triangle) is no constraint in the forward clip, whose corner there is
-        // the crossing of the two neighbouring lines: clip_area_backward
-        // differentiates that corner; this decomposition would not
-        if (nn < kDegenerateEdge2) return false;
-        P.n[k] = nk;
+        n[k] = cross(c[k], c[(k + 1) % NC] - c[k]);
+        const double nn = dot(n[k], n[k]);
+        ok = ok && nn >= kDegenerateEdge2;
         tol[k] = kEdgeTol * nn;  // |side| below this: within ~1e-10 edge lengths of the line
     }
-    double u_lo[NC], u_hi[NC];
+    if (!ok) return false;
+    // vertices outside each line; a vertex on a clip line is a degenerate point
+    // only on the clip edge's segment (inside the lines through its two corners)
+    uint64_t out[NC];
 #pragma unroll
-    for (int k = 0; k < NC; ++k) u_lo[k] = u_hi[k] = -1.0;
-    bool have_O = false, overflow = false;
-    // a subject vertex on a clip line is a degenerate point only on the
-    // clip edge's segment (inside the lines through its two corners); off it,
-    // both clips take the line's side test the same way
-    auto on_edge = [&](const double (&a)[NC]) {
-        bool hit = false;
+    for (int k = 0; k < NC; ++k) out[k] = 0;
+    for (int j = 0; j < ns; ++j) {
+        const d3 v = load3(subj + 3 * j);
+        double a[NC];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            a[k] = dot(n[k], v - c[k]);
+            out[k] |= (uint64_t)(a[k] < 0.0) << j;
+        }
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
             const int b = (k + NC - 1) % NC, f = (k + 1) % NC;
-            hit = hit || (fabs(a[k]) <= tol[k] && a[b] >= -tol[b] && a[f] >= -tol[f]);
+            ok = ok && !(fabs(a[k]) <= tol[k] && a[b] >= -tol[b] && a[f] >= -tol[f]);
         }
-        return hit;
-    };
-    d3 p = load3(subj);
-    double ap[NC];
+    }
+    if (!ok) return false;
+    const uint64_t all = ns >= 64 ? ~0ull : (1ull << ns) - 1ull;
+    auto next = [&](uint64_t m) { return ((m >> 1) | (m << (ns - 1))) & all; };  // bit j: vertex j + 1
+    uint64_t any_out = 0, apart = 0;
 #pragma unroll
-    for (int k = 0; k < NC; ++k) ap[k] = dot(P.n[k], p - P.c[k]);
-    if (on_edge(ap)) return false;
-    for (int j = 0; j < ns; ++j) {
-        const d3 q = load3(subj + 3 * (j + 1 == ns ? 0 : j + 1));
-        double aq[NC];
+    for (int k = 0; k < NC; ++k) {
+        any_out |= out[k];
+        apart |= out[k] & next(out[k]);
+    }
+    P.full = ~any_out & next(~any_out & all) & all;
+    P.part = all & ~apart & ~P.full;
+    // the crossings on each clip edge (at most two): the first's place along the
+    // edge, and whether a clip-edge arc begins (the subject leaves) at the first
+    // and at the last
+    double u_lo[NC];
+    unsigned one = 0, two = 0, lo_leaves = 0, hi_leaves = 0;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) u_lo[k] = 0.0;
+    for (uint64_t left = P.part; left; left &= left - 1) {
+        const int j = __builtin_ctzll(left);
+        const d3 p = load3(subj + 3 * j), q = load3(subj + 3 * (j + 1 == ns ? 0 : j + 1));
+        double ap[NC], aq[NC];
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
-            aq[k] = dot(P.n[k], q - P.c[k]);
-            P.any_out = P.any_out || aq[k] < 0.0;
+            ap[k] = dot(n[k], p - c[k]);
+            aq[k] = dot(n[k], q - c[k]);
         }
-        if (on_edge(aq)) return false;
         EdgeCut<NC> cut;
-        cut.template make<true>(ap, aq, tol);
+        cut.make(ap, aq, tol);
         if (cut.k_in >= 0 && cut.k_out >= 0 && fabs(cut.t_in - cut.t_out) <= kEdgeTol) return false;
-        if (cut.inside()) {
-            if (!have_O) {
-                P.O = cut.k_in >= 0 ? crossing(p, cut.ap_in, q, cut.aq_in) : p;
-                have_O = true;
+        if (!(cut.t_in < cut.t_out)) {
+            P.part &= ~(1ull << j);
+            continue;
+        }
+        code(j, cut.k_in, cut.k_out);
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            const int k = side == 0 ? cut.k_in : cut.k_out;
+            if (k < 0) continue;
+            // the crossing's place along clip edge k: its side values (linear
+            // along the chord) against the line through the edge's first corner
+            // (0 there, growing along the edge) and through its last
+            const double t = side == 0 ? cut.t_in : cut.t_out;
+            const double u = side == 0 ? (1.0 - t) * cut.bp_in + t * cut.bq_in
+                                       : (1.0 - t) * cut.bp_out + t * cut.bq_out;
+            const double v = side == 0 ? (1.0 - t) * cut.fp_in + t * cut.fq_in
+                                       : (1.0 - t) * cut.fp_out + t * cut.fq_out;
+            const double utol = side == 0 ? cut.btol_in : cut.btol_out;
+            if (u <= utol || v <= (side == 0 ? cut.ftol_in : cut.ftol_out)) return false;  // at a clip corner
+            const unsigned bit = 1u << k, leaves = side == 1 ? bit : 0u;
+            if (two & bit) return false;
+            double first = 0.0;
+#pragma unroll
+            for (int m = 0; m < NC; ++m)
+                if (m == k) {
+                    first = u_lo[m];
+                    if (!(one & bit) || u < first) u_lo[m] = u;
+                }
+            if (!(one & bit)) {
+                one |= bit;
+                lo_leaves |= leaves;
+                hi_leaves |= leaves;
+            } else {
+                if (fabs(u - first) <= utol) return false;
+                two |= bit;
+                if (u > first) hi_leaves = (hi_leaves & ~bit) | leaves;
+                else lo_leaves = (lo_leaves & ~bit) | leaves;
             }
+        }
+    }
+    if (two & ~(lo_leaves ^ hi_leaves)) return false;  // not an arc's two ends
+    // a clip vertex's state is that after the last crossing before it along the
+    // clip boundary; with no crossing P is the clip polygon (some subject vertex
+    // outside it) or the subject
+    if (one) {
 #pragma unroll
-            for (int side = 0; side < 2; ++side) {
-                const int k = side == 0 ? cut.k_in : cut.k_out;
-                if (k < 0) continue;
-                // the crossing's place along clip edge k: its side values (linear
-                // along the chord) against the line through the edge's first
-                // corner (0 there, growing along the edge) and through its last
-                const double t = side == 0 ? cut.t_in : cut.t_out;
-                const double u = side == 0 ? (1.0 - t) * cut.bp_in + t * cut.bq_in
-                                           : (1.0 - t) * cut.bp_out + t * cut.bq_out;
-                const double v = side == 0 ? (1.0 - t) * cut.fp_in + t * cut.fq_in
-                                           : (1.0 - t) * cut.fp_out + t * cut.fq_out;
-                if (u <= (side == 0 ? cut.btol_in : cut.btol_out) || v <= (side == 0 ? cut.ftol_in : cut.ftol_out))
-                    return false;  // within ~1e-10 of a clip corner
-                // entering the clip polygon through line k ends a clip-edge arc there (kind 0),
-                // leaving through it begins one (kind 1)
-                const int32_t lab = lab_make(kLabXF, j, k);
+        for (int k = 0; k < NC; ++k) {
+            bool found = false;
 #pragma unroll
-                for (int m = 0; m < NC; ++m) {
-                    if (m != k) continue;
-                    if (P.cnt[m] == 0) {
-                        u_lo[m] = u;
-                        P.lab_lo[m] = lab;
-                        P.kind_lo[m] = side;
-                    } else if (P.cnt[m] == 1) {
-                        if (fabs(u - u_lo[m]) <= tol[(m + NC - 1) % NC]) overflow = true;
-                        if (u > u_lo[m]) {
-                            u_hi[m] = u;
-                            P.lab_hi[m] = lab;
-                            P.kind_hi[m] = side;
-                        } else {
-                            u_hi[m] = u_lo[m];
-                            P.lab_hi[m] = P.lab_lo[m];
-                            P.kind_hi[m] = P.kind_lo[m];
-                            u_lo[m] = u;
-                            P.lab_lo[m] = lab;
-                            P.kind_lo[m] = side;
-                        }
-                    } else {
-                        overflow = true;
-                    }
-                    P.cnt[m] += 1;
+            for (int s = 1; s <= NC; ++s) {
+                const int m = (k - s + NC) % NC;
+                if (!found && (one >> m & 1u)) {
+                    P.corners |= (hi_leaves >> m & 1u) << k;
+                    found = true;
                 }
             }
         }
-        p = q;
-#pragma unroll
-        for (int k = 0; k < NC; ++k) ap[k] = aq[k];
+    } else if (any_out) {
+        P.corners = (1u << NC) - 1u;
     }
-    if (overflow) return false;
-#pragma unroll
-    for (int k = 0; k < NC; ++k)
-        if (P.cnt[k] == 2 && P.kind_lo[k] == P.kind_hi[k]) return false;  // not an arc's two ends
-    if (!have_O) P.O = P.any_out ? P.c[0] : load3(subj);  // P is the clip polygon, or the subject
     return true;
 }
 
-template <int NC>
-CR_HD bool edges_plan(const double *clip, int nc, const double *subj, int ns, EdgesPlan<NC> &P) {
-    if (edges_plan_<NC>(clip, nc, subj, ns, P)) return true;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) P.cnt[k] = 0;
-    return false;
+// M_p and M_q of a line's arcs.
+struct LineSum {
+    double p, q;
+};
+// ... of the arc a -> b of the line p -> q (as products of differences: a short
+// arc keeps its relative accuracy), and of the whole line.
+CR_HD LineSum arc_sum(const d3 &p, const d3 &q, const d3 &a, const d3 &b) {
+    const d3 h = 0.5 * (b - a);
+    return LineSum{-dot(h, (a - q) + (b - q)), dot(h, (a - p) + (b - p))};
+}
+CR_HD double whole_sum(const d3 &p, const d3 &q) {
+    const d3 e = q - p;
+    return 0.5 * dot(e, e);
 }
 
-// The arcs of clip edge K: the state at c_K (inside the subject or not) is
-// carried from the last crossing before it along the clip boundary; with no
-// crossing anywhere P is the clip polygon (some subject vertex outside it) or
-// the subject.  Clip-vertex parts go to gc, crossings to emit.
-template <int K, int NC, class Emit>
-CR_HD void clip_arcs(const EdgesPlan<NC> &P, const double *subj, int ns, double coef, bool any_ev,
-                     d3 (&gc)[NC], Emit &emit) {
-    constexpr int K1 = (K + 1) % NC;
-    const d3 &O = P.O;
-    int in_start = P.any_out ? 1 : 0;
-    if (any_ev) {
-        bool found = false;
+// The arcs of a plan: arc(j, sums) for the part of every subject edge of `part`,
+// and S[k] = the sums of the parts of clip edge k inside the subject.  lines(j,
+// k_in, k_out) gives back what code stored.
+template <int NC, class Lines, class Arc>
+CR_HD void edges_arcs(const double *clip, int nc, const double *subj, int ns, const EdgesPlan &P, Lines &&lines,
+                      Arc &&arc, LineSum (&S)[NC]) {
 #pragma unroll
-        for (int s = 1; s <= NC; ++s) {
-            const int m = (K - s + NC) % NC;
-            if (!found && P.cnt[m] > 0) {
-                in_start = P.cnt[m] == 2 ? P.kind_hi[m] : P.kind_lo[m];
-                found = true;
-            }
+    for (int k = 0; k < NC; ++k) S[k] = LineSum{0.0, 0.0};
+    for (uint64_t left = P.part; left; left &= left - 1) {
+        const int j = __builtin_ctzll(left);
+        int line[2];
+        lines(j, line[0], line[1]);
+        const d3 p = load3(subj + 3 * j), q = load3(subj + 3 * (j + 1 == ns ? 0 : j + 1));
+        d3 end[2] = {p, q};
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            const int k = line[side];
+            if (k < 0) continue;
+            const d3 c = load3(clip + 3 * k), e = load3(clip + 3 * (k + 1 == nc ? 0 : k + 1));
+            const d3 n = cross(c, e - c);
+            const d3 x = crossing(p, dot(n, p - c), q, dot(n, q - c));
+            end[side] = x;
+            // a clip-edge arc ends where the subject enters, begins where it leaves
+            const double h = side == 0 ? 0.5 : -0.5;
+            const double sp = -h * dot(x - e, x - e), sq = h * dot(x - c, x - c);
+#pragma unroll
+            for (int m = 0; m < NC; ++m)
+                if (m == k) {
+                    S[m].p += sp;
+                    S[m].q += sq;
+                }
         }
+        arc(j, arc_sum(p, q, end[0], end[1]));
     }
-    if (P.cnt[K] == 0) {
-        if (in_start) {
-            d3 ga, gb;
-            fan_grad(O, P.c[K], P.c[K1], coef, ga, gb);
-            gc[K] = gc[K] + ga;
-            gc[K1] = gc[K1] + gb;
-        }
-        return;
-    }
-    const int32_t l1 = P.lab_lo[K];
-    const d3 x1 = edge_cut_point(subj, ns, lab_hi(l1), P.c[K], P.n[K]);
-    if (P.kind_lo[K] == 0) {  // an arc from c_K ends at the first crossing
-        d3 ga, gb;
-        fan_grad(O, P.c[K], x1, coef, ga, gb);
-        gc[K] = gc[K] + ga;
-        emit(l1, x1, gb);
-    }
-    if (P.cnt[K] == 1) {
-        if (P.kind_lo[K] == 1) {  // an arc begins there and runs to c_K+1
-            d3 ga, gb;
-            fan_grad(O, x1, P.c[K1], coef, ga, gb);
-            emit(l1, x1, ga);
-            gc[K1] = gc[K1] + gb;
-        }
-        return;
-    }
-    const int32_t l2 = P.lab_hi[K];
-    const d3 x2 = edge_cut_point(subj, ns, lab_hi(l2), P.c[K], P.n[K]);
-    d3 ga, gb;
-    if (P.kind_lo[K] == 1) {  // one arc between the two crossings
-        fan_grad(O, x1, x2, coef, ga, gb);
-        emit(l1, x1, ga);
-        emit(l2, x2, gb);
-    } else {  // the second crossing begins an arc to c_K+1
-        fan_grad(O, x2, P.c[K1], coef, ga, gb);
-        emit(l2, x2, ga);
-        gc[K1] = gc[K1] + gb;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        const double h = whole_sum(load3(clip + 3 * (k < nc ? k : nc - 1)), load3(clip + 3 * (k + 1 < nc ? k + 1 : 0)));
+        if (P.corners >> k & 1u) S[k].p += h;
+        if (P.corners >> ((k + 1) % NC) & 1u) S[k].q += h;
     }
 }
 
-template <int K, int NC, class Emit, class Sync>
-CR_HD void clip_arcs_from(const EdgesPlan<NC> &P, const double *subj, int ns, double coef, bool any_ev,
-                          d3 (&gc)[NC], Emit &emit, Sync &sync) {
-    clip_arcs<K, NC>(P, subj, ns, coef, any_ev, gc, emit);
-    sync();
-    if constexpr (K + 1 < NC) clip_arcs_from<K + 1, NC>(P, subj, ns, coef, any_ev, gc, emit, sync);
-}
-
-// Pass 2: every arc's end-point derivatives through emit.  sync() is called
-// after every subject edge and every clip edge, the same number of times
-// whatever the pair (a caller running lanes in step may act there).
-template <int NC, class Emit, class Sync>
-CR_HD void edges_emit(const EdgesPlan<NC> &P, const double *subj, int ns, double coef, Emit &emit, Sync &&sync) {
-    const d3 O = P.O;
-    // the subject arcs
-    const int32_t labS = lab_make(kLabS, 0, 0);
-    d3 p = load3(subj), g_first = mk3(0.0, 0.0, 0.0), g_pend = mk3(0.0, 0.0, 0.0);
-    double ap[NC];
-#pragma unroll
-    for (int k = 0; k < NC; ++k) ap[k] = dot(P.n[k], p - P.c[k]);
-    for (int j = 0; j < ns; ++j) {
-        const d3 q = load3(subj + 3 * (j + 1 == ns ? 0 : j + 1));
-        double aq[NC];
-#pragma unroll
-        for (int k = 0; k < NC; ++k) aq[k] = dot(P.n[k], q - P.c[k]);
-        EdgeCut<NC> cut;
-        cut.template make<false>(ap, aq, ap);  // no positions: the third argument is not read
-        d3 g_p = mk3(0.0, 0.0, 0.0), g_q = mk3(0.0, 0.0, 0.0);  // this edge's parts of s_j and s_j+1
-        if (cut.inside()) {
-            const d3 xa = cut.k_in >= 0 ? crossing(p, cut.ap_in, q, cut.aq_in) : p;
-            const d3 xb = cut.k_out >= 0 ? crossing(p, cut.ap_out, q, cut.aq_out) : q;
-            d3 ga, gb;
-            fan_grad(O, xa, xb, coef, ga, gb);
-            if (cut.k_in >= 0) emit(lab_make(kLabXF, j, cut.k_in), xa, ga);
-            else g_p = ga;
-            if (cut.k_out >= 0) emit(lab_make(kLabXF, j, cut.k_out), xb, gb);
-            else g_q = gb;
-        }
-        if (j == 0) {
-            g_first = g_p;
-        } else {
-            const d3 g = g_pend + g_p;  // subject vertex j: from edges j - 1 and j
-            if (g.x != 0.0 || g.y != 0.0 || g.z != 0.0) emit(labS | j, p, g);
-        }
-        g_pend = g_q;
-        p = q;
-#pragma unroll
-        for (int k = 0; k < NC; ++k) ap[k] = aq[k];
-        sync();
-    }
-    {
-        const d3 g = g_first + g_pend;  // vertex 0: from the first and the closing edge
-        if (g.x != 0.0 || g.y != 0.0 || g.z != 0.0) emit(labS, p, g);
-    }
-    // the clip arcs, one clip edge at a time (K a template argument: every
-    // index stays compile-time whatever the compiler unrolls)
-    bool any_ev = false;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) any_ev = any_ev || P.cnt[k] > 0;
-    d3 gc[NC];
-#pragma unroll
-    for (int k = 0; k < NC; ++k) gc[k] = mk3(0.0, 0.0, 0.0);
-    clip_arcs_from<0, NC>(P, subj, ns, coef, any_ev, gc, emit, sync);
-#pragma unroll
-    for (int k = 0; k < NC; ++k)
-        if (gc[k].x != 0.0 || gc[k].y != 0.0 || gc[k].z != 0.0) emit(lab_make(kLabC, 0, k), P.c[k], gc[k]);
+// The derivative of the area w.r.t. the vertices p, q of a boundary line (zero
+// for a line of no length).
+CR_HD void line_grad(const d3 &p, const d3 &q, const LineSum &S, d3 &gp, d3 &gq) {
+    const d3 n = cross(p, q - p);
+    const double nn = dot(n, n), f = nn > 0.0 ? -1.0 / nn : 0.0;
+    gp = (f * S.p) * n;
+    gq = (f * S.q) * n;
 }
 
 // coef * d(signed ring area)/d(vertices) through emit(slot, grad): one call per
