@@ -22,13 +22,6 @@
 
 namespace cr {
 
-// Row index of every non-zero of CSR(A) (rows = dst).
-__global__ void k_pair_rows(const int64_t *__restrict__ rowptr, int64_t nrows, int32_t *__restrict__ rowid) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nrows) return;
-    for (int64_t k = rowptr[i]; k < rowptr[i + 1]; ++k) rowid[k] = (int32_t)i;
-}
-
 // Per non-zero of CSR(A) (rows = dst, cols = src), one thread each: the
 // coefficient dL/dA_u,ij (unit-sphere areas).
 __global__ void k_pair_coef(const int32_t *__restrict__ rowid, const int32_t *__restrict__ col, int64_t nnz,
@@ -196,47 +189,87 @@ __device__ __forceinline__ void add_line(double *g, const int32_t *vi, int j, in
 // Destination rows of a wave summed in LDS: at most 256 lines of three doubles.
 inline int arc_rows(int dst_nv) { return std::max(1, std::min(64, 256 / dst_nv)); }
 
-// The vertex pass by boundary arcs (edges_plan + edges_arcs), one wave per 64
-// consecutive non-zeros, a lane each.  Nothing but two numbers per line is summed
-// per pair: a destination cell's lines are summed in LDS over the wave's pairs (an
-// edge wholly inside the other cell adds its coefficient alone) and turned into
+// The destination cells' area term: cell i's area has dL/da_i = -kappa / a_i
+// sum_f gy_if y_if (y null: no term).
+struct AreaTerm {
+    const double *y, *gy, *a_to;
+    const int64_t *rowptr;
+    int64_t yc, yf, gc, gf, nf;
+    double kappa;
+};
+__device__ __forceinline__ double area_coef(const AreaTerm &A, int64_t i) {
+    if (A.a_to[i] == 0.0) return 0.0;  // zero-area (ghost) cells have no area term
+    double s = 0.0;
+    for (int64_t f = 0; f < A.nf; ++f) s += A.gy[i * A.gc + f * A.gf] * A.y[i * A.yc + f * A.yf];
+    return -A.kappa * s / A.a_to[i];
+}
+
+// Subject edges a pair may have inside the clip polygon in part (more: declined),
+// kept in LDS; a quad's are at most 4, a 16-gon's rarely more than 8.
+template <class M>
+constexpr int kArcs = sizeof(M) == 1 ? 6 : 8;
+template <class M>
+constexpr int kOwn = 2 * kArcs<M> + 1;  // a lane's doubles in LDS (odd: lanes on different banks)
+
+// The vertex pass by boundary arcs (pair_arcs), one wave per 64 consecutive
+// non-zeros, a lane each.  Nothing but two numbers per line is summed per pair: a
+// destination cell's lines are summed in LDS over the wave's pairs (an edge
+// wholly inside the other cell adds its coefficient alone, and so does the cell's
+// own area term, in the wave that holds the row's first non-zero) and turned into
 // vertex gradients once per wave and row; a source cell's lines once per pair, in
-// registers (it clips) or in LDS (it is clipped, at most 4 vertices).  A pair
-// near a degenerate configuration is appended to `list` (wave by wave, in order)
-// for k_clip_grad_list.
+// registers.  A pair near a degenerate configuration is appended to `list` (wave
+// by wave, in order) for k_clip_grad_list.  M: a bit per subject vertex.
 //
-// Bound: FP64 VALU of the plan (side values of every subject vertex against the
+// Bound: FP64 VALU of the arcs (side values of every subject vertex against the
 // clip lines, then the few edges that cross) and the gradients' own traffic.
 // Differentiating every crossing and fan triangle instead, with the crossings
-// queued in LDS, took 15 600 VALU instructions a wave against 5 500 here: quarter
-// degree -> HEALPix 256 (16-gons, nnz 4.35 M) 3.62 -> 1.49 ms, C96 -> 1 degree
-// 200 -> 95 us.  The lane-to-double mapping of the atomics matters as much: with
-// a lane per pair and vertex the same arithmetic ran 2.55 ms.
-template <int NC>
-__global__ void __launch_bounds__(64) k_clip_grad_arcs(
+// queued in LDS, took 15 600 VALU instructions a wave against 5 000 here: the whole
+// vertex pass on quarter degree -> HEALPix 256 (16-gons, nnz 4.35 M), with the
+// declined pairs and the area term, 4.39 -> 1.62 ms; C96 -> 1 degree 276 -> 100 us.
+// The lane-to-double mapping of the atomics matters as much: with a lane per pair
+// and vertex this kernel ran 2.55 ms.  Three waves a SIMD (168 registers, a few
+// spilled) against two: 1.88 and 2.11 ms for the whole reverse mode.
+template <int NC, class M>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC == 4 ? 3 : 2))) k_clip_grad_arcs(
     const int32_t *__restrict__ rowid, const int32_t *__restrict__ col, const double *__restrict__ coef,
     int64_t nnz, const double *__restrict__ dst_cells, int dst_nv, const int32_t *__restrict__ dst_vi,
     const double *__restrict__ src_cells, int src_nv, const int32_t *__restrict__ src_vi, int clip_is_dst, int window,
-    int private_v, double *__restrict__ g_dst, double *__restrict__ g_src, int32_t *__restrict__ list,
+    int private_v, AreaTerm area, double *__restrict__ g_dst, double *__restrict__ g_src, int32_t *__restrict__ list,
     uint32_t *__restrict__ count) {
-    extern __shared__ double lds[];
+    // a lane's arcs of subject edges (M_p, M_q), then its source vertices' gradients
+    __shared__ double own[64 * kOwn<M>];
+    __shared__ double acoef[64];  // the rows' area terms
+    __shared__ uint8_t lead[64];  // a lane of each source cell
+    extern __shared__ double rows[];  // window x dst_nv x (M_p, M_q, coefficient of whole edges)
     const int lane = threadIdx.x;
-    double *rows = lds;  // window x dst_nv x (M_p, M_q, coefficient of whole edges)
     const int nrow = window * dst_nv * 3;
-    // a source cell of at most 4 vertices: the sums of its lines (it is clipped),
-    // then its vertices' gradients, 12 a pair
-    double *own = rows + nrow;
     const bool use_own = src_nv <= 4;
-    uint8_t *codes = (uint8_t *)(own + (use_own ? 64 * 12 : 0));  // [subject edge][lane]: k_in + 1 | k_out + 1 << 4
     const int64_t k0 = (int64_t)blockIdx.x * 64, k = k0 + lane;
     const int64_t r0 = rowid[k0];
     for (int i = lane; i < nrow; i += 64) rows[i] = 0.0;
-    double *mine = own + 12 * lane;
-    if (use_own)
-        for (int i = 0; i < 12; ++i) mine[i] = 0.0;
     __syncthreads();
     const double w = k < nnz ? coef[k] : 0.0;
-    bool planned = true;
+    double *mine = own + kOwn<M> * lane;
+    bool planned = true, zero = true;  // zero: no source vertex gradients in `mine`
+    // the wave's rows; their area terms, a lane per row
+    const int64_t last = rowid[min(nnz, k0 + 64) - 1] - r0 + 1;
+    acoef[lane] = 0.0;
+    if (area.y && g_dst) {
+        for (int64_t r = lane; r < last; r += 64) {
+            const double c = area.rowptr[r0 + r] >= k0 ? area_coef(area, r0 + r) : 0.0;
+            if (r < window) {
+                acoef[r] = c;
+            } else if (c != 0.0) {
+                const double *cell = dst_cells + 3 * (int64_t)dst_nv * (r0 + r);
+                for (int v = 0; v < dst_nv; ++v) {
+                    const int v1 = v + 1 == dst_nv ? 0 : v + 1;
+                    const d3 p = load3(cell + 3 * v), q = load3(cell + 3 * v1);
+                    const double h = whole_sum(p, q);
+                    add_line(g_dst, dst_vi + (r0 + r) * dst_nv, v, v1, p, q, c, LineSum{h, h});
+                }
+            }
+        }
+    }
     if (w != 0.0) {
         const int64_t d = rowid[k], s = col[k];
         const double *dp = dst_cells + 3 * (int64_t)dst_nv * d, *sp = src_cells + 3 * (int64_t)src_nv * s;
@@ -244,101 +277,90 @@ __global__ void __launch_bounds__(64) k_clip_grad_arcs(
         const int nc = clip_is_dst ? dst_nv : src_nv, ns = clip_is_dst ? src_nv : dst_nv;
         const int32_t *dvi = dst_vi + (int64_t)dst_nv * d, *svi = src_vi + (int64_t)src_nv * s;
         double *row = d - r0 < window ? rows + (d - r0) * dst_nv * 3 : nullptr;
-        uint8_t *code = codes + lane;
-        EdgesPlan P;
-        planned = edges_plan<NC>(clip, nc, subj, ns, P, [&](int j, int k_in, int k_out) {
-            code[64 * j] = (uint8_t)((k_in + 1) | (k_out + 1) << 4);
+        M full;
+        LineSum S[NC];
+        int arcs = 0;
+        uint64_t edge = 0;  // the arcs' subject edges, a byte each
+        planned = pair_arcs<NC, M>(clip, nc, subj, ns, full, S, [&](int i, int j, const LineSum &a) {
+            if (i >= kArcs<M>) return false;
+            mine[2 * i] = a.p;
+            mine[2 * i + 1] = a.q;
+            edge |= (uint64_t)j << (8 * i);
+            arcs = i + 1;
+            return true;
         });
         if (planned) {
-            auto subject_line = [&](int j, const LineSum &S) {
-                if (clip_is_dst && use_own) {
-                    mine[2 * j] = S.p;
-                    mine[2 * j + 1] = S.q;
-                } else if (!clip_is_dst && row) {
-                    atomicAdd(row + 3 * j, w * S.p);
-                    atomicAdd(row + 3 * j + 1, w * S.q);
-                } else {
-                    const int j1 = j + 1 == ns ? 0 : j + 1;
-                    add_line(clip_is_dst ? g_src : g_dst, clip_is_dst ? svi : dvi, j, j1, load3(subj + 3 * j),
-                             load3(subj + 3 * j1), w, S);
-                }
+            auto after = [&](int j) { return j + 1 == ns ? 0 : j + 1; };
+            auto clear = [&] {
+                zero = false;
+#pragma unroll
+                for (int i = 0; i < 12; ++i) mine[i] = 0.0;
             };
-            for (uint64_t m = P.full; m; m &= m - 1) {
-                const int j = __builtin_ctzll(m);
-                if (!clip_is_dst && row) {
-                    atomicAdd(row + 3 * j + 2, w);
-                } else {
-                    const double h = whole_sum(load3(subj + 3 * j), load3(subj + 3 * (j + 1 == ns ? 0 : j + 1)));
-                    subject_line(j, LineSum{h, h});
+            auto add_own = [&](int v, int v1, const d3 &p, const d3 &q, const LineSum &L) {
+                d3 gp, gq;
+                line_grad(p, q, L, gp, gq);
+                mine[3 * v] += gp.x;
+                mine[3 * v + 1] += gp.y;
+                mine[3 * v + 2] += gp.z;
+                mine[3 * v1] += gq.x;
+                mine[3 * v1 + 1] += gq.y;
+                mine[3 * v1 + 2] += gq.z;
+            };
+            if (!clip_is_dst && row) {
+                for (M m = full; m; m &= m - 1) atomicAdd(row + 3 * __builtin_ctzll((unsigned long long)m) + 2, w);
+                for (int i = 0; i < arcs; ++i, edge >>= 8) {
+                    double *line = row + 3 * (int)(edge & 255);
+                    atomicAdd(line, w * mine[2 * i]);
+                    atomicAdd(line + 1, w * mine[2 * i + 1]);
                 }
-            }
-            LineSum S[NC];
-            edges_arcs<NC>(
-                clip, nc, subj, ns, P,
-                [&](int j, int &k_in, int &k_out) {
-                    const int c = code[64 * j];
-                    k_in = (c & 15) - 1;
-                    k_out = (c >> 4) - 1;
-                },
-                subject_line, S);
-            if (clip_is_dst) {
-#pragma unroll
-                for (int m = 0; m < NC; ++m) {
-                    if (row) {
-                        atomicAdd(row + 3 * m, w * S[m].p);
-                        atomicAdd(row + 3 * m + 1, w * S[m].q);
-                    } else {
-                        const int m1 = (m + 1) % NC;
-                        add_line(g_dst, dvi, m, m1, load3(clip + 3 * m), load3(clip + 3 * m1), w, S[m]);
-                    }
-                }
-            } else {
-                // vertex m: its parts from the lines before and after it
-                d3 g[NC];
-#pragma unroll
-                for (int m = 0; m < NC; ++m) g[m] = mk3(0.0, 0.0, 0.0);
-#pragma unroll
-                for (int m = 0; m < NC; ++m) {
-                    d3 gp, gq;
-                    line_grad(load3(clip + 3 * m), load3(clip + 3 * ((m + 1) % NC)), LineSum{w * S[m].p, w * S[m].q}, gp,
-                              gq);
-                    g[m] = g[m] + gp;
-                    g[(m + 1) % NC] = g[(m + 1) % NC] + gq;
-                }
-#pragma unroll
-                for (int m = 0; m < NC; ++m) {
-                    if (m < 4 && use_own) {
-                        mine[3 * m] = g[m].x;
-                        mine[3 * m + 1] = g[m].y;
-                        mine[3 * m + 2] = g[m].z;
-                    } else {
-                        VertexSink<NC>::add(g_src, svi[m], g[m]);
-                    }
-                }
-            }
-            if (clip_is_dst && use_own) {
-                d3 g[4];
+            } else if (clip_is_dst && use_own) {
                 LineSum L[4];
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
-                    g[m] = mk3(0.0, 0.0, 0.0);
-                    L[m] = LineSum{w * mine[2 * m], w * mine[2 * m + 1]};
+                    L[m] = LineSum{0.0, 0.0};
+                    if (m < ns && (full >> m & 1))
+                        L[m].p = L[m].q = w * whole_sum(load3(subj + 3 * m), load3(subj + 3 * after(m)));
                 }
+                for (int i = 0; i < arcs; ++i, edge >>= 8) {
+#pragma unroll
+                    for (int m = 0; m < 4; ++m)
+                        if (m == (int)(edge & 255)) L[m] = LineSum{w * mine[2 * i], w * mine[2 * i + 1]};
+                }
+                clear();
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
-                    if (m >= src_nv) continue;
-                    const int m1 = m + 1 == src_nv ? 0 : m + 1;
-                    d3 gp, gq;
-                    line_grad(load3(subj + 3 * m), load3(subj + 3 * m1), L[m], gp, gq);
-                    g[m] = g[m] + gp;
-                    if (m1 == 0) g[0] = g[0] + gq;
-                    else g[(m + 1) % 4] = g[(m + 1) % 4] + gq;
+                    if (m >= ns) continue;
+                    add_own(m, after(m), load3(subj + 3 * m), load3(subj + 3 * after(m)), L[m]);
                 }
+            } else {  // a subject of more vertices, or a row past the window
+                double *g = clip_is_dst ? g_src : g_dst;
+                const int32_t *vi = clip_is_dst ? svi : dvi;
+                for (M m = full; m; m &= m - 1) {
+                    const int j = __builtin_ctzll((unsigned long long)m);
+                    const d3 p = load3(subj + 3 * j), q = load3(subj + 3 * after(j));
+                    const double h = whole_sum(p, q);
+                    add_line(g, vi, j, after(j), p, q, w, LineSum{h, h});
+                }
+                for (int i = 0; i < arcs; ++i, edge >>= 8) {
+                    const int j = (int)(edge & 255);
+                    add_line(g, vi, j, after(j), load3(subj + 3 * j), load3(subj + 3 * after(j)), w,
+                             LineSum{mine[2 * i], mine[2 * i + 1]});
+                }
+            }
+            if (NC == 4 && !clip_is_dst) clear();
+            // the clip cell's lines (one without a length has no sums)
 #pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    mine[3 * m] = g[m].x;
-                    mine[3 * m + 1] = g[m].y;
-                    mine[3 * m + 2] = g[m].z;
+            for (int m = 0; m < NC; ++m) {
+                const int i0 = clip_first<NC>(m, nc), i1 = clip_second<NC>(m, nc);
+                if (i0 == i1) continue;
+                if (clip_is_dst && row) {
+                    atomicAdd(row + 3 * i0, w * S[m].p);
+                    atomicAdd(row + 3 * i0 + 1, w * S[m].q);
+                } else if (NC == 4 && !clip_is_dst) {  // nc <= 4: its vertices are the pair's own
+                    add_own(i0, i1, load3(clip + 3 * i0), load3(clip + 3 * i1), LineSum{w * S[m].p, w * S[m].q});
+                } else {
+                    add_line(clip_is_dst ? g_dst : g_src, clip_is_dst ? dvi : svi, i0, i1, load3(clip + 3 * i0),
+                             load3(clip + 3 * i1), w, S[m]);
                 }
             }
         }
@@ -351,24 +373,57 @@ __global__ void __launch_bounds__(64) k_clip_grad_arcs(
         base = __shfl(base, 0);
         if (!planned) list[base + __popcll(m & ((1ull << lane) - 1ull))] = (int32_t)k;
     }
-    __syncthreads();
-    // the pairs' source vertices, neighbouring lanes on neighbouring doubles (a
+    // the pairs' source vertices: neighbouring lanes take neighbouring doubles (a
     // quad's 12 are two runs of 48 bytes: an atomic of 64 lanes then touches about
-    // 11 lines; a lane per pair touched 64)
+    // 11 lines; a lane per pair touched 64).  Subjects of few vertices, whose arcs
+    // take little time, have the pairs of one source cell summed first (a wave
+    // holds about half as many cells as pairs): C96 -> 1 degree 195 -> 177 us; for
+    // 16-gons the search costs what it saves (1.88 -> 1.93 ms).
     if (use_own && g_src) {
-        const int32_t s = k < nnz ? col[k] : 0;
-        for (int i = lane; i < 64 * 12; i += 64) {
-            const int pair = i / 12, e = i - 12 * pair;
-            const int64_t sp = __shfl(s, pair, 64);
-            const double v = own[i];
-            if (v != 0.0) atomicAdd(g_src + 3 * (int64_t)src_vi[sp * src_nv + e / 3] + e % 3, v);
+        const int32_t s = k < nnz && !zero ? col[k] : -1;
+        if constexpr (sizeof(M) == 1) {
+            int leader = lane, place = 0, cells = 0;
+            for (uint64_t todo = __ballot(s >= 0); todo; ++cells) {
+                const int l = __builtin_ctzll(todo);
+                const int32_t sl = __builtin_amdgcn_readlane(s, l);
+                todo &= ~__ballot(s == sl);
+                if (s == sl) leader = l;
+                if (lane == l) place = cells;
+            }
+            __syncthreads();
+            if (leader != lane) {
+                double *to = own + kOwn<M> * leader;
+#pragma unroll
+                for (int i = 0; i < 12; ++i) atomicAdd(to + i, mine[i]);
+            } else if (s >= 0) {
+                lead[place] = (uint8_t)lane;
+            }
+            __syncthreads();
+            for (int i = lane; i < (cells * 12 + 63) / 64 * 64; i += 64) {
+                const int c = min(i / 12, cells - 1), e = i % 12, l = lead[c];
+                const int64_t sp = __shfl(s, l, 64);
+                const double v = i < cells * 12 ? own[kOwn<M> * l + e] : 0.0;
+                if (v != 0.0) atomicAdd(g_src + 3 * (int64_t)src_vi[sp * src_nv + e / 3] + e % 3, v);
+            }
+        } else {
+            if (s < 0) {
+#pragma unroll
+                for (int i = 0; i < 12; ++i) mine[i] = 0.0;
+            }
+            __syncthreads();
+            for (int i = lane; i < 64 * 12; i += 64) {
+                const int l = i / 12, e = i % 12;
+                const int64_t sp = __shfl(s, l, 64);
+                const double v = own[kOwn<M> * l + e];
+                if (v != 0.0) atomicAdd(g_src + 3 * (int64_t)src_vi[sp * src_nv + e / 3] + e % 3, v);
+            }
         }
     }
     if (!g_dst) return;
-    // the wave's destination rows: a lane per vertex, from the lines before and
-    // after it, then a lane per double
-    const int64_t last = rowid[min(nnz, k0 + 64) - 1] - r0 + 1;
+    // the destination rows: a lane per vertex, from the lines before and after it;
+    // then a lane per double
     const int n = (int)min((int64_t)window, last) * dst_nv;
+    __syncthreads();
     d3 g[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -378,9 +433,10 @@ __global__ void __launch_bounds__(64) k_clip_grad_arcs(
         const int r = i / dst_nv, v = i - r * dst_nv, u = v == 0 ? dst_nv - 1 : v - 1, v1 = v + 1 == dst_nv ? 0 : v + 1;
         const double *cell = dst_cells + 3 * (int64_t)dst_nv * (r0 + r), *line = rows + 3 * dst_nv * r;
         const d3 pu = load3(cell + 3 * u), pv = load3(cell + 3 * v), pn = load3(cell + 3 * v1);
+        const double cu = line[3 * u + 2] + acoef[r], cv = line[3 * v + 2] + acoef[r];
         d3 gp, gq, unused;
-        line_grad(pu, pv, LineSum{0.0, line[3 * u + 1] + line[3 * u + 2] * whole_sum(pu, pv)}, unused, gq);
-        line_grad(pv, pn, LineSum{line[3 * v] + line[3 * v + 2] * whole_sum(pv, pn), 0.0}, gp, unused);
+        line_grad(pu, pv, LineSum{0.0, line[3 * u + 1] + cu * whole_sum(pu, pv)}, unused, gq);
+        line_grad(pv, pn, LineSum{line[3 * v] + cv * whole_sum(pv, pn), 0.0}, gp, unused);
         g[t] = gq + gp;
     }
     __syncthreads();
@@ -405,7 +461,7 @@ __global__ void __launch_bounds__(64) k_clip_grad_arcs(
 }
 
 // The vertex pass through the clip pipeline (clip_area_backward) for the
-// pairs the boundary decomposition declines: list[0 .. *count), 64 per wave,
+// pairs the boundary arcs decline: list[0 .. *count), 64 per wave,
 // the waves striding over the list.  The list holds each wave's declined
 // pairs in order, so a window of 64 entries mostly shares rows: rows r0 ..
 // r0 + kGradRows - 1 of its first entry are summed in LDS, the rest go to
@@ -430,14 +486,16 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
     double *my_own = own + 12 * threadIdx.x;
     const int64_t total = *count;
     const int nacc = kGradRows * dst_nv * 3;
-    for (int64_t base = (int64_t)blockIdx.x * 64; base < total; base += (int64_t)gridDim.x * 64) {
+    // a short list is spread over all waves: fewer pairs a wave, fewer paths in it
+    const int64_t per = min((int64_t)64, (total + gridDim.x - 1) / gridDim.x);
+    for (int64_t base = (int64_t)blockIdx.x * per; base < total; base += (int64_t)gridDim.x * per) {
         const int64_t r0 = rowid[list[base]];
         for (int i = threadIdx.x; i < nacc; i += 64) lacc[i] = 0.0;
 #pragma unroll
         for (int i = 0; i < 12; ++i) my_own[i] = 0.0;
         __syncthreads();
         const int64_t i = base + threadIdx.x;
-        if (i < total) {
+        if (threadIdx.x < per && i < total) {
             const int64_t k = list[i];
             const double c = coef[k];
             const int64_t d = rowid[k];
@@ -619,7 +677,7 @@ bool apply_ready(const cr_regridder *R, bool transpose, int dtype, int64_t nf, i
 
 // Scratch of the reverse mode: w (n_to x nfields doubles, the field adjoint's
 // input), coef (a double per non-zero), rowid (an int32 per non-zero), list
-// (the non-zeros the boundary decomposition declines, at most one int32 per
+// (the non-zeros the boundary arcs decline, at most one int32 per
 // non-zero) and its count.
 struct BackwardScratch {
     double *w = nullptr, *coef = nullptr;
@@ -687,13 +745,13 @@ static void backward(const cr_regridder *R, const cr_grid *dst, const cr_grid *s
         coef = coef_b.p;
         rowid = rowid_b.p;
     }
-    hipLaunchKernelGGL(k_pair_rows, dim3(grid_for(F.nrows, B)), dim3(B), 0, s, F.rowptr.p, F.nrows, rowid);
+    row_ids(F, rowid, s);
     if (F.nnz)
         hipLaunchKernelGGL(k_pair_coef, dim3(grid_for(F.nnz, B)), dim3(B), 0, s, rowid, F.col.p, F.nnz,
                            (int)(transpose != 0), (int)(normalize != 0), kappa, a_to, nfields, x, xc, xf, gy, gc,
                            gf, coef);
     if (F.nnz) {
-        // most pairs by boundary decomposition; the pairs it declines through the clip pipeline
+        // most pairs by boundary arcs; the pairs that declines through the clip pipeline
         DevBuf<int32_t> list_b;
         DevBuf<uint32_t> count_b;
         int32_t *list = ws ? ws->list : nullptr;
@@ -708,25 +766,35 @@ static void backward(const cr_regridder *R, const cr_grid *dst, const cr_grid *s
         const size_t lds = (size_t)kGradRows * dst->nv * 3 * sizeof(double);
         const bool cd = R->stats.clip_with_dst != 0;
         const int window = arc_rows(dst->nv);
-        const size_t arcs_lds = ((size_t)window * dst->nv * 3 + (src->nv <= 4 ? 64 * 12 : 0)) * sizeof(double) +
-                                64 * (size_t)(cd ? src->nv : dst->nv);
-        auto vertex_pass = [&](auto nc) {
+        const size_t arcs_lds = (size_t)window * dst->nv * 3 * sizeof(double);
+        const AreaTerm area{normalize && !transpose ? y : nullptr, gy, a_to, F.rowptr.p, yc, yf, gc, gf, nfields,
+                            kappa};
+        auto vertex_pass = [&](auto nc, auto mask) {
             constexpr int NC = decltype(nc)::value;
-            hipLaunchKernelGGL(k_clip_grad_arcs<NC>, dim3(grid_for(F.nnz, 64)), dim3(64), arcs_lds, s, rowid, F.col.p,
-                               coef, F.nnz, dst->cells.p, dst->nv, dst->vidx.p, src->cells.p, src->nv, src->vidx.p,
-                               (int)cd, window, dst->private_vertices, g_dst_verts, g_src_verts, list, count);
+            hipLaunchKernelGGL((k_clip_grad_arcs<NC, decltype(mask)>), dim3(grid_for(F.nnz, 64)), dim3(64), arcs_lds, s,
+                               rowid, F.col.p, coef, F.nnz, dst->cells.p, dst->nv, dst->vidx.p, src->cells.p, src->nv,
+                               src->vidx.p, (int)cd, window, dst->private_vertices, area, g_dst_verts, g_src_verts,
+                               list, count);
             hipLaunchKernelGGL(k_clip_grad_list<NC>, dim3(kListBlocks), dim3(64), lds, s, rowid, F.col.p, coef,
                                dst->cells.p, dst->nv, dst->vidx.p, src->cells.p, src->nv, src->vidx.p,
                                R->stats.clip_with_dst, g_dst_verts, g_src_verts, (const int32_t *)list,
                                (const uint32_t *)count, F.nrows);
         };
-        if (clip_nv <= 4) vertex_pass(std::integral_constant<int, 4>());
-        else vertex_pass(std::integral_constant<int, 8>());
+        using C4 = std::integral_constant<int, 4>;
+        using C8 = std::integral_constant<int, 8>;
+        const int ns = cd ? src->nv : dst->nv;  // the subject's vertices: a bit each
+        auto with_clip = [&](auto nc) {
+            if (ns <= 8) vertex_pass(nc, uint8_t());
+            else if (ns <= 32) vertex_pass(nc, uint32_t());
+            else vertex_pass(nc, uint64_t());
+        };
+        if (clip_nv <= 4) with_clip(C4());
+        else with_clip(C8());
         CR_HIP(hipGetLastError());
     }
-    double *g_to = transpose ? g_src_verts : g_dst_verts;
-    const cr_grid *gto = transpose ? src : dst;
-    if (normalize && g_to) {
+    double *g_to = g_src_verts;
+    const cr_grid *gto = src;
+    if (normalize && transpose && g_to) {  // forward: with the pairs above
         const bool table = gto->private_vertices && gto->flipped == 0;  // slot -> vertex is the identity
         if (table && gto->nv == 4)
             hipLaunchKernelGGL(k_area_grad_table<4>, dim3(grid_for(n_to, 64)), dim3(128), 0, s, gto->cells.p, n_to,

@@ -232,15 +232,10 @@ __device__ WindowTile window_tile(int64_t s, int64_t nrows, const int64_t *__res
     return out;
 }
 
-// Row of every non-zero, and the non-zero indices 0..nnz-1 (sort payload).
-__global__ void k_plan_rows(int64_t nrows, const int64_t *__restrict__ rp, int32_t *__restrict__ row,
-                            int32_t *__restrict__ iota) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrows) return;
-    for (int64_t k = rp[r]; k < rp[r + 1]; ++k) {
-        row[k] = (int32_t)r;
-        iota[k] = (int32_t)k;
-    }
+// The non-zero indices 0..nnz-1 (sort payload).
+__global__ void k_plan_iota(int64_t nnz, int32_t *__restrict__ iota) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < nnz) iota[k] = (int32_t)k;
 }
 
 // prev[k] for the non-zeros of non-huge rows, from the non-zeros sorted by
@@ -744,8 +739,8 @@ void make_plan(const Csr &A, TilePlan &P, hipStream_t s) {
     DevBuf<int32_t> prev(nnz > 0 ? nnz : 1, s);
     if (nnz > 0) {
         DevBuf<int32_t> row(nnz, s), iota(nnz, s), scol(nnz, s), sk(nnz, s);
-        hipLaunchKernelGGL(k_plan_rows, dim3(grid_for(nrows, 256)), dim3(256), 0, s, nrows, A.rowptr.p, row.p,
-                           iota.p);
+        row_ids(A, row.p, s);
+        hipLaunchKernelGGL(k_plan_iota, dim3(grid_for(nnz, 256)), dim3(256), 0, s, nnz, iota.p);
         sort_pairs<int32_t, int32_t>(T, A.col.p, scol.p, iota.p, sk.p, nnz, col_bits, s);
         hipLaunchKernelGGL(k_plan_prev, dim3(grid_for(nnz, 256)), dim3(256), 0, s, nnz, scol.p, sk.p, row.p,
                            A.rowptr.p, (int64_t)G::kCols, (int64_t)G::kRows, prev.p);

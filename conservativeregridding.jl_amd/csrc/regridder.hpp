@@ -115,6 +115,8 @@ template <class In, class Out>
 void exclusive_sum(Temp &T, In in, Out out, int64_t n, hipStream_t s);
 template <class K, class V>
 void sort_pairs(Temp &T, const K *kin, K *kout, const V *vin, V *vout, int64_t n, int end_bit, hipStream_t s);
+// Row of every non-zero of A.
+void row_ids(const Csr &A, int32_t *row, hipStream_t s);
 // CSR(A^T) of the device CSR(A) F whose entry k lies in row coo_row[k].
 void csr_transpose(const Csr &F, const int32_t *coo_row, Csr &Bk, Temp &T, hipStream_t s);
 }  // namespace cr

@@ -474,8 +474,7 @@ CR_HD bool crossing_backward(const d3 &x, const d3 &g, const d3 &p1, const d3 &q
 }
 
 // ============================================================================
-// Backward by boundary arcs (no clip pipeline): edges_plan, then edges_arcs and
-// line_grad.
+// Backward by boundary arcs (no clip pipeline): pair_arcs, then line_grad.
 //
 // To first order the area of P = subject ∩ clip changes only by the motion of
 // the great circles that carry its boundary (the motion of a corner along them
@@ -501,203 +500,18 @@ CR_HD bool crossing_backward(const d3 &x, const d3 &g, const d3 &p1, const d3 &q
 // the subject, and end where a subject edge enters or at the next clip vertex,
 // so their sums are signed sums over those points.
 //
-// edges_plan returns false when the pair is near a configuration where the area
-// is not differentiable or where the decisions above could differ from the
-// forward clip's by rounding -- a subject vertex within ~1e-10 of a clip edge's
-// length from that edge (on its line between the lines through its corners), a
-// crossing within that distance of a clip corner or of another crossing on its
-// clip edge, an edge entering and leaving through neighbouring lines at one
-// point -- when a clip edge meets the subject's boundary more than twice, or
-// when a clip edge is degenerate (the forward's corner there is the crossing of
-// the neighbouring lines).  The caller then uses clip_area_backward.
+// pair_arcs returns false when the pair is near a configuration where the area is
+// not differentiable or where the decisions above could differ from the forward
+// clip's by rounding: a subject vertex within ~1e-10 of a clip edge's length from
+// two clip lines, two neighbouring ones that near one line, a crossing that near
+// a clip corner, an edge that enters and leaves at one point; or when a clip edge
+// meets the subject's boundary more than twice.  The caller then uses
+// clip_area_backward.  (A single subject vertex on a clip line is fine: the
+// decisions use the forward's side test, the two crossings it may make cancel.)
+// A clip edge without a length (a polar cell's, a padded polygon's) is no line;
+// its neighbours' crossing is the corner, as in the forward clip.
 // ============================================================================
 constexpr double kEdgeTol = 1e-10;
-
-// The crossings of one subject edge with the clip lines: the latest entry
-// (k_in, t_in) and the earliest exit (k_out, t_out); empty when its end points
-// lie outside one line.  The winners' neighbours' side values (against the lines
-// through their clip edge's first and last corner) are carried out of the
-// unrolled loop, so no array is indexed by a run-time line number (which would
-// put it in scratch memory).
-template <int NC>
-struct EdgeCut {
-    double t_in, t_out;
-    double bp_in, bq_in, fp_in, fq_in, btol_in, ftol_in;
-    double bp_out, bq_out, fp_out, fq_out, btol_out, ftol_out;
-    int k_in, k_out;
-    CR_HD void make(const double (&ap)[NC], const double (&aq)[NC], const double (&tol)[NC]) {
-        t_in = 0.0;
-        t_out = 1.0;
-        k_in = -1;
-        k_out = -1;
-        bp_in = bq_in = fp_in = fq_in = btol_in = ftol_in = 0.0;
-        bp_out = bq_out = fp_out = fq_out = btol_out = ftol_out = 0.0;
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            const bool pin = ap[k] >= 0.0, qin = aq[k] >= 0.0;
-            if (pin == qin) continue;
-            const double t = fabs(ap[k]) / (fabs(ap[k]) + fabs(aq[k]));
-            const int b = (k + NC - 1) % NC, f = (k + 1) % NC;
-            if (!pin && t > t_in) {
-                t_in = t;
-                k_in = k;
-                bp_in = ap[b];
-                bq_in = aq[b];
-                fp_in = ap[f];
-                fq_in = aq[f];
-                btol_in = tol[b];
-                ftol_in = tol[f];
-            }
-            if (pin && t < t_out) {
-                t_out = t;
-                k_out = k;
-                bp_out = ap[b];
-                bq_out = aq[b];
-                fp_out = ap[f];
-                fq_out = aq[f];
-                btol_out = tol[b];
-                ftol_out = tol[f];
-            }
-        }
-    }
-};
-
-struct EdgesPlan {
-    uint64_t full, part;  // subject edges inside the clip polygon as a whole, in part
-    unsigned corners;     // bit k: clip vertex k lies inside the subject
-};
-
-// The checks (false: use clip_area_backward) and the plan.  code(j, k_in,
-// k_out): the lines (or -1) through which edge j, a bit of `part`, enters and
-// leaves.  At most 64 subject vertices.
-template <int NC, class Code>
-CR_HD bool edges_plan(const double *clip, int nc, const double *subj, int ns, EdgesPlan &P, Code &&code) {
-    P.full = P.part = 0;
-    P.corners = 0;
-    d3 c[NC], n[NC];
-    double tol[NC];
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) c[k] = load3(clip + 3 * (k < nc ? k : nc - 1));
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-        n[k] = cross(c[k], c[(k + 1) % NC] - c[k]);
-        const double nn = dot(n[k], n[k]);
-        ok = ok && nn >= kDegenerateEdge2;
-        tol[k] = kEdgeTol * nn;  // |side| below this: within ~1e-10 edge lengths of the line
-    }
-    if (!ok) return false;
-    // vertices outside each line; a vertex on a clip line is a degenerate point
-    // only on the clip edge's segment (inside the lines through its two corners)
-    uint64_t out[NC];
-#pragma unroll
-    for (int k = 0; k < NC; ++k) out[k] = 0;
-    for (int j = 0; j < ns; ++j) {
-        const d3 v = load3(subj + 3 * j);
-        double a[NC];
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            a[k] = dot(n[k], v - c[k]);
-            out[k] |= (uint64_t)(a[k] < 0.0) << j;
-        }
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            const int b = (k + NC - 1) % NC, f = (k + 1) % NC;
-            ok = ok && !(fabs(a[k]) <= tol[k] && a[b] >= -tol[b] && a[f] >= -tol[f]);
-        }
-    }
-    if (!ok) return false;
-    const uint64_t all = ns >= 64 ? ~0ull : (1ull << ns) - 1ull;
-    auto next = [&](uint64_t m) { return ((m >> 1) | (m << (ns - 1))) & all; };  // bit j: vertex j + 1
-    uint64_t any_out = 0, apart = 0;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-        any_out |= out[k];
-        apart |= out[k] & next(out[k]);
-    }
-    P.full = ~any_out & next(~any_out & all) & all;
-    P.part = all & ~apart & ~P.full;
-    // the crossings on each clip edge (at most two): the first's place along the
-    // edge, and whether a clip-edge arc begins (the subject leaves) at the first
-    // and at the last
-    double u_lo[NC];
-    unsigned one = 0, two = 0, lo_leaves = 0, hi_leaves = 0;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) u_lo[k] = 0.0;
-    for (uint64_t left = P.part; left; left &= left - 1) {
-        const int j = __builtin_ctzll(left);
-        const d3 p = load3(subj + 3 * j), q = load3(subj + 3 * (j + 1 == ns ? 0 : j + 1));
-        double ap[NC], aq[NC];
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            ap[k] = dot(n[k], p - c[k]);
-            aq[k] = dot(n[k], q - c[k]);
-        }
-        EdgeCut<NC> cut;
-        cut.make(ap, aq, tol);
-        if (cut.k_in >= 0 && cut.k_out >= 0 && fabs(cut.t_in - cut.t_out) <= kEdgeTol) return false;
-        if (!(cut.t_in < cut.t_out)) {
-            P.part &= ~(1ull << j);
-            continue;
-        }
-        code(j, cut.k_in, cut.k_out);
-#pragma unroll
-        for (int side = 0; side < 2; ++side) {
-            const int k = side == 0 ? cut.k_in : cut.k_out;
-            if (k < 0) continue;
-            // the crossing's place along clip edge k: its side values (linear
-            // along the chord) against the line through the edge's first corner
-            // (0 there, growing along the edge) and through its last
-            const double t = side == 0 ? cut.t_in : cut.t_out;
-            const double u = side == 0 ? (1.0 - t) * cut.bp_in + t * cut.bq_in
-                                       : (1.0 - t) * cut.bp_out + t * cut.bq_out;
-            const double v = side == 0 ? (1.0 - t) * cut.fp_in + t * cut.fq_in
-                                       : (1.0 - t) * cut.fp_out + t * cut.fq_out;
-            const double utol = side == 0 ? cut.btol_in : cut.btol_out;
-            if (u <= utol || v <= (side == 0 ? cut.ftol_in : cut.ftol_out)) return false;  // at a clip corner
-            const unsigned bit = 1u << k, leaves = side == 1 ? bit : 0u;
-            if (two & bit) return false;
-            double first = 0.0;
-#pragma unroll
-            for (int m = 0; m < NC; ++m)
-                if (m == k) {
-                    first = u_lo[m];
-                    if (!(one & bit) || u < first) u_lo[m] = u;
-                }
-            if (!(one & bit)) {
-                one |= bit;
-                lo_leaves |= leaves;
-                hi_leaves |= leaves;
-            } else {
-                if (fabs(u - first) <= utol) return false;
-                two |= bit;
-                if (u > first) hi_leaves = (hi_leaves & ~bit) | leaves;
-                else lo_leaves = (lo_leaves & ~bit) | leaves;
-            }
-        }
-    }
-    if (two & ~(lo_leaves ^ hi_leaves)) return false;  // not an arc's two ends
-    // a clip vertex's state is that after the last crossing before it along the
-    // clip boundary; with no crossing P is the clip polygon (some subject vertex
-    // outside it) or the subject
-    if (one) {
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            bool found = false;
-#pragma unroll
-            for (int s = 1; s <= NC; ++s) {
-                const int m = (k - s + NC) % NC;
-                if (!found && (one >> m & 1u)) {
-                    P.corners |= (hi_leaves >> m & 1u) << k;
-                    found = true;
-                }
-            }
-        }
-    } else if (any_out) {
-        P.corners = (1u << NC) - 1u;
-    }
-    return true;
-}
 
 // M_p and M_q of a line's arcs.
 struct LineSum {
@@ -714,48 +528,6 @@ CR_HD double whole_sum(const d3 &p, const d3 &q) {
     return 0.5 * dot(e, e);
 }
 
-// The arcs of a plan: arc(j, sums) for the part of every subject edge of `part`,
-// and S[k] = the sums of the parts of clip edge k inside the subject.  lines(j,
-// k_in, k_out) gives back what code stored.
-template <int NC, class Lines, class Arc>
-CR_HD void edges_arcs(const double *clip, int nc, const double *subj, int ns, const EdgesPlan &P, Lines &&lines,
-                      Arc &&arc, LineSum (&S)[NC]) {
-#pragma unroll
-    for (int k = 0; k < NC; ++k) S[k] = LineSum{0.0, 0.0};
-    for (uint64_t left = P.part; left; left &= left - 1) {
-        const int j = __builtin_ctzll(left);
-        int line[2];
-        lines(j, line[0], line[1]);
-        const d3 p = load3(subj + 3 * j), q = load3(subj + 3 * (j + 1 == ns ? 0 : j + 1));
-        d3 end[2] = {p, q};
-#pragma unroll
-        for (int side = 0; side < 2; ++side) {
-            const int k = line[side];
-            if (k < 0) continue;
-            const d3 c = load3(clip + 3 * k), e = load3(clip + 3 * (k + 1 == nc ? 0 : k + 1));
-            const d3 n = cross(c, e - c);
-            const d3 x = crossing(p, dot(n, p - c), q, dot(n, q - c));
-            end[side] = x;
-            // a clip-edge arc ends where the subject enters, begins where it leaves
-            const double h = side == 0 ? 0.5 : -0.5;
-            const double sp = -h * dot(x - e, x - e), sq = h * dot(x - c, x - c);
-#pragma unroll
-            for (int m = 0; m < NC; ++m)
-                if (m == k) {
-                    S[m].p += sp;
-                    S[m].q += sq;
-                }
-        }
-        arc(j, arc_sum(p, q, end[0], end[1]));
-    }
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-        const double h = whole_sum(load3(clip + 3 * (k < nc ? k : nc - 1)), load3(clip + 3 * (k + 1 < nc ? k + 1 : 0)));
-        if (P.corners >> k & 1u) S[k].p += h;
-        if (P.corners >> ((k + 1) % NC) & 1u) S[k].q += h;
-    }
-}
-
 // The derivative of the area w.r.t. the vertices p, q of a boundary line (zero
 // for a line of no length).
 CR_HD void line_grad(const d3 &p, const d3 &q, const LineSum &S, d3 &gp, d3 &gq) {
@@ -763,6 +535,201 @@ CR_HD void line_grad(const d3 &p, const d3 &q, const LineSum &S, d3 &gp, d3 &gq)
     const double nn = dot(n, n), f = nn > 0.0 ? -1.0 / nn : 0.0;
     gp = (f * S.p) * n;
     gq = (f * S.q) * n;
+}
+
+// The vertices of clip line k of NC (padding: a cell of nc < NC vertices repeats
+// its last one, and line NC - 1 closes the ring).
+template <int NC>
+CR_HD int clip_first(int k, int nc) {
+    return k < nc ? k : nc - 1;
+}
+template <int NC>
+CR_HD int clip_second(int k, int nc) {
+    return k + 1 == NC ? 0 : clip_first<NC>(k + 1, nc);
+}
+
+// One interval of the subject edge p -> q: where it enters through a line and
+// where it leaves, the side values' sizes at p and q against that line.
+struct EdgeCut {
+    double p_in, q_in, p_out, q_out;  // the chord parameter is p / (p + q)
+    int k_in, k_out;
+};
+
+// The arcs of a pair: `full`, a bit per subject edge wholly inside the clip
+// polygon; arc(i, j, sums) for the i-th subject edge inside it in part, edge j
+// (returns false if it has no room: the pair is declined); S[k] for clip line k.
+// M: an unsigned integer of at least ns bits.
+template <int NC, class M, class Arc>
+CR_HD bool pair_arcs(const double *clip, int nc, const double *subj, int ns, M &full, LineSum (&S)[NC], Arc &&arc) {
+    // side values n.(v - c) of clip line k as n.(v - o) - h, o the first clip vertex
+    // (v - o is exact, both terms are of the cells' size): 3 FMAs a line
+    const d3 o = load3(clip);
+    d3 n[NC];
+    double h[NC], tol[NC];
+    {
+        d3 c = o;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            S[k] = LineSum{0.0, 0.0};
+            const d3 c1 = load3(clip + 3 * clip_second<NC>(k, nc));
+            n[k] = cross(c, c1 - c);
+            const double nn = dot(n[k], n[k]);
+            tol[k] = kEdgeTol * nn;  // |side| below this: within ~1e-10 edge lengths of the line
+            if (nn < kDegenerateEdge2) {
+                n[k] = mk3(0.0, 0.0, 0.0);  // every point is inside
+                tol[k] = -1.0;              // and none is near
+            }
+            h[k] = dot(n[k], c - o);
+            c = c1;
+        }
+    }
+    auto side = [&](int k, const d3 &v) { return fma(n[k].x, v.x, fma(n[k].y, v.y, fma(n[k].z, v.z, -h[k]))); };
+    M out[NC], near = 0;  // subject vertices outside each line, near one
+#pragma unroll
+    for (int k = 0; k < NC; ++k) out[k] = 0;
+    for (int j = 0; j < ns; ++j) {
+        const d3 v = load3(subj + 3 * j) - o;
+        bool close = false;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            const double a = side(k, v);
+            out[k] |= (M)(a < 0.0) << j;
+            close = close || fabs(a) <= tol[k];
+        }
+        near |= (M)close << j;
+    }
+    const M all = (M)(~(M)0) >> (8 * sizeof(M) - ns);
+    auto next = [&](M m) { return (M)((m >> 1 | m << (ns - 1)) & all); };  // bit j: vertex j + 1
+    M any_out = 0, apart = 0;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        any_out |= out[k];
+        apart |= out[k] & next(out[k]);
+    }
+    full = ~any_out & next(~any_out & all) & all;
+    M part = all & ~apart & ~full;
+    for (M left = near; left; left &= left - 1) {
+        const int j = __builtin_ctzll((unsigned long long)left), j1 = j + 1 == ns ? 0 : j + 1;
+        const d3 v = load3(subj + 3 * j) - o, w = load3(subj + 3 * j1) - o;
+        int lines = 0;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            if (!(fabs(side(k, v)) <= tol[k])) continue;
+            ++lines;
+            if (!(fabs(side(k, w)) <= tol[k])) continue;
+            // an edge along the line: declined unless another line keeps it away
+            bool away = false;
+#pragma unroll
+            for (int m = 0; m < NC; ++m) away = away || (m != k && (out[m] & next(out[m])) >> j & 1);
+            if (!away) return false;
+        }
+        if (lines > 1) return false;
+    }
+    // the crossings on each clip edge (at most two): the first's place along the
+    // edge, and whether a clip-edge arc begins (the subject leaves) at the first
+    // and at the last
+    double u_lo[NC];
+    unsigned one = 0, two = 0, lo_leaves = 0, hi_leaves = 0, none = 0;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) u_lo[k] = 0.0;
+    bool any_arc = full != 0;
+    int count = 0;
+    for (M left = part; left; left &= left - 1) {
+        const int j = __builtin_ctzll((unsigned long long)left);
+        const d3 p = load3(subj + 3 * j), q = load3(subj + 3 * (j + 1 == ns ? 0 : j + 1));
+        EdgeCut cut{0.0, 1.0, 1.0, 0.0, -1, -1};
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            const double ap = side(k, p - o), aq = side(k, q - o);
+            const bool pin = ap >= 0.0;
+            if (pin == (aq >= 0.0)) continue;
+            const double fp = fabs(ap), fq = fabs(aq);
+            // fp / (fp + fq) against the latest entry, the earliest exit
+            if (!pin && fp * cut.q_in > cut.p_in * fq) {
+                cut.p_in = fp;
+                cut.q_in = fq;
+                cut.k_in = k;
+            }
+            if (pin && fp * cut.q_out < cut.p_out * fq) {
+                cut.p_out = fp;
+                cut.q_out = fq;
+                cut.k_out = k;
+            }
+        }
+        if (cut.k_in >= 0 && cut.k_out >= 0) {
+            const double in = cut.p_in * (cut.p_out + cut.q_out), out_ = cut.p_out * (cut.p_in + cut.q_in);
+            if (fabs(in - out_) <= kEdgeTol * ((cut.p_in + cut.q_in) * (cut.p_out + cut.q_out))) return false;
+            if (in > out_) continue;  // outside
+        }
+        any_arc = true;
+        d3 end[2] = {p, q};
+#pragma unroll
+        for (int way = 0; way < 2; ++way) {
+            const int k = way == 0 ? cut.k_in : cut.k_out;
+            if (k < 0) continue;
+            // crossing() of the edge's end points
+            d3 x = (way == 0 ? cut.q_in : cut.q_out) * p + (way == 0 ? cut.p_in : cut.p_out) * q;
+            x = inv_norm(dot(x, x)) * x;
+            end[way] = x;
+            const d3 c0 = load3(clip + 3 * clip_first<NC>(k, nc)), c1 = load3(clip + 3 * clip_second<NC>(k, nc));
+            const d3 e = c1 - c0, d = x - c0, f = x - c1;
+            const double ee = dot(e, e), u = dot(d, e);
+            if (u <= kEdgeTol * ee || u >= (1.0 - kEdgeTol) * ee) return false;  // at a clip corner
+            // a clip-edge arc ends where the subject enters, begins where it leaves
+            const double half = way == 0 ? 0.5 : -0.5, sp = -half * dot(f, f), sq = half * dot(d, d);
+            const unsigned bit = 1u << k, leaves = way == 1 ? bit : 0u;
+            double first = 0.0;
+#pragma unroll
+            for (int m = 0; m < NC; ++m)
+                if (m == k) {
+                    S[m].p += sp;
+                    S[m].q += sq;
+                    first = u_lo[m];
+                    if (!(one & bit) || u < first) u_lo[m] = u;
+                }
+            if (two & bit) return false;
+            if (!(one & bit)) {
+                one |= bit;
+                lo_leaves |= leaves;
+                hi_leaves |= leaves;
+            } else {
+                two |= bit;
+                if (fabs(u - first) <= kEdgeTol * ee) none |= bit;  // out and in again at one point
+                if (u > first) hi_leaves = (hi_leaves & ~bit) | leaves;
+                else lo_leaves = (lo_leaves & ~bit) | leaves;
+            }
+        }
+        if (!arc(count++, j, arc_sum(p, q, end[0], end[1]))) return false;
+    }
+    if (two & ~(lo_leaves ^ hi_leaves)) return false;  // not an arc's two ends
+    // clip vertices inside the subject: a vertex's state is that after the last
+    // crossing before it along the clip boundary; with no crossing P is the
+    // subject, or the clip polygon if no subject edge lies in it
+    unsigned corners = 0;
+    one &= ~none;
+    if (one) {
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            bool found = false;
+#pragma unroll
+            for (int s = 1; s <= NC; ++s) {
+                const int m = (k - s + NC) % NC;
+                if (!found && (one >> m & 1u)) {
+                    corners |= (hi_leaves >> m & 1u) << k;
+                    found = true;
+                }
+            }
+        }
+    } else if (!any_arc) {
+        corners = (1u << NC) - 1u;
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        const double whole = whole_sum(load3(clip + 3 * clip_first<NC>(k, nc)), load3(clip + 3 * clip_second<NC>(k, nc)));
+        if (corners >> k & 1u) S[k].p += whole;
+        if (corners >> ((k + 1) % NC) & 1u) S[k].q += whole;
+    }
+    return true;
 }
 
 // coef * d(signed ring area)/d(vertices) through emit(slot, grad): one call per
