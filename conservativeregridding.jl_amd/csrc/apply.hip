@@ -157,7 +157,8 @@ __global__ void __launch_bounds__(64) k_apply_long(
 
 // Row of every non-zero: a block's rows hold one run of non-zeros, written in
 // order; each finds its row by bisection of the row starts in LDS.  (A thread per
-// row writing its own non-zeros took 45 us for 4.35 M, this 12.)
+// row writing its own non-zeros took 45 to 51 us for the 4.35 M of quarter degree ->
+// HEALPix 256; this 40, a tail of the blocks with the poles' rows, and 13 transposed.)
 __global__ void __launch_bounds__(256) k_row_ids(const int64_t *__restrict__ rowptr, int64_t nrows,
                                                  int32_t *__restrict__ row) {
     __shared__ int start[257];  // from the block's first non-zero
@@ -235,6 +236,8 @@ static void ensure_long_rows(const Csr &A, hipStream_t s) {
 }
 
 void finalize_regridder(cr_regridder *R, hipStream_t s) {
+    // (not the other way round: A's rows keep the order they were made in)
+    R->fwd.transposed = &R->bwd;
     // one buffer: both directions' reciprocal areas, the two counters, the two lists
     int64_t n[2], cap[2];
     for (int t = 0; t < 2; ++t) {

@@ -52,6 +52,8 @@ struct Csr {
     const double *inv_area = nullptr;
     const int32_t *wide = nullptr, *nwide = nullptr;
     int64_t wide_cap = 0;  // places in the list
+    // the transposed matrix, each of whose rows has its columns ascending; null: none
+    const Csr *transposed = nullptr;
     int tuned_variant = -1;    // FP32 kernel variant (cr_regrid_tune / set_variant); -1: default
     mutable std::atomic<int> default_variant{-1};  // the default FP32 variant chosen for this matrix; -1: not yet
     int f64_variant = -1;      // FP64 kernel variant; -1: default

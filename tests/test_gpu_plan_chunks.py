@@ -39,3 +39,26 @@ def test_plan_over_chunks(cr, orc, nrows):
             assert_same_plan(dev, orc.tile_plan(style, geom, rp, col, val, ncols))
     finally:
         cr._lib.lib.cr_regridder_destroy(h)
+
+
+@pytest.mark.parametrize("ncols", [1, 40, 1500])
+def test_plan_long_columns(cr, orc, ncols):
+    """Columns that hundreds to thousands of rows hold (the earlier row is looked up
+    in the transposed matrix): repeats inside a row, empty rows, columns last held
+    more than a tile's rows ago or only by rows too long for a tile."""
+    rng = np.random.default_rng(ncols)
+    nrows = 4000
+    n = rng.integers(0, 7, nrows)
+    n[1000:2200] = 0
+    n[::97] = 2500
+    rp = np.concatenate(([0], np.cumsum(n))).astype(np.int64)
+    col = rng.integers(0, ncols, rp[-1]).astype(np.int32)
+    val = rng.random(rp[-1]) + 0.1
+    h = raw_regridder(cr._lib, nrows, ncols, rp, col, val)
+    try:
+        for style, geom in ((ROUNDS, 0), (ROUNDS, 1), (EVEN, 0), (EVEN, 1)):
+            print(f"[case] plan columns ncols={ncols} style={style} geom={geom}", flush=True)
+            dev = device_plan(cr._lib, h, 0, style, geom, orc.empty_tile_plan)
+            assert_same_plan(dev, orc.tile_plan(style, geom, rp, col, val, ncols))
+    finally:
+        cr._lib.lib.cr_regridder_destroy(h)
