@@ -6,9 +6,9 @@
 //     -> k_cell_bounds: FP64 area + bounding cap of every cell
 //        space-filling-curve sort (cube face + Hilbert) of source caps +
 //        implicit 8-ary tree of caps (k_build_level)
-//        k_search<false/true>: one wave per curve-order cluster of 64 destination
-//        cells walks the tree with the cluster's cap, then every lane tests its
-//        cell against the cluster's leaf list; count pass + scan + fill pass
+//        k_search<false/true>: one wave per curve-order cluster of 16 destination
+//        cells walks the tree with the cluster's cap, then each cell's lanes test
+//        it against the cluster's leaf list; count pass + scan + fill pass
 //        emit candidates grouped by destination row in a deterministic order
 //   compute_intersection_areas with ConvexConvexSutherlandHodgman + GO.area
 //     -> k_clip_compact<4>: a uniform outside-one-edge test settles about a
@@ -107,24 +107,33 @@ __global__ void k_build_level(const float4 *__restrict__ child, int64_t nchild,
     parent[p] = parent_cap(child, c0, c1);
 }
 
-// Candidate search, one wave per 64 destination cells taken in space-filling-
-// curve order of their caps (a compact cluster).  The wave bounds its 64 caps
+// Candidate search, one wave per 16 (or 8) destination cells taken in space-filling-
+// curve order of their caps (a compact cluster).  The wave bounds its cells' caps
 // by one cap, walks the source tree level by level with that cap (lanes test
 // the children of the current frontier side by side; ballot + prefix count
 // compact the survivors into LDS), and ends with the list of source leaves
-// that touch the cluster.  Each lane then tests its own cap against that list
-// (LDS broadcast reads, no divergence).  A cluster whose frontier or leaf list
-// overflows the LDS lists is retried as 4 clusters of 16 lanes; the cells of
-// a 16-lane cluster that still overflows are walked one at a time by the
-// whole wave, which counts or writes the hits straight from its ballots (no
+// that touch the cluster.  The lanes of each cell then test its cap against that
+// list, a part each (LDS broadcast reads, no divergence).  The cells of a cluster
+// whose frontier or leaf list overflows the LDS lists are walked one at a time by a
+// wave each, which counts or writes the hits straight from its ballots (no
 // leaf list); only a cell whose frontier overflows even then walks the tree
 // alone (tree_query).  Every leaf that touches a cell's cap touches any cluster cap
 // that contains it and all of its ancestors, so every route emits exactly the
 // leaves whose caps touch the cell's cap, in a fixed order.  FILL=false
 // counts; FILL=true writes at the scanned offsets (never past the cell's
 // segment).
-constexpr int kSearchLeaves = 1024;
 constexpr int kSearchFront = 256;
+// 8 cells to a wave up to this many destination cells, where 16 leave the chip half
+// empty: 1 degree -> C48 (13 824 cells) 25 + 34 us against 33 + 55, from 49 k cells on
+// the same, at 786 k 420 + 485 against 270 + 367.
+constexpr int64_t kFewQueries = 32768;
+// From this many source cells to a destination cell lists of 1024 leaves, else 384: a
+// short list leaves room for three times the waves (quarter degree -> HEALPix 256 121
+// + 165 us against 249 + 364), one that overflows costs each of its cells a walk of its
+// own (builds at ratio 16 2.35 against 2.53 ms, at 7.7 3.86 against 3.97, at 4.7 the
+// same).
+constexpr int64_t kFineSources = 4;
+constexpr int kDeferredFront = 4096;
 
 template <int W>
 __device__ __forceinline__ float group_sum(float v) {
@@ -167,6 +176,7 @@ __device__ __forceinline__ float4 shfl4(const float4 &v, int src) {
 // The whole wave walks the tree with the (wave-uniform) cap wc and lists the
 // leaves that touch it in lcap/lid.  Returns the count, or -1 when a frontier
 // or the leaf list overflows (or wc cannot be bounded).
+template <int LEAVES>
 __device__ int coop_collect(const float4 &wc, const float4 *__restrict__ nodes, const Levels &lv,
                             const int32_t *__restrict__ perm, float4 *lcap, int32_t *lid,
                             int32_t (*front)[kSearchFront]) {
@@ -214,7 +224,7 @@ __device__ int coop_collect(const float4 &wc, const float4 *__restrict__ nodes, 
                 if (hit) {
                     if (lev > 1) {
                         if (pos < kSearchFront) front[cur ^ 1][pos] = (int32_t)child[u];
-                    } else if (pos < kSearchLeaves) {
+                    } else if (pos < LEAVES) {
                         lcap[pos] = cc[u];
                         lid[pos] = perm[child[u]];
                     }
@@ -223,151 +233,11 @@ __device__ int coop_collect(const float4 &wc, const float4 *__restrict__ nodes, 
             }
         }
         __syncthreads();
-        if (nn > (lev > 1 ? kSearchFront : kSearchLeaves)) return -1;
+        if (nn > (lev > 1 ? kSearchFront : LEAVES)) return -1;
         cur ^= 1;
         nf = nn;
     }
     return nf;
-}
-
-// The whole wave walks the tree once with the four 16-lane cluster caps
-// gc[0..3] (wave-uniform): the frontier is the union of what touches any of
-// them, and the leaf level lists, for each cluster g, the leaves that touch
-// gc[g] in lcap/lid[g * kSubLeaves ...] (n[g] of them, in tree order).  Each
-// lane then tests only its own cluster's list, a quarter of the lanes' region
-// and far fewer leaves than one 64-cell list.  Returns false when the union
-// frontier or a list overflows or a cap cannot be bounded; an empty cluster
-// (w < 0) gets an empty list.
-constexpr int kSubLeaves = kSearchLeaves / 4;
-
-__device__ bool coop_collect4(const float4 (&gc)[4], const float4 *__restrict__ nodes, const Levels &lv,
-                              const int32_t *__restrict__ perm, float4 *lcap, int32_t *lid,
-                              int32_t (*front)[kSearchFront], int (&n)[4]) {
-    const int lane = threadIdx.x;
-    bool live[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        if (gc[g].w >= 1.4f) return false;
-        live[g] = gc[g].w >= 0.0f;
-        n[g] = 0;
-    }
-    if (lv.top == 0) {  // a single leaf
-        __syncthreads();
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-            if (live[g] && caps_overlap(gc[g], nodes[0])) {
-                if (lane == 0) {
-                    lcap[g * kSubLeaves] = nodes[0];
-                    lid[g * kSubLeaves] = perm[0];
-                }
-                n[g] = 1;
-            }
-        __syncthreads();
-        return true;
-    }
-    __syncthreads();  // the previous lists are no longer read
-    if (lane == 0) front[0][0] = 0;
-    __syncthreads();
-    int cur = 0, nf = 1;
-    const uint64_t below = (1ull << lane) - 1ull;
-    for (int lev = lv.top; lev >= 1; --lev) {
-        const int64_t csize = lv.size[lev - 1], coff = lv.off[lev - 1];
-        const int tot = nf * kTreeFanout;
-        int nn = 0;
-        for (int base = 0; base < tot; base += 4 * 64) {
-            int64_t child[4];
-            float4 cc[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int t = base + 64 * u + lane;
-                child[u] = -1;
-                cc[u] = make_float4(0.f, 0.f, 0.f, -8.0f);
-                if (t < tot) {
-                    const int64_t ch = (int64_t)front[cur][t >> 3] * kTreeFanout + (t & 7);
-                    if (ch < csize) {
-                        child[u] = ch;
-                        cc[u] = nodes[coff + ch];
-                    }
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                bool h[4];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) h[g] = child[u] >= 0 && live[g] && caps_overlap(gc[g], cc[u]);
-                if (lev > 1) {
-                    const bool hit = h[0] || h[1] || h[2] || h[3];
-                    const uint64_t m = __ballot(hit);
-                    const int pos = nn + (int)__popcll(m & below);
-                    if (hit && pos < kSearchFront) front[cur ^ 1][pos] = (int32_t)child[u];
-                    nn += (int)__popcll(m);
-                } else {
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const uint64_t m = __ballot(h[g]);
-                        const int pos = n[g] + (int)__popcll(m & below);
-                        if (h[g] && pos < kSubLeaves) {
-                            lcap[g * kSubLeaves + pos] = cc[u];
-                            lid[g * kSubLeaves + pos] = perm[child[u]];
-                        }
-                        n[g] += (int)__popcll(m);
-                    }
-                }
-            }
-        }
-        __syncthreads();
-        if (lev > 1) {
-            if (nn > kSearchFront) return false;
-            cur ^= 1;
-            nf = nn;
-        }
-    }
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-        if (n[g] > kSubLeaves) return false;
-    return true;
-}
-
-// One lane's tests against the collected list (four independent tests per
-// step: a wave per SIMD has no other wave to hide a dependent chain).
-template <bool FILL>
-__device__ void lane_emit(const float4 &c, int64_t d, int nleaf, const float4 *lcap, const int32_t *lid,
-                          int64_t *__restrict__ count_or_offset, int32_t *__restrict__ cand_src,
-                          int32_t *__restrict__ cand_dst) {
-    if (FILL) {
-        int64_t pos = count_or_offset[d];
-        const int64_t end = count_or_offset[d + 1];
-        int j = 0;
-        for (; j + 4 <= nleaf; j += 4) {
-            bool h[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) h[u] = caps_overlap(c, lcap[j + u]);
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (h[u] && pos < end) {
-                    cand_src[pos] = lid[j + u];
-                    cand_dst[pos] = (int32_t)d;
-                    ++pos;
-                }
-        }
-        for (; j < nleaf; ++j)
-            if (caps_overlap(c, lcap[j]) && pos < end) {
-                cand_src[pos] = lid[j];
-                cand_dst[pos] = (int32_t)d;
-                ++pos;
-            }
-    } else {
-        int c0 = 0, c1 = 0, c2 = 0, c3 = 0;
-        int j = 0;
-        for (; j + 4 <= nleaf; j += 4) {
-            c0 += caps_overlap(c, lcap[j]);
-            c1 += caps_overlap(c, lcap[j + 1]);
-            c2 += caps_overlap(c, lcap[j + 2]);
-            c3 += caps_overlap(c, lcap[j + 3]);
-        }
-        for (; j < nleaf; ++j) c0 += caps_overlap(c, lcap[j]);
-        count_or_offset[d] = (int64_t)(c0 + c1 + c2 + c3);
-    }
 }
 
 template <bool FILL>
@@ -394,9 +264,8 @@ __device__ void lane_walk(const float4 &c, int64_t d, const float4 *__restrict__
 // One cell (cap qc, row d, wave-uniform) walked by the whole wave; the leaf
 // level is tested 64 children at a time and the hits are counted, or written
 // in order at the cell's offset, straight from the ballot (no leaf list).
-// The frontier lives in `scratch` (kSearchBigFront entries).  Returns false
+// The frontier lives in `scratch` (kDeferredFront entries).  Returns false
 // when a frontier overflows (nothing was counted or written then).
-constexpr int kSearchBigFront = kSearchLeaves * 4;  // int32 entries in the lcap storage
 
 template <bool FILL>
 __device__ bool coop_emit_one(const float4 &qc, int64_t d, const float4 *__restrict__ nodes, const Levels &lv,
@@ -404,8 +273,8 @@ __device__ bool coop_emit_one(const float4 &qc, int64_t d, const float4 *__restr
                               int64_t *__restrict__ count_or_offset, int32_t *__restrict__ cand_src,
                               int32_t *__restrict__ cand_dst) {
     const int lane = threadIdx.x;
-    int32_t *fa = scratch, *fb = scratch + kSearchBigFront / 2;
-    const int cap = kSearchBigFront / 2;
+    int32_t *fa = scratch, *fb = scratch + kDeferredFront / 2;
+    const int cap = kDeferredFront / 2;
     __syncthreads();
     if (lane == 0) fa[0] = 0;
     __syncthreads();
@@ -476,69 +345,68 @@ __device__ bool coop_emit_one(const float4 &qc, int64_t d, const float4 *__restr
     return true;
 }
 
-template <bool FILL>
+// One wave per CELLS destination cells in curve order: the wave walks the tree with
+// the cap around their caps, then 64 / CELLS lanes to a cell test a part of the
+// leaves listed each.
+//
+// Bound by the latency of the walk (a chain of barriers, one a level) and of the LDS
+// reads, so by the waves a CU holds, which the lists' LDS decides.  Quarter degree ->
+// HEALPix 256 (786 k cells, 7.3 M candidates): count 120 and fill 165 us, with the
+// deferred cells 369 in all; 64 cells to a wave as four clusters of one walk, a lane to
+// a cell, took 297 and 426, 762 in all; 1 degree -> C48 55 against 326 us (one wave to
+// a CU there, and the clusters whose lists overflowed one after the other).
+template <bool FILL, int CELLS, int LEAVES>
 __global__ void __launch_bounds__(64) k_search(const float4 *__restrict__ qcap,
-                                               const int32_t *__restrict__ qorder, int64_t nq,
-                                               const float4 *__restrict__ nodes, Levels lv,
-                                               const int32_t *__restrict__ perm,
-                                               int64_t *__restrict__ count_or_offset,
-                                               int32_t *__restrict__ cand_src,
-                                               int32_t *__restrict__ cand_dst,
-                                               int32_t *__restrict__ defer, unsigned *__restrict__ ndefer) {
-    __shared__ float4 lcap[kSearchLeaves];
-    __shared__ int32_t lid[kSearchLeaves];
+                                                   const int32_t *__restrict__ qorder, int64_t nq,
+                                                   const float4 *__restrict__ nodes, Levels lv,
+                                                   const int32_t *__restrict__ perm,
+                                                   int64_t *__restrict__ count_or_offset,
+                                                   int32_t *__restrict__ cand_src, int32_t *__restrict__ cand_dst,
+                                                   int32_t *__restrict__ defer, unsigned *__restrict__ ndefer) {
+    constexpr int PARTS = 64 / CELLS;
+    __shared__ float4 lcap[LEAVES];
+    __shared__ int32_t lid[LEAVES];
     __shared__ int32_t front[2][kSearchFront];
-    const int lane = threadIdx.x;
-    const int64_t i = (int64_t)blockIdx.x * 64 + lane;
+    const int lane = threadIdx.x, cell = lane % CELLS, part = lane / CELLS;
+    const int64_t i = (int64_t)blockIdx.x * CELLS + cell;
     const bool active = i < nq;
     const int64_t d = active ? qorder[i] : 0;
     const float4 c = active ? qcap[d] : make_float4(0.f, 0.f, 0.f, 0.f);
-
-    // four 16-cell clusters in one walk
-    const float4 gcap = group_cap<16>(c, active);
-    {
-        float4 gcs[4];
-        int n4[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) gcs[g] = shfl4(gcap, 16 * g);
-        if (coop_collect4(gcs, nodes, lv, perm, lcap, lid, front, n4)) {
-            const int g = lane >> 4;
-            const int n = g == 0 ? n4[0] : (g == 1 ? n4[1] : (g == 2 ? n4[2] : n4[3]));
-            if (active)
-                lane_emit<FILL>(c, d, n, lcap + g * kSubLeaves, lid + g * kSubLeaves, count_or_offset, cand_src,
-                                cand_dst);
-            return;
-        }
-    }
-    // the four clusters one after the other with full-size lists; the lanes of
-    // a cluster that still overflows walk the tree alone, all together at the end
-    int n;
-    bool walk = false;
-    for (int g = 0; g < 4; ++g) {
-        const float4 gc = shfl4(gcap, 16 * g);
-        n = coop_collect(gc, nodes, lv, perm, lcap, lid, front);
-        if ((lane >> 4) != g) continue;
-        if (n >= 0) {
-            if (active) lane_emit<FILL>(c, d, n, lcap, lid, count_or_offset, cand_src, cand_dst);
-        } else {
-            walk = true;
-        }
-    }
-    // cells left over (about 0.15% of them, with hundreds to thousands of
-    // candidates each): listed by the count pass for k_search_deferred, which
-    // gives each its own wave (walked here one at a time they would hold this
-    // wave for a long tail)
-    if (!FILL) {
-        const bool mine = walk && active;
-        const uint64_t m = __ballot(mine);
-        if (m) {
-            const int leader = (int)__ffsll((long long)m) - 1;
+    const int n = coop_collect<LEAVES>(shfl4(group_cap<CELLS>(c, active), 0), nodes, lv, perm, lcap, lid, front);
+    if (n < 0) {  // to k_search_deferred, listed by the count pass
+        if (!FILL) {
+            const uint64_t m = __ballot(active && part == 0);
             unsigned base = 0;
-            if (lane == leader) base = atomicAdd(ndefer, (unsigned)__popcll(m));
-            base = (unsigned)__shfl((int)base, leader, 64);
-            if (mine) defer[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = (int32_t)d;
+            if (lane == 0) base = atomicAdd(ndefer, (unsigned)__popcll(m));
+            base = (unsigned)__shfl((int)base, 0, 64);
+            if (active && part == 0) defer[base + (unsigned)cell] = (int32_t)d;
         }
+        return;
     }
+    const int a = n * part / PARTS, b = n * (part + 1) / PARTS;
+    int hits = 0;
+#pragma unroll 4
+    for (int j = a; j < b; ++j) hits += caps_overlap(c, lcap[j]);
+    int before = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q) {
+        const int h = __shfl(hits, q * CELLS + cell, 64);
+        before += q < part ? h : 0;
+        all += h;
+    }
+    if (!active) return;
+    if (!FILL) {
+        if (part == 0) count_or_offset[d] = all;
+        return;
+    }
+    int64_t pos = count_or_offset[d] + before;
+    const int64_t end = count_or_offset[d + 1];
+    for (int j = a; j < b; ++j)
+        if (caps_overlap(c, lcap[j]) && pos < end) {
+            cand_src[pos] = lid[j];
+            cand_dst[pos] = (int32_t)d;
+            ++pos;
+        }
 }
 
 // The listed cells, one wave each (grid-stride over the list): the whole wave
@@ -554,7 +422,7 @@ __global__ void __launch_bounds__(64) k_search_deferred(const float4 *__restrict
                                                         int64_t *__restrict__ count_or_offset,
                                                         int32_t *__restrict__ cand_src,
                                                         int32_t *__restrict__ cand_dst) {
-    __shared__ int32_t scratch[kSearchBigFront];
+    __shared__ int32_t scratch[kDeferredFront];
     const unsigned n = *ndefer;
     for (unsigned i = blockIdx.x; i < n; i += gridDim.x) {
         const int64_t d = defer[i];
@@ -1107,18 +975,25 @@ void build_regridder(cr_regridder *R, const cr_grid *dst, const cr_grid *src,
 
     // 3. candidate search: destination cells in curve order, count, scan, fill
     DevBuf<int64_t> cand_off(nd + 1, s);
-    const unsigned qblocks = grid_for(nd, 64);
+    const bool few = nd <= kFewQueries, fine = ns > kFineSources * nd;
+    const unsigned qblocks = grid_for(nd, few ? 8 : 16);
     DevBuf<int32_t> defer(nd, s);  // cells whose clusters overflow, listed by the count pass
     DevBuf<unsigned> ndefer(1, s);
     CR_HIP(hipMemsetAsync(ndefer.p, 0, sizeof(unsigned), s));
     constexpr unsigned kDeferBlocks = 2048;
+    const auto search = [&](auto fill, int64_t *count_or_offset, int32_t *out_src, int32_t *out_dst) {
+        constexpr bool FILL = decltype(fill)::value;
+        const auto kernel = few ? (fine ? k_search<FILL, 8, 1024> : k_search<FILL, 8, 384>)
+                                : (fine ? k_search<FILL, 16, 1024> : k_search<FILL, 16, 384>);
+        hipLaunchKernelGGL(kernel, dim3(qblocks), dim3(64), 0, s, cap_dst.p, qorder, nd, nodes.p, lv, perm,
+                           count_or_offset, out_src, out_dst, defer.p, ndefer.p);
+        hipLaunchKernelGGL(k_search_deferred<FILL>, dim3(kDeferBlocks), dim3(64), 0, s, cap_dst.p, defer.p, ndefer.p,
+                           nodes.p, lv, perm, count_or_offset, out_src, out_dst);
+    };
     {
         DevBuf<int64_t> cand_cnt(nd + 1, s);
         CR_HIP(hipMemsetAsync(cand_cnt.p + nd, 0, sizeof(int64_t), s));
-        hipLaunchKernelGGL(k_search<false>, dim3(qblocks), dim3(64), 0, s, cap_dst.p, qorder, nd, nodes.p,
-                           lv, perm, cand_cnt.p, (int32_t *)nullptr, (int32_t *)nullptr, defer.p, ndefer.p);
-        hipLaunchKernelGGL(k_search_deferred<false>, dim3(kDeferBlocks), dim3(64), 0, s, cap_dst.p, defer.p,
-                           ndefer.p, nodes.p, lv, perm, cand_cnt.p, (int32_t *)nullptr, (int32_t *)nullptr);
+        search(std::false_type{}, cand_cnt.p, nullptr, nullptr);
         CR_HIP(hipGetLastError());
         exclusive_sum(T, cand_cnt.p, cand_off.p, nd + 1, s);
     }
@@ -1139,12 +1014,7 @@ void build_regridder(cr_regridder *R, const cr_grid *dst, const cr_grid *src,
         CR_HIP(hipMemsetAsync(cand_src.p, 0, cand_src.bytes(), s));
         CR_HIP(hipMemsetAsync(cand_dst.p, 0, cand_dst.bytes(), s));
     }
-    if (ncand) {
-        hipLaunchKernelGGL(k_search<true>, dim3(qblocks), dim3(64), 0, s, cap_dst.p, qorder, nd, nodes.p,
-                           lv, perm, cand_off.p, cand_src.p, cand_dst.p, defer.p, ndefer.p);
-        hipLaunchKernelGGL(k_search_deferred<true>, dim3(kDeferBlocks), dim3(64), 0, s, cap_dst.p, defer.p,
-                           ndefer.p, nodes.p, lv, perm, cand_off.p, cand_src.p, cand_dst.p);
-    }
+    if (ncand) search(std::true_type{}, cand_off.p, cand_src.p, cand_dst.p);
     CR_HIP(hipGetLastError());
     tm.mark();  // 3
 

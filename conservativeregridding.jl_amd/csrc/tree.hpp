@@ -109,9 +109,10 @@ CR_HD float4 parent_cap(const float4 *child, int64_t c0, int64_t c1) {
 }
 
 CR_HD bool caps_overlap(const float4 &a, const float4 &b) {
+    // the sum written out: a test made twice (count and fill) rounds alike
     float dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z;
     float rr = a.w + b.w;
-    return dx * dx + dy * dy + dz * dz <= rr * rr;
+    return fmaf(dz, dz, fmaf(dy, dy, dx * dx)) <= rr * rr;
 }
 
 // Level sizes of the implicit kTreeFanout-ary tree over n leaves (level 0).
