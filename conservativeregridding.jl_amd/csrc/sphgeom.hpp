@@ -505,8 +505,9 @@ CR_HD bool crossing_backward(const d3 &x, const d3 &g, const d3 &p1, const d3 &q
 // clip's by rounding: a subject vertex within ~1e-10 of a clip edge's length from
 // two clip lines, two neighbouring ones that near one line, a crossing that near
 // a clip corner, an edge that enters and leaves at one point; or when a clip edge
-// meets the subject's boundary more than twice.  The caller then uses
-// clip_area_backward.  (A single subject vertex on a clip line is fine: the
+// meets the subject's boundary more than twice; or when the boundaries meet only
+// where the subject goes out and in again at one point (a reflex vertex on a clip
+// edge).  The caller then uses clip_area_backward.  (A single subject vertex on a clip line is fine: the
 // decisions use the forward's side test, the two crossings it may make cancel.)
 // A clip edge without a length (a polar cell's, a padded polygon's) is no line;
 // its neighbours' crossing is the corner, as in the forward clip.
@@ -707,6 +708,7 @@ CR_HD bool pair_arcs(const double *clip, int nc, const double *subj, int ns, M &
     // subject, or the clip polygon if no subject edge lies in it
     unsigned corners = 0;
     one &= ~none;
+    if (none && !one) return false;  // one cell inside the other but for a touch: which, the arcs there do not tell
     if (one) {
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
