@@ -507,8 +507,11 @@ CR_HD bool crossing_backward(const d3 &x, const d3 &g, const d3 &p1, const d3 &q
 // a clip corner, an edge that enters and leaves at one point; or when a clip edge
 // meets the subject's boundary more than twice; or when the boundaries meet only
 // where the subject goes out and in again at one point (a reflex vertex on a clip
-// edge).  The caller then uses clip_area_backward.  (A single subject vertex on a clip line is fine: the
-// decisions use the forward's side test, the two crossings it may make cancel.)
+// edge), or nowhere while a subject vertex is that near a clip line (cells that only
+// touch: n.(v - o) - h may round to another sign than the forward's n.(v - c)).  The
+// caller then uses clip_area_backward.  (Any other single subject vertex on a clip
+// line is fine, on whichever side it comes out: its side counts as one for both of
+// its edges, and the two crossings it may make cancel.)
 // A clip edge without a length (a polar cell's, a padded polygon's) is no line;
 // its neighbours' crossing is the corner, as in the forward clip.
 // ============================================================================
@@ -723,6 +726,7 @@ CR_HD bool pair_arcs(const double *clip, int nc, const double *subj, int ns, M &
             }
         }
     } else if (!any_arc) {
+        if (near) return false;
         corners = (1u << NC) - 1u;
     }
 #pragma unroll

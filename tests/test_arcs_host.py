@@ -50,3 +50,32 @@ def test_reflex_vertex_at_a_clip_edge(host, orc, shape, seed):
                 # decisions within ~1e-10 edge lengths may go either way
                 for g, want in zip(got, (gs, gc)):
                     assert np.abs(g - want).max() <= 1e-9 * np.abs(gc).max(), (h, eps, turn)
+
+
+def test_cells_that_only_touch(host):
+    """A vertex of a quad on a clip edge from outside: rounding decides whether the
+    intersection is empty or a sliver of ~1e-16 edge lengths; its gradient is small
+    either way."""
+    rng = np.random.default_rng(3)
+    square, planned, slivers = np.array([(0.0, 0.0), (1.0, 0.0), (1.0, 1.0), (0.0, 1.0)]), 0, 0
+    for it in range(60000):
+        if it % 100 == 0:
+            seed, turn = int(rng.integers(1 << 30)), int(rng.integers(4))
+            clip = np.roll(plane(square, 0.01, seed), turn, axis=0)
+        # the touching vertex: a point of the clip edge as the doubles have it
+        t = rng.uniform(0.1, 0.9)
+        k = (0 + turn) % 4
+        tip = (1 - t) * clip[k] + t * clip[(k + 1) % 4]
+        tip /= np.linalg.norm(tip)
+        rest = plane([(t - 0.4, -0.6), (t + 0.1, -1.0), (t + 0.5, -0.5)], 0.01, seed)
+        subj = np.concatenate([tip[None], rest])
+        if arcs_host.area(host, subj, clip) <= 0.0:
+            continue
+        slivers += 1
+        got = arcs_host.grad(host, subj, clip)
+        if got is None:
+            continue
+        planned += 1
+        # a sliver of depth d has a derivative of the order of d; the whole cell's is ~0.01
+        assert max(np.abs(got[0]).max(), np.abs(got[1]).max()) <= 1e-11, it
+    assert slivers > 1000

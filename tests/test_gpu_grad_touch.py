@@ -1,5 +1,5 @@
-"""Vertex gradients of cells that touch: each pair of cells by itself (far from the
-others), against the oracle's dual numbers of that pair."""
+"""Vertex gradients of cells that touch, each pair of cells by itself (far from the
+others)."""
 import numpy as np
 import pytest
 import torch
@@ -43,3 +43,30 @@ def test_reflex_vertex_at_a_clip_edge(cr, orc, shape):
         assert np.abs(g_dst[4 * i:4 * i + 4] - gd).max() <= tol, EPS[i]
         n = len(src[i])
         assert np.abs(g_src[n * i:n * i + n] - gs).max() <= tol, EPS[i]
+
+
+def test_cells_that_only_touch(cr):
+    """A vertex of the source quad on an edge of the destination quad, from outside:
+    whether rounding makes that a pair (threshold_rel = 0 keeps every sliver) or not,
+    the gradient is that of a sliver."""
+    print("[case] touching cells", flush=True)
+    rng = np.random.default_rng(7)
+    h, square = 0.004, np.array([(0.0, 0.0), (1.0, 0.0), (1.0, 1.0), (0.0, 1.0)])
+    dst, src = [], []
+    for lat in np.linspace(-1.2, 1.2, 100):
+        for lon in np.linspace(0.0, 2 * np.pi, 60, endpoint=False):
+            c = np.array([np.cos(lat) * np.cos(lon), np.cos(lat) * np.sin(lon), np.sin(lat)])
+            u = np.cross(c, rng.standard_normal(3))
+            u /= np.linalg.norm(u)
+            frame = np.stack([u, np.cross(c, u), c])
+            place = lambda xy: (lambda p: p / np.linalg.norm(p, axis=1, keepdims=True))(  # noqa: E731
+                np.concatenate([h * np.asarray(xy), np.ones((len(xy), 1))], 1) @ frame)
+            d, turn, t = place(square), int(rng.integers(4)), rng.uniform(0.1, 0.9)
+            tip = (1 - t) * d[0] + t * d[1]
+            dst.append(np.roll(d, turn, axis=0))
+            src.append(np.concatenate([(tip / np.linalg.norm(tip))[None],
+                                       place([(t - 0.4, -0.6), (t + 0.1, -1.0), (t + 0.5, -0.5)])]))
+    R, g_dst, g_src = _pair_grads(cr, dst, src, True, threshold_rel=0.0)
+    assert R.intersections.nnz > 100
+    # a sliver of depth d has a derivative of the order of d (1e-16 here); the whole cell's is h / 2
+    assert max(np.abs(g_dst).max(), np.abs(g_src).max()) <= 1e-9 * h
