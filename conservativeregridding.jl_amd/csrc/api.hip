@@ -87,7 +87,7 @@ cr_status cr_regridder_from_csr(cr_regridder **R, int64_t n_dst, int64_t n_src, 
             upload(r->a_dst, dst_areas, n_dst, s);
             upload(r->a_src, src_areas, n_src, s);
             finalize_regridder(r, s);
-            CR_HIP(hipStreamSynchronize(s));
+            synchronise(s);
             r->stats.n_dst = n_dst;
             r->stats.n_src = n_src;
             r->stats.nnz = nnz;
@@ -171,6 +171,10 @@ cr_status cr_regridder_copy_areas(const cr_regridder *R, double *dst_areas, doub
     });
 }
 
-void cr_regridder_destroy(cr_regridder *R) { delete R; }
+void cr_regridder_destroy(cr_regridder *R) {
+    if (!R) return;
+    ReleaseScope as(R->uses);
+    delete R;
+}
 
 }  // extern "C"

@@ -225,11 +225,13 @@ static void ensure_long_rows(const Csr &A, hipStream_t s) {
         CR_HIP(hipGetLastError());
         unsigned long long h = 0;
         CR_HIP(hipMemcpyAsync(&h, count.p, sizeof(h), hipMemcpyDeviceToHost, s));
-        CR_HIP(hipStreamSynchronize(s));
+        synchronise(s);
         nlong = (int64_t)h;
         if (nlong) {
             A.long_rows.alloc_kept(nlong, s);
             CR_HIP(hipMemcpyAsync(A.long_rows.p, list.p, nlong * sizeof(int32_t), hipMemcpyDeviceToDevice, s));
+            release(list, count);
+            synchronise(s);  // calls on other streams may use the long rows next
         }
     }
     A.nlong = nlong;
@@ -245,7 +247,8 @@ void finalize_regridder(cr_regridder *R, hipStream_t s) {
         n[t] = A.nrows;
         cap[t] = A.wide_cap = std::min<int64_t>(A.nrows, A.nnz / (kWideRow + 1));
     }
-    R->finish.alloc_kept(n[0] + n[1] + 1 + (cap[0] + cap[1] + 1) / 2, s);
+    const size_t size = n[0] + n[1] + 1 + (cap[0] + cap[1] + 1) / 2;
+    if (R->finish.n != size) R->finish.alloc_kept(size, s);  // else made again after normalize!
     int32_t *count = (int32_t *)(R->finish.p + n[0] + n[1]);
     hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(2), 0, s, count);
     FinishDir dir[2];
@@ -479,7 +482,7 @@ void prepare(const cr_regridder *R, bool transpose, int dtype, int64_t nf, int64
             ensure_long_rows(A, s);
         }
     }
-    CR_HIP(hipStreamSynchronize(s));
+    synchronise(s);
 }
 
 // Fold partners: y[partner] = y[primary] for every field (the mirror kernel of
@@ -522,6 +525,7 @@ cr_status cr_mirror_fold_partners(const cr_regridder *R, int32_t transpose, int3
         CR_REQUIRE(dst, CR_INVALID_ARGUMENT, "cr_mirror_fold_partners: null field pointer");
         const int32_t *pairs = transpose ? R->fold_src.p : R->fold_dst.p;
         hipStream_t s = as_stream(stream);
+        R->uses.on(s);
         const unsigned g = grid_for(n * nfields, 256);
         if (dtype == CR_F64)
             hipLaunchKernelGGL(k_mirror<double>, dim3(g), dim3(256), 0, s, (double *)dst, dst_cell_stride,
@@ -542,6 +546,7 @@ cr_status cr_mirror_fold_partners_adjoint(const cr_regridder *R, int32_t transpo
         const int64_t n = transpose ? R->nfold_src : R->nfold_dst;
         if (n == 0 || nfields == 0) return;
         CR_REQUIRE(g, CR_INVALID_ARGUMENT, "cr_mirror_fold_partners_adjoint: null gradient pointer");
+        R->uses.on(as_stream(stream));
         hipLaunchKernelGGL(k_mirror_adjoint, dim3(grid_for(n * nfields, 256)), dim3(256), 0, as_stream(stream), g,
                            cell_stride, field_stride, nfields, transpose ? R->fold_src.p : R->fold_dst.p, n);
         CR_HIP(hipGetLastError());
@@ -562,6 +567,7 @@ cr_status cr_regrid(const cr_regridder *R, int32_t transpose, int32_t dtype, int
         CR_REQUIRE(nfields <= 1 || (src_field_stride > 0 && dst_field_stride > 0), CR_INVALID_ARGUMENT,
                    "cr_regrid: field strides must be positive for several fields");
         CR_REQUIRE(nfields == 0 || (src && dst), CR_INVALID_ARGUMENT, "cr_regrid: null field pointer");
+        R->uses.on(as_stream(stream));
         apply(R, transpose != 0, dtype, nfields, src, src_cell_stride, src_field_stride, dst,
               dst_cell_stride, dst_field_stride, normalize != 0, as_stream(stream));
     });
@@ -588,6 +594,7 @@ cr_status cr_regrid_tune(cr_regridder *R, int32_t transpose, int64_t nfields, co
                        dst_field_stride > 0,
                    CR_INVALID_ARGUMENT, "cr_regrid_tune: strides must be positive");
         hipStream_t s = as_stream(stream);
+        R->uses.on(s);
         Csr &A = transpose ? R->bwd : R->fwd;
         hipEvent_t e0, e1;
         CR_HIP(hipEventCreate(&e0));

@@ -1000,7 +1000,7 @@ void build_regridder(cr_regridder *R, const cr_grid *dst, const cr_grid *src,
     int64_t ncand = 0;
     CR_HIP(hipMemcpyAsync(&ncand, cand_off.p + nd, sizeof(int64_t), hipMemcpyDeviceToHost, s));
     CR_HIP(hipMemcpyAsync(h_acct, acct.p, sizeof(h_acct), hipMemcpyDeviceToHost, s));
-    CR_HIP(hipStreamSynchronize(s));
+    synchronise(s);
     if (h_acct[kAcctNonfiniteCells]) {
         const int64_t c = (int64_t)h_acct[kAcctFirstBadCell];
         set_failed_pair(c < nd ? c : -1, c < nd ? -1 : c - nd);
@@ -1062,14 +1062,14 @@ void build_regridder(cr_regridder *R, const cr_grid *dst, const cr_grid *src,
     int64_t nnz = 0;
     CR_HIP(hipMemcpyAsync(&nnz, blk.p + nblk, sizeof(int64_t), hipMemcpyDeviceToHost, s));
     CR_HIP(hipMemcpyAsync(h_acct, acct.p, sizeof(h_acct), hipMemcpyDeviceToHost, s));
-    CR_HIP(hipStreamSynchronize(s));
+    synchronise(s);
     if (h_acct[kAcctNonfinitePairs]) {
         // the reference's DefaultIntersectionFailureError (regridder.jl:64-73): name the pair
         const int64_t c = (int64_t)h_acct[kAcctFirstBadPair];
         int32_t pd = -1, ps = -1;
         CR_HIP(hipMemcpyAsync(&pd, cand_dst.p + c, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         CR_HIP(hipMemcpyAsync(&ps, cand_src.p + c, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        CR_HIP(hipStreamSynchronize(s));
+        synchronise(s);
         set_failed_pair(pd, ps);
         throw Error{CR_DEGENERATE_GEOMETRY, std::to_string(h_acct[kAcctNonfinitePairs]) +
                                                 " intersection(s) have a non-finite area, the first of source cell " +
@@ -1107,7 +1107,9 @@ void build_regridder(cr_regridder *R, const cr_grid *dst, const cr_grid *src,
     R->area_scale = r2;
     finalize_regridder(R, s);
     tm.mark();  // 5
-    CR_HIP(hipStreamSynchronize(s));
+    release(T.buf, acct, cap_dst, cap_src, nodes, order, cand_off, defer, ndefer, cand_src, cand_dst, cval, blk,
+            keep_mask);
+    synchronise(s);
 
     auto &st = R->stats;
     st.n_dst = nd;
@@ -1141,7 +1143,7 @@ void normalize_regridder(cr_regridder *R, hipStream_t s) {
     CR_HIP(rocprim::reduce(p, bytes, F.val.p, mx.p, lowest, (size_t)F.nnz, rocprim::maximum<double>(), s));
     double m = 0;
     CR_HIP(hipMemcpyAsync(&m, mx.p, sizeof(double), hipMemcpyDeviceToHost, s));
-    CR_HIP(hipStreamSynchronize(s));
+    synchronise(s);
     CR_REQUIRE(m > 0.0, CR_DEGENERATE_GEOMETRY, "normalize!: maximum(A) is not positive");
     const int B = 256;
     hipLaunchKernelGGL(k_scale, dim3(grid_for(F.nnz, B)), dim3(B), 0, s, F.val.p, F.nnz, 1.0, m);
@@ -1154,7 +1156,8 @@ void normalize_regridder(cr_regridder *R, hipStream_t s) {
     drop_tile_plan(F);
     drop_tile_plan(R->bwd);
     finalize_regridder(R, s);
-    CR_HIP(hipStreamSynchronize(s));
+    release(T.buf, mx);
+    synchronise(s);
 }
 
 }  // namespace cr
@@ -1196,6 +1199,8 @@ cr_status cr_regridder_build(cr_regridder **R, const cr_grid *dst, const cr_grid
                 if (g->nfold) {
                     f.alloc(2 * g->nfold);
                     CR_HIP(hipMemcpyAsync(f.p, g->fold.p, f.bytes(), hipMemcpyDeviceToDevice, s));
+                    g->uses.on(s);
+                    r->uses.on(s);
                 }
             }
             if (o.normalize) normalize_regridder(r, s);

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -34,24 +35,6 @@ struct Error {
         if (!(cond)) throw ::cr::Error{(status), std::string(msg)}; \
     } while (0)
 
-// Run a body and turn exceptions into a status + thread-local message.
-template <class F>
-cr_status guard(F &&f) {
-    try {
-        f();
-        return CR_OK;
-    } catch (const Error &e) {
-        set_error(e.msg);
-        return e.status;
-    } catch (const std::bad_alloc &) {
-        set_error("host allocation failed");
-        return CR_OUT_OF_MEMORY;
-    } catch (const std::exception &e) {
-        set_error(e.what());
-        return CR_INTERNAL;
-    }
-}
-
 // True while `s` is being captured into a HIP graph.  Lazy per-regridder set-up
 // (tile plans, long-row lists, the default variant) allocates, copies to the
 // host and synchronises: none of that may run inside a capture.
@@ -69,15 +52,44 @@ inline bool stream_capturing(hipStream_t s) {
                std::string(what) + " is not made yet and cannot be made during stream capture: call "   \
                                    "cr_regrid_prepare (or one cr_regrid) with the same arguments first")
 
-// Device memory (memory.hip keeps freed blocks for the next allocation).
-// device_alloc: first used in order on stream s, or (ordered false) on any
-// stream; device_free: every use in order on stream s, or unknown.
-void *device_alloc(size_t bytes, bool ordered, hipStream_t s);
-void device_free(void *p, bool ordered, hipStream_t s);
+// Device memory (memory.hip keeps freed blocks for the next allocation and says
+// who gets which).
+enum Memory {
+    kTemporary,  // used and freed in order on its stream, within one library call
+    kKept,       // owned by a handle: first used in order on its stream, then on any
+    kAnyStream   // owned by a handle: used on any stream from the start
+};
+void *device_alloc(size_t bytes, Memory use, hipStream_t s);
+void device_free(void *p, bool ordered, hipStream_t s);  // ordered: a temporary's
 
-// DevBuf(n): memory for any stream (buffers of grids); DevBuf(n, stream): a
-// temporary, used and freed in order on its stream; alloc_kept(n, stream):
-// owned by a handle, filled on `stream`, afterwards used on any stream.
+// One library call on this thread (guard() holds one).
+struct CallScope {
+    CallScope();
+    ~CallScope();
+    CallScope(const CallScope &) = delete;
+};
+// Wait for stream s: what this call has freed in order on it so far is free for anyone.
+void synchronise(hipStream_t s);
+
+// The streams on which a handle may have work pending: marked by every call that
+// returns without synchronising its stream.
+struct Uses {
+    static constexpr unsigned kOnNull = 1, kElsewhere = 2;
+    mutable std::atomic<unsigned> bits{0};
+    void on(hipStream_t s) const {
+        const unsigned b = s ? kElsewhere : kOnNull;
+        if (!(bits.load(std::memory_order_relaxed) & b)) bits.fetch_or(b);
+    }
+};
+// Buffers of a handle released on this thread in its lifetime are free once the
+// work those uses left pending is done.
+struct ReleaseScope {
+    explicit ReleaseScope(const Uses &u);
+    ~ReleaseScope();
+    ReleaseScope(const ReleaseScope &) = delete;
+};
+
+// DevBuf(n): kAnyStream; DevBuf(n, stream): kTemporary; alloc_kept(n, stream): kKept.
 template <class T>
 struct DevBuf {
     T *p = nullptr;
@@ -102,9 +114,9 @@ struct DevBuf {
         return *this;
     }
     ~DevBuf() { release(); }
-    void alloc(size_t count) { get(count, false, false, nullptr); }
-    void alloc_async(size_t count, hipStream_t s) { get(count, true, true, s); }
-    void alloc_kept(size_t count, hipStream_t s) { get(count, true, false, s); }
+    void alloc(size_t count) { get(count, kAnyStream, nullptr); }
+    void alloc_async(size_t count, hipStream_t s) { get(count, kTemporary, s); }
+    void alloc_kept(size_t count, hipStream_t s) { get(count, kKept, s); }
     void release() {
         device_free(p, ordered, st);
         p = nullptr;
@@ -113,14 +125,39 @@ struct DevBuf {
     size_t bytes() const { return n * sizeof(T); }
 
   private:
-    void get(size_t count, bool first_on_s, bool freed_on_s, hipStream_t s) {
+    void get(size_t count, Memory use, hipStream_t s) {
         release();
         st = s;
-        ordered = freed_on_s;
-        if (count) p = (T *)device_alloc(count * sizeof(T), first_on_s, s);
+        ordered = use == kTemporary;
+        if (count) p = (T *)device_alloc(count * sizeof(T), use, s);
         n = count;
     }
 };
+
+// Free temporaries (in order on their stream).
+template <class... T>
+void release(DevBuf<T> &...b) {
+    (b.release(), ...);
+}
+
+// Run a body and turn exceptions into a status + thread-local message.
+template <class F>
+cr_status guard(F &&f) {
+    CallScope call;
+    try {
+        f();
+        return CR_OK;
+    } catch (const Error &e) {
+        set_error(e.msg);
+        return e.status;
+    } catch (const std::bad_alloc &) {
+        set_error("host allocation failed");
+        return CR_OUT_OF_MEMORY;
+    } catch (const std::exception &e) {
+        set_error(e.what());
+        return CR_INTERNAL;
+    }
+}
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
@@ -142,6 +179,7 @@ inline unsigned grid_for(int64_t n, int block) {
 
 // ------------------------------------------------------------- handles --
 struct cr_grid {
+    cr::Uses uses;
     int64_t ncells = 0;
     int32_t nv = 0;
     int32_t convex = 0;

@@ -143,6 +143,7 @@ cr_status cr_cell_averages(const cr_grid *grid, int32_t field, const double *par
         }
         const TriRule rule = tri_rule(degree);
         hipStream_t s = as_stream(stream);
+        grid->uses.on(s);
         if (grid->ncells)
             hipLaunchKernelGGL(k_cell_averages, dim3(grid_for(grid->ncells, 128)), dim3(128), 0, s, grid->cells.p,
                                grid->nv, grid->ncells, rule, F, out);

@@ -722,7 +722,7 @@ static void backward(const cr_regridder *R, const cr_grid *dst, const cr_grid *s
         apply(R, !transpose, CR_F64, nfields, w, 1, n_to, gx, gxc, gxf, false, s, -1);
     }
     if (!want_verts) {
-        if (!ws) CR_HIP(hipStreamSynchronize(s));
+        if (!ws) synchronise(s);
         return;
     }
     CR_REQUIRE(R->area_scale > 0.0, CR_UNSUPPORTED,
@@ -815,7 +815,8 @@ static void backward(const cr_regridder *R, const cr_grid *dst, const cr_grid *s
                                gto->private_vertices);
     }
     CR_HIP(hipGetLastError());
-    if (!ws) CR_HIP(hipStreamSynchronize(s));
+    release(coef_b, rowid_b);
+    if (!ws) synchronise(s);
 }
 
 // The allocation-free reverse mode's scratch: one static array per device
@@ -874,6 +875,9 @@ cr_status cr_regrid_backward_noalloc(const cr_regridder *R, const cr_grid *dst, 
         ws.rowid = rbytes ? (int32_t *)(base + wbytes + cbytes) : nullptr;
         ws.count = lbytes ? (uint32_t *)(base + wbytes + cbytes + rbytes) : nullptr;
         ws.list = lbytes ? (int32_t *)(base + wbytes + cbytes + rbytes + 256) : nullptr;
+        R->uses.on(as_stream(stream));
+        if (dst) dst->uses.on(as_stream(stream));
+        if (src) src->uses.on(as_stream(stream));
         backward(R, dst, src, transpose, normalize, nfields, x, xc, xf, y, yc, yf, gy, gc, gf, gx, gxc, gxf,
                  g_dst_verts, g_src_verts, as_stream(stream), &ws);
     });

@@ -142,7 +142,8 @@ void orient_grid(cr_grid *g, hipStream_t s) {
     CR_HIP(hipGetLastError());
     int h = 0;
     CR_HIP(hipMemcpyAsync(&h, cnt.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    CR_HIP(hipStreamSynchronize(s));
+    release(cnt);
+    synchronise(s);
     g->flipped = h;
 }
 
@@ -666,7 +667,7 @@ cr_grid *grid_from_polygon_list(const double *xyz, int64_t nverts, const int64_t
             g->xy.alloc((size_t)nverts * 2);
             CR_HIP(hipMemcpyAsync(g->xy.p, planar_xy, g->xy.bytes(), hipMemcpyHostToDevice, s));
         }
-        CR_HIP(hipStreamSynchronize(s));  // the host tables end with this scope
+        synchronise(s);  // the host tables end with this scope
         orient_grid(g, s);
     } catch (...) {
         (void)hipStreamSynchronize(s);
@@ -742,7 +743,7 @@ cr_status cr_grid_from_points(cr_grid **grid, const double *pts, int64_t nblocks
             CR_HIP(hipGetLastError());
             unsigned long long h[2] = {0, 0};
             CR_HIP(hipMemcpyAsync(h, res.p, sizeof(h), hipMemcpyDeviceToHost, s));
-            CR_HIP(hipStreamSynchronize(s));
+            synchronise(s);
             auto cell = [](unsigned long long v) { return v == ~0ull ? INT64_MAX : (int64_t)v; };
             raise_point_cells("cr_grid_from_points", cell(h[0]), cell(h[1]));
         }
@@ -757,6 +758,7 @@ cr_status cr_grid_from_points(cr_grid **grid, const double *pts, int64_t nblocks
             hipLaunchKernelGGL(k_points_to_cells, dim3(grid_for(g->ncells, 256)), dim3(256), 0, s,
                                dpts.p, nblocks, ni, nj, g->cells.p, g->vidx.p);
             CR_HIP(hipGetLastError());
+            release(dpts);
             orient_grid(g, s);
         } catch (...) {
             delete g;
@@ -794,6 +796,7 @@ cr_status cr_grid_tripolar(cr_grid **grid, const double *pts, int64_t nx, int64_
                 hipLaunchKernelGGL(k_fold_pairs, dim3(grid_for(g->nfold, 256)), dim3(256), 0, s, nx, ny, g->fold.p);
             }
             CR_HIP(hipGetLastError());
+            release(dpts);
             orient_grid(g, s);
         } catch (...) {
             (void)hipStreamSynchronize(s);
@@ -853,7 +856,7 @@ cr_status cr_grid_healpix(cr_grid **grid, int64_t nside, int32_t order, int32_t 
             hipLaunchKernelGGL(k_iota_i32, dim3(grid_for(nthr, 256)), dim3(256), 0, s, g->vidx.p, nthr);
             g->private_vertices = 1;
             CR_HIP(hipGetLastError());
-            CR_HIP(hipStreamSynchronize(s));
+            synchronise(s);
         } catch (...) {
             delete g;
             throw;
@@ -910,7 +913,7 @@ cr_status cr_grid_copy_planar_cells(const cr_grid *grid, double *cells_xy) {
 cr_status cr_grid_areas(const cr_grid *grid, double *areas_host) {
     return guard([&] {
         CR_REQUIRE(grid && areas_host, CR_INVALID_ARGUMENT, "null argument");
-        DevBuf<double> a(grid->ncells);
+        DevBuf<double> a(grid->ncells, nullptr);
         if (grid->planar)
             launch_planar_areas(grid, a.p, 0);
         else
@@ -921,6 +924,10 @@ cr_status cr_grid_areas(const cr_grid *grid, double *areas_host) {
     });
 }
 
-void cr_grid_destroy(cr_grid *grid) { delete grid; }
+void cr_grid_destroy(cr_grid *grid) {
+    if (!grid) return;
+    ReleaseScope as(grid->uses);
+    delete grid;
+}
 
 }  // extern "C"

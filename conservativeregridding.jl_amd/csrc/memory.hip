@@ -5,26 +5,35 @@
 // pool and given back each time they cost more than the build's kernels: the
 // pool unmaps large blocks when they are freed (5.5 + 2.2 ms for one quarter
 // degree regridder, whatever its release threshold) and maps them again at the
-// next build.  So freed blocks are kept here and handed out again:
+// next build.  So freed blocks are kept here and handed out again, by who may
+// still be using them:
 //
-//   * a block freed in order on a stream (a temporary) serves the next
-//     allocation on that stream at once, as a stream-ordered pool would;
-//   * a block owned by a handle (any stream may still be using it when the
-//     handle is destroyed) serves again only after a device synchronisation,
-//     made when such a block is first wanted: one per build in a loop of builds;
-//   * a temporary of another stream is left to that stream: the allocation gets
-//     a new block, so threads that build on their own streams do not wait for
-//     one another;
-//   * the kept blocks are bounded (1/64 of the device's memory: 4.5 GB); past
-//     that, and for blocks no allocation has taken over the last kKeep frees,
-//     the oldest go back to the driver, and all of them when an allocation fails.
+//   * kCall: a temporary of a library call that still runs serves that call's next
+//     allocation on its stream at once, as a stream-ordered pool would, and nobody
+//     else.  Once the call has synchronised that stream it is clean (what it frees
+//     after its last synchronise() costs another one at its end).  A stream's handle
+//     says nothing between calls: hipStreamPerThread is another stream on every
+//     thread, and a handle may come back for a new stream.  Only the null stream is
+//     always the same one: its temporaries become kNull without a synchronisation;
+//   * kNull: pending work on the null stream only (also a handle's blocks that was
+//     used on no other stream): serves the next allocation in order on that stream,
+//     and any new handle's buffer once the null stream is synchronised;
+//   * kUnknown: a handle that was used on another stream, possibly by a graph: its
+//     blocks serve a new handle's buffers once the device's pending work is done.
+//     Temporaries do not wait for that, so calls that only need those stay ordered by
+//     their own stream;
+//   * kClean: nobody.
+//
+// The kept blocks are bounded (1/64 of the device's memory: 4.5 GB): past that the
+// oldest go back to the driver, and so do blocks that no allocation took over the last
+// kKeep frees, and all of them when an allocation fails.
 //
 // A build from host inputs and one field there and back: quarter degree ->
 // HEALPix 256 21.6 -> 7.9 ms, 1 degree -> C48 3.0 -> 1.8 ms, 4 -> 5 degrees
 // 2.2 -> 1.1 ms; the reverse mode's temporaries 0.42 -> 0.37 ms (C96 -> 1 degree).
-#include <unistd.h>
+#include <pthread.h>
 
-#include <cstring>
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <unordered_map>
@@ -38,11 +47,12 @@ namespace {
 
 constexpr uint64_t kKeep = 4096;  // frees a block may wait for its next use
 
-enum State { kClean, kOnStream, kUnknown };  // who may still be using a free block: nobody, `stream`, anybody
+enum State { kClean, kNull, kCall, kUnknown };
 
 struct Free {
     void *p;
     State state;
+    uint64_t call;  // kCall: the call and the stream it was freed in order on
     hipStream_t stream;
     bool pool;       // from hipMallocAsync
     uint64_t stamp;  // number of frees when it was freed
@@ -64,14 +74,30 @@ struct Cache {
     std::mutex mu;
     std::unordered_map<void *, Live> live;
     std::map<int, Device> devices;
-    pid_t pid = getpid();
+    uint64_t calls = 0;
 };
+
+// A forked child owns no device memory, and the lock may be held forever there.
+std::atomic<bool> g_child{false};
 
 // never destroyed: handles may be released while the process ends
 Cache &cache() {
-    static Cache *c = new Cache;
+    static Cache *c = [] {
+        pthread_atfork(nullptr, nullptr, [] { g_child = true; });
+        return new Cache;
+    }();
     return *c;
 }
+
+// The library call of this thread, and how a handle's buffers are released.
+struct Call {
+    int depth = 0;
+    uint64_t id = 0;  // 0: no temporaries yet
+};
+thread_local Call t_call;
+thread_local State t_release = kUnknown;
+
+using Lock = std::unique_lock<std::mutex>;
 
 // sizes in steps of an eighth, so that nearly equal requests share blocks
 size_t rounded(size_t bytes) {
@@ -80,30 +106,11 @@ size_t rounded(size_t bytes) {
     return (bytes + step - 1) / step * step;
 }
 
-bool synchronise(Device &d) {
-    if (hipDeviceSynchronize() != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    for (auto &f : d.free) f.second.state = kClean;
-    return true;
-}
-
-// Give blocks back to the driver until `most` bytes are kept; those older than
-// `before` in any case.  The caller has made the device current.
-void trim(Device &d, size_t most, uint64_t before) {
-    bool synced = false;
-    while (!d.free.empty()) {
-        auto oldest = d.free.begin();
-        for (auto it = d.free.begin(); it != d.free.end(); ++it)
-            if (it->second.stamp < oldest->second.stamp) oldest = it;
-        if (d.kept <= most && oldest->second.stamp >= before) return;
-        if (!synced && !(synced = synchronise(d))) return;
-        d.kept -= oldest->first;
-        if (oldest->second.pool) (void)hipFreeAsync(oldest->second.p, nullptr);
-        else (void)hipFree(oldest->second.p);
-        d.free.erase(oldest);
-    }
+// Wait for the device's pending work (the caller has made it current).
+bool device_wait() {
+    if (hipDeviceSynchronize() == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
 }
 
 // The smallest free block of `bytes` that `ok` accepts and that is not much larger.
@@ -115,15 +122,130 @@ std::multimap<size_t, Free>::iterator find(Device &d, size_t bytes, F ok) {
     return d.free.end();
 }
 
+// Wait until the free blocks in state st are clean.
+bool wait_and_clean(Device &d, State st) {
+    const uint64_t now = d.frees;
+    const bool done = st == kNull ? hipStreamSynchronize(nullptr) == hipSuccess : device_wait();
+    if (!done) (void)hipGetLastError();
+    if (done)
+        for (auto &f : d.free)
+            if (f.second.stamp < now && f.second.state == st) f.second.state = kClean;
+    return done;
+}
+
+// Give blocks back to the driver: the oldest until `most` bytes are kept, and those
+// older than `before`.  Blocks of running calls stay, but for this thread's own when
+// `own`.  The caller has made the device current.
+void trim(Device &d, size_t most, uint64_t before, bool own) {
+    auto mine = [&](const Free &f) { return own && f.call && f.call == t_call.id; };
+    std::vector<std::multimap<size_t, Free>::iterator> order;
+    for (auto it = d.free.begin(); it != d.free.end(); ++it)
+        if (it->second.state != kCall || mine(it->second)) order.push_back(it);
+    std::sort(order.begin(), order.end(), [](auto a, auto b) { return a->second.stamp < b->second.stamp; });
+    std::vector<std::pair<size_t, Free>> out;
+    for (auto it : order) {
+        if (d.kept <= most && it->second.stamp >= before) break;
+        d.kept -= it->first;
+        out.push_back(*it);
+        d.free.erase(it);
+    }
+    if (out.empty()) return;
+    auto give = [](const Free &f) {
+        if (f.pool) (void)hipFreeAsync(f.p, f.state == kCall ? f.stream : nullptr);
+        else (void)hipFree(f.p);
+    };
+    std::vector<std::pair<size_t, Free>> back;
+    for (auto &b : out) {
+        if (b.second.state == kUnknown) back.push_back(b);
+        else give(b.second);
+    }
+    if (!back.empty() && device_wait()) {
+        for (auto &b : back) give(b.second);
+        back.clear();
+    }
+    (void)hipGetLastError();
+    for (auto &b : back) {
+        d.free.insert(b);
+        d.kept += b.first;
+    }
+}
+
+// Keep the bounds of device `index`, on whatever device this thread is.
+void bound(Device &d, int index) {
+    const uint64_t before = d.frees > kKeep ? d.frees - kKeep : 0;
+    const bool over = d.kept > d.cap;
+    if (!over && !(before && d.frees % 64 == 0)) return;
+    int dev = index;
+    if (hipGetDevice(&dev) != hipSuccess) return;
+    if (dev != index && hipSetDevice(index) != hipSuccess) return;
+    trim(d, d.cap, before, false);
+    if (dev != index) (void)hipSetDevice(dev);
+}
+
+// Each block this call freed in order on its streams.
+template <class F>
+void freed_by_call(Cache &c, F f) {
+    for (auto &dev : c.devices)
+        for (auto &b : dev.second.free)
+            if (b.second.state == kCall && b.second.call == t_call.id) f(b.second);
+}
+
+// The call is over: synchronise the streams it freed temporaries on.
+void end_call() {
+    Cache &c = cache();
+    std::vector<hipStream_t> pending;
+    Lock lock(c.mu);
+    freed_by_call(c, [&](Free &f) {
+        if (!f.stream) f.state = kNull;
+        else if (std::find(pending.begin(), pending.end(), f.stream) == pending.end()) pending.push_back(f.stream);
+    });
+    for (hipStream_t s : pending) {
+        const State st = hipStreamSynchronize(s) == hipSuccess ? kClean : kUnknown;
+        if (st != kClean) (void)hipGetLastError();
+        freed_by_call(c, [&](Free &f) {
+            if (f.stream == s) f.state = st;
+        });
+    }
+    for (auto &dev : c.devices) bound(dev.second, dev.first);
+}
+
 }  // namespace
 
-// `ordered`: the memory is first used on stream s; else on any stream.
-void *device_alloc(size_t bytes, bool ordered, hipStream_t s) {
+CallScope::CallScope() { ++t_call.depth; }
+
+CallScope::~CallScope() {
+    if (--t_call.depth) return;
+    try {
+        if (t_call.id && !g_child) end_call();
+    } catch (const std::exception &) {  // no host memory: the call's blocks stay its own
+    }
+    t_call = Call{};
+}
+
+void synchronise(hipStream_t s) {
+    CR_HIP(hipStreamSynchronize(s));
+    if (!t_call.id) return;
+    Cache &c = cache();
+    Lock lock(c.mu);
+    freed_by_call(c, [&](Free &f) {
+        if (f.stream == s) f.state = kClean;
+    });
+}
+
+ReleaseScope::ReleaseScope(const Uses &u) {
+    const unsigned b = u.bits.load();
+    t_release = b == 0 ? kClean : b == Uses::kOnNull ? kNull : kUnknown;
+}
+ReleaseScope::~ReleaseScope() { t_release = kUnknown; }
+
+void *device_alloc(size_t bytes, Memory use, hipStream_t s) {
+    const bool ordered = use != kAnyStream;
     int dev = 0;
     CR_HIP(hipGetDevice(&dev));
     const size_t want = rounded(bytes);
     Cache &c = cache();
-    std::lock_guard<std::mutex> lock(c.mu);
+    CR_REQUIRE(!g_child, CR_HIP_ERROR, "a forked child has no device memory");
+    Lock lock(c.mu);
     Device &d = c.devices[dev];
     if (!d.cap) {
         size_t avail = 0, total = 0;
@@ -134,13 +256,17 @@ void *device_alloc(size_t bytes, bool ordered, hipStream_t s) {
         if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess)
             (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &thr);
     }
+    if (use == kTemporary && t_call.depth && !t_call.id) t_call.id = ++c.calls;
     auto usable = [&](const Free &f) {
-        return f.state == kClean || (f.state == kOnStream && ordered && f.stream == s);
+        return f.state == kClean || (f.state == kNull && ordered && !s) ||
+               (f.state == kCall && ordered && f.call == t_call.id && f.stream == s);
     };
     auto it = find(d, want, usable);
-    if (it == d.free.end() && find(d, want, [](const Free &f) { return f.state == kUnknown; }) != d.free.end() &&
-        synchronise(d))
-        it = find(d, want, usable);
+    for (State st : {kNull, kUnknown}) {
+        if (it != d.free.end() || use == kTemporary) break;
+        auto in_state = [st](const Free &f) { return f.state == st; };
+        if (find(d, want, in_state) != d.free.end() && wait_and_clean(d, st)) it = find(d, want, usable);
+    }
     if (it != d.free.end()) {
         void *p = it->second.p;
         c.live[p] = {it->first, dev, it->second.pool};
@@ -151,10 +277,10 @@ void *device_alloc(size_t bytes, bool ordered, hipStream_t s) {
     auto fresh = [&](void **p) { return ordered ? hipMallocAsync(p, want, s) : hipMalloc(p, want); };
     void *p = nullptr;
     hipError_t e = fresh(&p);
-    if (e == hipErrorOutOfMemory && !d.free.empty()) {
+    if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        trim(d, 0, UINT64_MAX);
-        (void)hipDeviceSynchronize();
+        trim(d, 0, UINT64_MAX, true);
+        (void)device_wait();
         e = fresh(&p);
     }
     CR_HIP(e);
@@ -162,26 +288,24 @@ void *device_alloc(size_t bytes, bool ordered, hipStream_t s) {
     return p;
 }
 
-// `ordered`: every use of the memory is in order on stream s; else unknown.
 void device_free(void *p, bool ordered, hipStream_t s) {
     if (!p) return;
     Cache &c = cache();
-    if (getpid() != c.pid) return;  // a forked child owns no device memory (and the lock may be held forever)
-    std::lock_guard<std::mutex> lock(c.mu);
-    auto l = c.live.find(p);
-    if (l == c.live.end()) return;
-    const Live b = l->second;
-    c.live.erase(l);
-    Device &d = c.devices[b.device];
-    d.free.insert({b.bytes, Free{p, ordered ? kOnStream : kUnknown, s, b.pool, d.frees++}});
-    d.kept += b.bytes;
-    const uint64_t before = d.frees > kKeep ? d.frees - kKeep : 0;
-    if (d.kept > d.cap || (before && d.frees % 64 == 0)) {
-        int dev = b.device;
-        if (hipGetDevice(&dev) != hipSuccess) return;
-        if (dev != b.device && hipSetDevice(b.device) != hipSuccess) return;
-        trim(d, d.cap, before);
-        if (dev != b.device) (void)hipSetDevice(dev);
+    if (g_child) return;
+    try {
+        Lock lock(c.mu);
+        auto l = c.live.find(p);
+        if (l == c.live.end()) return;
+        const Live b = l->second;
+        Device &d = c.devices[b.device];
+        State st = t_release;
+        if (ordered) st = t_call.id ? kCall : s ? kUnknown : kNull;
+        d.free.insert({b.bytes, Free{p, st, st == kCall ? t_call.id : 0, s, b.pool, d.frees}});
+        c.live.erase(l);
+        d.frees++;
+        d.kept += b.bytes;
+        bound(d, b.device);
+    } catch (const std::exception &) {  // no host memory for the list: the block is lost, not handed out twice
     }
 }
 

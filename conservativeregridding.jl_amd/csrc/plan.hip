@@ -806,7 +806,7 @@ void make_plan(const Csr &A, TilePlan &P, hipStream_t s) {
     int64_t h[3], nh = 0;
     CR_HIP(hipMemcpyAsync(h, totals.p, sizeof(h), hipMemcpyDeviceToHost, s));
     CR_HIP(hipMemcpyAsync(&nh, hpos.p + nrows, sizeof(nh), hipMemcpyDeviceToHost, s));
-    CR_HIP(hipStreamSynchronize(s));
+    synchronise(s);
     P.ntiles = h[0];
     P.nslots = h[1];
     P.nhuge = nh;
@@ -830,7 +830,8 @@ void make_plan(const Csr &A, TilePlan &P, hipStream_t s) {
     CR_HIP(hipGetLastError());
     unsigned long long f[3] = {0, 0, 0};
     CR_HIP(hipMemcpyAsync(f, fstat.p, sizeof(f), hipMemcpyDeviceToHost, s));
-    CR_HIP(hipStreamSynchronize(s));
+    release(T.buf, prev, table, exits, sub, recs, totals, hflag, hpos, fstat);
+    synchronise(s);
     CR_REQUIRE(!f[0], CR_INTERNAL, "tile plan: a tile broke its budgets");
     P.tile_cols = (int64_t)f[1];
     P.tile_lines = (int64_t)f[2];
@@ -891,7 +892,7 @@ cr_status cr_regrid_tile_plan(const cr_regridder *R, int32_t transpose, int32_t 
         for (int i = 0; i < 6; ++i) sizes[i] = 0;
         if (A.nrows == 0) return;
         const TilePlan &P = tile_plan(A, style & 1, geom, s, (style & 2) != 0);
-        CR_HIP(hipStreamSynchronize(s));
+        synchronise(s);
         sizes[0] = P.ntiles;
         sizes[1] = P.nslots;
         sizes[2] = (int64_t)P.cols.n;

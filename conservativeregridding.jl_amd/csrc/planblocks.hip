@@ -103,7 +103,8 @@ void make_block_plan(const Csr &A, TilePlan &P, hipStream_t s) {
         hipLaunchKernelGGL(k_map_rows, dim3(grid_for(P.nhuge, 256)), dim3(256), 0, s, P.huge.p, P.nhuge,
                            rowmap.p);
     CR_HIP(hipGetLastError());
-    CR_HIP(hipStreamSynchronize(s));  // B's buffers are released after this
+    release(T.buf, B.rowptr, B.col, B.val);
+    synchronise(s);
     P.rowmap = std::move(rowmap);
 }
 

@@ -78,6 +78,7 @@ bool plan_ready(const Csr &A, int style, int geom, bool blocks);
 }  // namespace cr
 
 struct cr_regridder {
+    cr::Uses uses;
     cr::Csr fwd;  // A:   n_dst x n_src
     cr::Csr bwd;  // A^T: n_src x n_dst
     cr::DevBuf<double> a_dst, a_src;

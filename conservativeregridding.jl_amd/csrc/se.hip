@@ -432,7 +432,7 @@ void launch_moments(const cr_regridder *R, const cr_grid *cells, const cr_grid *
     CR_HIP(hipGetLastError());
     int h = 0;
     CR_HIP(hipMemcpyAsync(&h, err.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    CR_HIP(hipStreamSynchronize(s));
+    synchronise(s);
     CR_REQUIRE(h == 0, CR_INTERNAL, "spectral-element moments: clipped polygon buffer overflow");
 }
 
@@ -464,7 +464,7 @@ void node_weights(const cr_grid *elems, const NodeSet &ns, double r2, const doub
     wj.alloc_kept(n, s);
     if (user) {
         CR_HIP(hipMemcpyAsync(wj.p, user, n * sizeof(double), hipMemcpyHostToDevice, s));
-        CR_HIP(hipStreamSynchronize(s));
+        synchronise(s);
     } else {
         hipLaunchKernelGGL(k_se_nodes, dim3(grid_for(n, 256)), dim3(256), 0, s, elems->cells.p, elems->ncells, ns,
                            r2, nullptr, wj.p);
@@ -603,7 +603,7 @@ cr_status cr_se_regridder_to_fv(cr_regridder **out, const cr_grid *cells, const 
         R->a_dst = std::move(P->a_dst);
         node_weights(elems, node_set(nq), P->area_scale, node_weights_host, R->a_src, s);
         finalize_regridder(R.get(), s);
-        CR_HIP(hipStreamSynchronize(s));
+        synchronise(s);
         R->stats = P->stats;
         R->stats.n_src = nodes;
         R->stats.nnz = nnz;
@@ -639,7 +639,7 @@ cr_status cr_se_regridder_from_fv(cr_regridder **out, const cr_grid *elems, cons
             DevBuf<double> dw;
             node_weights(elems, ns, P->area_scale, node_weights_host, dw, s);
             CR_HIP(hipMemcpyAsync(wj.data(), dw.p, dw.bytes(), hipMemcpyDeviceToHost, s));
-            CR_HIP(hipStreamSynchronize(s));
+            synchronise(s);
         }
         // pairs of each element, cells ascending
         std::vector<int64_t> eoff(ne + 1, 0);
