@@ -20,8 +20,10 @@
 //     and any new handle's buffer once the null stream is synchronised;
 //   * kUnknown: a handle that was used on another stream, possibly by a graph: its
 //     blocks serve a new handle's buffers once the device's pending work is done.
-//     Temporaries do not wait for that, so calls that only need those stay ordered by
-//     their own stream;
+//     The allocation waits for that by hipFree of a small block, which synchronises
+//     the device by contract; hipDeviceSynchronize would break every stream capture
+//     in progress, on whatever thread and in whatever mode.  Temporaries do not
+//     wait, so calls that only need those stay ordered by their own stream;
 //   * kClean: nobody.
 //
 // The kept blocks are bounded (1/64 of the device's memory: 4.5 GB): past that the
@@ -108,7 +110,8 @@ size_t rounded(size_t bytes) {
 
 // Wait for the device's pending work (the caller has made it current).
 bool device_wait() {
-    if (hipDeviceSynchronize() == hipSuccess) return true;
+    void *p = nullptr;
+    if (hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess) return true;
     (void)hipGetLastError();
     return false;
 }

@@ -1,5 +1,5 @@
 """Device memory between calls: two threads on hipStreamPerThread (one handle, two
-streams)."""
+streams), and builds beside a capture on another thread."""
 import ctypes
 import threading
 
@@ -10,6 +10,12 @@ import torch
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 PER_THREAD = 2  # hipStreamPerThread
+
+
+def _hip():
+    torch.ones(1, device=DEV)
+    with open("/proc/self/maps") as f:
+        return ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
 
 
 def _grids(cr, n):
@@ -72,3 +78,58 @@ def test_threads_on_the_per_thread_stream(cr):
         assert torch.equal(g[0], ref[0])
         for a, b in zip(g[1:], ref[1:]):  # sums in any order of a few dozen terms
             assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
+
+
+class _Capture:
+    """A capture on a stream of its own: mode 1 is hipStreamCaptureModeThreadLocal."""
+
+    def __init__(self, mode):
+        self.hip, self.s, self.mode = _hip(), ctypes.c_void_p(), mode
+        assert self.hip.hipStreamCreateWithFlags(ctypes.byref(self.s), 1) == 0
+
+    def __enter__(self):
+        torch.cuda.synchronize()
+        assert self.hip.hipStreamBeginCapture(self.s, self.mode) == 0
+        return self
+
+    def active(self):
+        st = ctypes.c_int()
+        return self.hip.hipStreamIsCapturing(self.s, ctypes.byref(st)) == 0 and st.value == 1
+
+    def __exit__(self, *exc):
+        g = ctypes.c_void_p()
+        self.ended = self.hip.hipStreamEndCapture(self.s, ctypes.byref(g))
+        if g.value:
+            self.hip.hipGraphDestroy(g)
+        self.hip.hipStreamDestroy(self.s)
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+def test_builds_beside_a_capture_on_another_thread(cr, mode):
+    print(f"[case] builds beside a capture, mode {mode}", flush=True)
+    L = cr._lib
+    dst, src = _grids(cr, 24)
+    x = torch.ones(src.ncells, dtype=torch.float64, device=DEV)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    bad = []
+
+    def work():
+        torch.cuda.set_device(0)
+        for _ in range(3):  # from the second on with blocks of a handle used on the side stream
+            st, h = _build(cr, dst, src, side.cuda_stream)
+            y = torch.empty(dst.ncells, dtype=torch.float64, device=DEV)
+            if st != L.CR_OK or L.lib.cr_regrid(h, 0, L.CR_F64, 1, x.data_ptr(), 1, 1, y.data_ptr(), 1, 1, 1,
+                                                side.cuda_stream) != L.CR_OK:
+                bad.append(L.last_error())
+            L.lib.cr_regridder_destroy(h)
+
+    work()  # memory for y, and what is made once
+    torch.cuda.synchronize()
+    with _Capture(mode) as c:
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        active = c.active()
+    assert active and c.ended == 0 and not bad
+    torch.cuda.synchronize()

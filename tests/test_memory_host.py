@@ -131,9 +131,21 @@ def test_handle_blocks_by_use(mem):
     for bits in (ELSEWHERE, ON_NULL | ELSEWHERE):
         t = handle(bits)
         assert mem.alloc(TEMP, SIDE) != t and mem.alloc(TEMP, NULL) != t
-        assert "devicesync" not in mem.log()  # temporaries do not wait for the device
+        assert "free" not in mem.log()  # temporaries do not wait for the device
         assert mem.alloc(KEPT, SIDE) == t
-        assert mem.log() == ["devicesync"]
+        assert mem.log() == ["malloc", "free"]  # hipFree waits for the device
+
+
+def test_the_device_is_never_synchronised_outright(mem):
+    """hipDeviceSynchronize breaks stream captures on other threads."""
+    for bits in (UNUSED, ON_NULL, ELSEWHERE):
+        for s in (NULL, SIDE, PER_THREAD):
+            for use in (KEPT, ANY):
+                mem.lib.handle_free(mem.alloc(use, s), bits)
+            mem.call(s, 3)
+    for i in range(400):
+        mem.lib.handle_free(mem.alloc(KEPT, SIDE, 20000 + 4096 * (i % 90)), ELSEWHERE)
+    assert "devicesync" not in mem.log()
 
 
 @pytest.mark.parametrize("bits", [UNUSED, ON_NULL, ELSEWHERE])
