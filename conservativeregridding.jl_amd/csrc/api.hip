@@ -70,6 +70,7 @@ cr_status cr_regridder_from_csr(cr_regridder **R, int64_t n_dst, int64_t n_src, 
             CR_REQUIRE(col[k] >= 0 && col[k] < n_src, CR_DIMENSION_MISMATCH, "column index out of range");
         check_device();
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_regridder_from_csr");
         std::vector<int64_t> trp;
         std::vector<int32_t> tcol;
         std::vector<double> tval;

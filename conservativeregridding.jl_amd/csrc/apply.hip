@@ -580,6 +580,7 @@ cr_status cr_regrid_prepare(const cr_regridder *R, int32_t transpose, int32_t dt
         CR_REQUIRE(dtype == CR_F64 || dtype == CR_F32, CR_UNSUPPORTED, "cr_regrid_prepare: dtype must be F64 or F32");
         CR_REQUIRE(nfields >= 0 && src_field_stride >= 0 && dst_field_stride >= 0, CR_INVALID_ARGUMENT,
                    "cr_regrid_prepare: bad sizes or strides");
+        refuse_capture(as_stream(stream), "cr_regrid_prepare");
         prepare(R, transpose != 0, dtype, nfields, src_field_stride, dst_field_stride, as_stream(stream));
     });
 }
@@ -594,6 +595,7 @@ cr_status cr_regrid_tune(cr_regridder *R, int32_t transpose, int64_t nfields, co
                        dst_field_stride > 0,
                    CR_INVALID_ARGUMENT, "cr_regrid_tune: strides must be positive");
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_regrid_tune");
         R->uses.on(s);
         Csr &A = transpose ? R->bwd : R->fwd;
         hipEvent_t e0, e1;

@@ -1189,6 +1189,7 @@ cr_status cr_regridder_build(cr_regridder **R, const cr_grid *dst, const cr_grid
         check_device();
         const auto t0 = std::chrono::steady_clock::now();
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_regridder_build");
         auto *r = new cr_regridder();
         try {
             build_regridder(r, dst, src, o, s);
@@ -1225,6 +1226,7 @@ cr_status cr_last_failed_pair(int64_t *dst_cell, int64_t *src_cell) {
 cr_status cr_regridder_normalize(cr_regridder *R, void *stream) {
     return guard([&] {
         CR_REQUIRE(R, CR_INVALID_ARGUMENT, "null regridder");
+        refuse_capture(as_stream(stream), "cr_regridder_normalize");
         normalize_regridder(R, as_stream(stream));
     });
 }

@@ -52,6 +52,15 @@ inline bool stream_capturing(hipStream_t s) {
                std::string(what) + " is not made yet and cannot be made during stream capture: call "   \
                                    "cr_regrid_prepare (or one cr_regrid) with the same arguments first")
 
+// Calls that allocate and synchronise whatever was prepared: refused before they
+// enqueue anything, so that the capture goes on without them.  (The null stream is
+// never captured; other captures do not concern it.)
+inline void refuse_capture(hipStream_t s, const char *call) {
+    CR_REQUIRE(!s || !stream_capturing(s), CR_UNSUPPORTED,
+               std::string(call) + " allocates device memory and synchronises its stream: it cannot run while that "
+                                   "stream is being captured");
+}
+
 // Device memory (memory.hip keeps freed blocks for the next allocation and says
 // who gets which).
 enum Memory {

@@ -889,6 +889,7 @@ cr_status cr_regrid_backward(const cr_regridder *R, const cr_grid *dst, const cr
                              const double *gy, int64_t gc, int64_t gf, double *gx, int64_t gxc,
                              int64_t gxf, double *g_dst_verts, double *g_src_verts, void *stream) {
     return guard([&] {
+        refuse_capture(as_stream(stream), "cr_regrid_backward (cr_regrid_backward_noalloc does neither)");
         backward(R, dst, src, transpose, normalize, nfields, x, xc, xf, y, yc, yf, gy, gc, gf, gx, gxc, gxf,
                  g_dst_verts, g_src_verts, as_stream(stream), nullptr);
     });

@@ -592,6 +592,7 @@ cr_status cr_grid_from_cells(cr_grid **grid, const double *cells, int64_t ncells
             "cr_grid_from_cells", nullptr);
         check_device();
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_grid_from_cells");
         auto *g = new cr_grid();
         try {
             g->ncells = ncells;
@@ -652,6 +653,7 @@ cr_grid *grid_from_polygon_list(const double *xyz, int64_t nverts, const int64_t
     validate_cells(
         ncells, nv, convex != 0, [&](int64_t c, int k) { return cp + 3 * (c * nv + k); }, what, nullptr);
     check_device();
+    refuse_capture(s, what);
     auto *g = new cr_grid();
     try {
         g->ncells = ncells;
@@ -732,6 +734,7 @@ cr_status cr_grid_from_points(cr_grid **grid, const double *pts, int64_t nblocks
         validate_point_units(pts, nblocks, ni, nj, "cr_grid_from_points");
         check_device();
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_grid_from_points");
         int64_t npts = nblocks * (ni + 1) * (nj + 1);
         DevBuf<double> dpts((size_t)npts * 3, s);  // pool memory, freed in order on s
         CR_HIP(hipMemcpyAsync(dpts.p, pts, dpts.bytes(), hipMemcpyHostToDevice, s));
@@ -777,6 +780,7 @@ cr_status cr_grid_tripolar(cr_grid **grid, const double *pts, int64_t nx, int64_
         validate_point_blocks(pts, 1, nx, ny, "cr_grid_tripolar", nullptr);
         check_device();
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_grid_tripolar");
         const int64_t npts = (nx + 1) * (ny + 1);
         DevBuf<double> dpts((size_t)npts * 3, s);
         CR_HIP(hipMemcpyAsync(dpts.p, pts, dpts.bytes(), hipMemcpyHostToDevice, s));
@@ -842,6 +846,7 @@ cr_status cr_grid_healpix(cr_grid **grid, int64_t nside, int32_t order, int32_t 
         CR_REQUIRE(nside <= 8192, CR_UNSUPPORTED, "nside above 8192");
         check_device();
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_grid_healpix");
         auto *g = new cr_grid();
         try {
             g->ncells = 12 * nside * nside;

@@ -95,6 +95,8 @@ Cache &cache() {
 struct Call {
     int depth = 0;
     uint64_t id = 0;  // 0: no temporaries yet
+    bool checked = false;
+    hipStream_t checked_stream = nullptr;  // not capturing
 };
 thread_local Call t_call;
 thread_local State t_release = kUnknown;
@@ -245,6 +247,12 @@ void *device_alloc(size_t bytes, Memory use, hipStream_t s) {
     const bool ordered = use != kAnyStream;
     int dev = 0;
     CR_HIP(hipGetDevice(&dev));
+    // memory allocated while its stream is being captured would belong to the graph
+    if (ordered && s && !(t_call.checked && t_call.checked_stream == s)) {
+        refuse_capture(s, "this call");
+        t_call.checked = t_call.depth > 0;
+        t_call.checked_stream = s;
+    }
     const size_t want = rounded(bytes);
     Cache &c = cache();
     CR_REQUIRE(!g_child, CR_HIP_ERROR, "a forked child has no device memory");

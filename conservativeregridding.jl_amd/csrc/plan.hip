@@ -889,6 +889,7 @@ cr_status cr_regrid_tile_plan(const cr_regridder *R, int32_t transpose, int32_t 
                    "cr_regrid_tile_plan: style is 0..3 and geom 0 or 1");
         const Csr &A = transpose ? R->bwd : R->fwd;
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_regrid_tile_plan");
         for (int i = 0; i < 6; ++i) sizes[i] = 0;
         if (A.nrows == 0) return;
         const TilePlan &P = tile_plan(A, style & 1, geom, s, (style & 2) != 0);

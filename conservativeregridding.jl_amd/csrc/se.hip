@@ -562,6 +562,7 @@ cr_status cr_se_moments(const cr_regridder *R, const cr_grid *cells, const cr_gr
     return guard([&] {
         CR_REQUIRE(R && cells && elems && (B || R->fwd.nnz == 0), CR_INVALID_ARGUMENT, "cr_se_moments: null argument");
         CR_REQUIRE(R->area_scale > 0.0, CR_UNSUPPORTED, "cr_se_moments needs a regridder built from grids");
+        refuse_capture(as_stream(stream), "cr_se_moments");
         moments(R, cells, elems, nq, tri_degree, R->area_scale, B, as_stream(stream), pair_cell, pair_elem);
     });
 }
@@ -574,6 +575,7 @@ cr_status cr_se_regridder_to_fv(cr_regridder **out, const cr_grid *cells, const 
         check_device();
         check_elements(elems);
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_se_regridder_to_fv");
         std::unique_ptr<cr_regridder> P(pair_regridder(cells, elems, opts, s));
         const int Q = nq * nq;
         const int64_t nnz = P->fwd.nnz * Q, nodes = elems->ncells * Q;
@@ -619,6 +621,7 @@ cr_status cr_se_regridder_from_fv(cr_regridder **out, const cr_grid *elems, cons
         check_device();
         check_elements(elems);
         hipStream_t s = as_stream(stream);
+        refuse_capture(s, "cr_se_regridder_from_fv");
         std::unique_ptr<cr_regridder> P(pair_regridder(cells, elems, opts, s));
         const NodeSet ns = node_set(nq);
         const int Q = nq * nq;

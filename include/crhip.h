@@ -23,7 +23,12 @@
  *     than nv vertices repeat their last vertex.
  *   - Rows of A are destination cells and columns are source cells
  *     (intersection_areas.jl:115-121).
- *   - `stream` is a hipStream_t passed as void*; NULL is the null stream.
+ *   - `stream` is a hipStream_t passed as void*; NULL is the null stream,
+ *     hipStreamPerThread the calling thread's own.  While it is being captured
+ *     into a graph only calls that allocate nothing run on it (cr_regrid after
+ *     its set-up, the fold mirrors, cr_regrid_backward_noalloc,
+ *     cr_cell_averages); the others return CR_UNSUPPORTED before they enqueue
+ *     anything, and the capture goes on without them.
  *   - Handles are immutable after creation except through cr_regridder_normalize;
  *     concurrent cr_regrid calls on one handle with distinct outputs are safe.
  */

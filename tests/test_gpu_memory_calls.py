@@ -1,5 +1,6 @@
 """Device memory between calls: two threads on hipStreamPerThread (one handle, two
-streams), and builds beside a capture on another thread."""
+streams), calls on a stream that is being captured, and builds beside a capture on
+another thread."""
 import ctypes
 import threading
 
@@ -102,6 +103,30 @@ class _Capture:
         if g.value:
             self.hip.hipGraphDestroy(g)
         self.hip.hipStreamDestroy(self.s)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_allocating_calls_are_refused_on_a_capturing_stream(cr, mode):
+    print(f"[case] refused while capturing, mode {mode}", flush=True)
+    L = cr._lib
+    dst, src = _grids(cr, 12)
+    R = cr.Regridder(dst, src)
+    x, gy = torch.ones(src.ncells, dtype=torch.float64, device=DEV), torch.ones(dst.ncells, dtype=torch.float64, device=DEV)
+    y = cr.regrid(R, x)
+    g = [torch.zeros(n, dtype=torch.float64, device=DEV) for n in (src.ncells, 3 * dst.nverts, 3 * src.nverts)]
+    pts = np.ascontiguousarray(cr.lonlat_points(12, 6).transpose(1, 0, 2))
+    with _Capture(mode) as c:
+        h = ctypes.c_void_p()
+        got = [_build(cr, dst, src, c.s)[0],
+               _backward(cr, R._core.h, dst, src, x, y, gy, g, c.s),
+               L.lib.cr_regridder_normalize(R._core.h, c.s),
+               L.lib.cr_regrid_prepare(R._core.h, 0, L.CR_F64, 1, 1, 1, c.s),
+               L.lib.cr_grid_healpix(ctypes.byref(h), 4, 0, 2, c.s),
+               L.lib.cr_grid_from_points(ctypes.byref(h), L.dptr(pts), 1, 12, 6, c.s)]
+        active, message = c.active(), L.last_error()
+    assert got == [L.CR_UNSUPPORTED] * len(got) and "captured" in message
+    assert active and c.ended == 0  # the capture goes on without them
+    assert _backward(cr, R._core.h, dst, src, x, y, gy, g, None) == L.CR_OK
 
 
 @pytest.mark.parametrize("mode", [1, 2])

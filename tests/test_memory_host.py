@@ -13,6 +13,7 @@ NULL, SIDE, OTHER, PER_THREAD = 0, 0x1000, 0x2000, 2
 UNUSED, ON_NULL, ELSEWHERE = 0, 1, 2
 N = 100000
 MB = 1 << 20
+UNSUPPORTED = 3  # cr_status
 
 
 class Memory:
@@ -146,6 +147,20 @@ def test_the_device_is_never_synchronised_outright(mem):
     for i in range(400):
         mem.lib.handle_free(mem.alloc(KEPT, SIDE, 20000 + 4096 * (i % 90)), ELSEWHERE)
     assert "devicesync" not in mem.log()
+
+
+@pytest.mark.parametrize("use", [TEMP, KEPT])
+def test_capturing_streams_are_refused(mem, use):
+    mem.call(SIDE)
+    mem.log()
+    mem.lib.set_capturing(SIDE, 1)
+    mem.lib.call_begin()
+    assert mem.alloc(use, SIDE) is None
+    assert mem.alloc(use, NULL) is not None  # the null stream is not captured
+    mem.lib.call_end()
+    assert mem.log()[0] == "error%d" % UNSUPPORTED
+    mem.lib.set_capturing(SIDE, 0)
+    assert mem.alloc(use, SIDE) is not None
 
 
 @pytest.mark.parametrize("bits", [UNUSED, ON_NULL, ELSEWHERE])
