@@ -26,9 +26,10 @@
 //     wait, so calls that only need those stay ordered by their own stream;
 //   * kClean: nobody.
 //
-// The kept blocks are bounded (1/64 of the device's memory: 4.5 GB): past that the
-// oldest go back to the driver, and so do blocks that no allocation took over the last
-// kKeep frees, and all of them when an allocation fails.
+// No lock is held while the driver works.  The kept blocks are bounded (1/64 of the
+// device's memory: 4.5 GB): past that the oldest go back to the driver until a quarter
+// of the bound is free, and so do blocks that no allocation took over the last kKeep
+// frees, and all of them when an allocation fails.
 //
 // A build from host inputs and one field there and back: quarter degree ->
 // HEALPix 256 21.6 -> 7.9 ms, 1 degree -> C48 3.0 -> 1.8 ms, 4 -> 5 degrees
@@ -110,7 +111,7 @@ size_t rounded(size_t bytes) {
     return (bytes + step - 1) / step * step;
 }
 
-// Wait for the device's pending work (the caller has made it current).
+// Wait for the device's pending work (the caller has made it current).  No lock held.
 bool device_wait() {
     void *p = nullptr;
     if (hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess) return true;
@@ -127,11 +128,13 @@ std::multimap<size_t, Free>::iterator find(Device &d, size_t bytes, F ok) {
     return d.free.end();
 }
 
-// Wait until the free blocks in state st are clean.
-bool wait_and_clean(Device &d, State st) {
+// Wait without the lock until the free blocks in state st are clean.
+bool wait_and_clean(Device &d, State st, Lock &lock) {
     const uint64_t now = d.frees;
+    lock.unlock();
     const bool done = st == kNull ? hipStreamSynchronize(nullptr) == hipSuccess : device_wait();
     if (!done) (void)hipGetLastError();
+    lock.lock();
     if (done)
         for (auto &f : d.free)
             if (f.second.stamp < now && f.second.state == st) f.second.state = kClean;
@@ -140,8 +143,8 @@ bool wait_and_clean(Device &d, State st) {
 
 // Give blocks back to the driver: the oldest until `most` bytes are kept, and those
 // older than `before`.  Blocks of running calls stay, but for this thread's own when
-// `own`.  The caller has made the device current.
-void trim(Device &d, size_t most, uint64_t before, bool own) {
+// `own`.  The caller has made the device current and holds the lock.
+void trim(Device &d, size_t most, uint64_t before, bool own, Lock &lock) {
     auto mine = [&](const Free &f) { return own && f.call && f.call == t_call.id; };
     std::vector<std::multimap<size_t, Free>::iterator> order;
     for (auto it = d.free.begin(); it != d.free.end(); ++it)
@@ -155,6 +158,7 @@ void trim(Device &d, size_t most, uint64_t before, bool own) {
         d.free.erase(it);
     }
     if (out.empty()) return;
+    lock.unlock();
     auto give = [](const Free &f) {
         if (f.pool) (void)hipFreeAsync(f.p, f.state == kCall ? f.stream : nullptr);
         else (void)hipFree(f.p);
@@ -169,6 +173,7 @@ void trim(Device &d, size_t most, uint64_t before, bool own) {
         back.clear();
     }
     (void)hipGetLastError();
+    lock.lock();
     for (auto &b : back) {
         d.free.insert(b);
         d.kept += b.first;
@@ -176,14 +181,14 @@ void trim(Device &d, size_t most, uint64_t before, bool own) {
 }
 
 // Keep the bounds of device `index`, on whatever device this thread is.
-void bound(Device &d, int index) {
+void bound(Device &d, int index, Lock &lock) {
     const uint64_t before = d.frees > kKeep ? d.frees - kKeep : 0;
     const bool over = d.kept > d.cap;
     if (!over && !(before && d.frees % 64 == 0)) return;
     int dev = index;
     if (hipGetDevice(&dev) != hipSuccess) return;
     if (dev != index && hipSetDevice(index) != hipSuccess) return;
-    trim(d, d.cap, before, false);
+    trim(d, over ? d.cap / 4 * 3 : d.cap, before, false, lock);
     if (dev != index) (void)hipSetDevice(dev);
 }
 
@@ -205,13 +210,15 @@ void end_call() {
         else if (std::find(pending.begin(), pending.end(), f.stream) == pending.end()) pending.push_back(f.stream);
     });
     for (hipStream_t s : pending) {
+        lock.unlock();
         const State st = hipStreamSynchronize(s) == hipSuccess ? kClean : kUnknown;
         if (st != kClean) (void)hipGetLastError();
+        lock.lock();
         freed_by_call(c, [&](Free &f) {
             if (f.stream == s) f.state = st;
         });
     }
-    for (auto &dev : c.devices) bound(dev.second, dev.first);
+    for (auto &dev : c.devices) bound(dev.second, dev.first, lock);
 }
 
 }  // namespace
@@ -276,7 +283,7 @@ void *device_alloc(size_t bytes, Memory use, hipStream_t s) {
     for (State st : {kNull, kUnknown}) {
         if (it != d.free.end() || use == kTemporary) break;
         auto in_state = [st](const Free &f) { return f.state == st; };
-        if (find(d, want, in_state) != d.free.end() && wait_and_clean(d, st)) it = find(d, want, usable);
+        if (find(d, want, in_state) != d.free.end() && wait_and_clean(d, st, lock)) it = find(d, want, usable);
     }
     if (it != d.free.end()) {
         void *p = it->second.p;
@@ -285,16 +292,20 @@ void *device_alloc(size_t bytes, Memory use, hipStream_t s) {
         d.free.erase(it);
         return p;
     }
+    lock.unlock();
     auto fresh = [&](void **p) { return ordered ? hipMallocAsync(p, want, s) : hipMalloc(p, want); };
     void *p = nullptr;
     hipError_t e = fresh(&p);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        trim(d, 0, UINT64_MAX, true);
+        lock.lock();
+        trim(d, 0, UINT64_MAX, true, lock);
+        lock.unlock();
         (void)device_wait();
         e = fresh(&p);
     }
     CR_HIP(e);
+    lock.lock();
     c.live[p] = {want, dev, ordered};
     return p;
 }
@@ -315,7 +326,7 @@ void device_free(void *p, bool ordered, hipStream_t s) {
         c.live.erase(l);
         d.frees++;
         d.kept += b.bytes;
-        bound(d, b.device);
+        bound(d, b.device, lock);
     } catch (const std::exception &) {  // no host memory for the list: the block is lost, not handed out twice
     }
 }

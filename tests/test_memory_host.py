@@ -1,5 +1,5 @@
-"""The library's device memory on the host: who gets a freed block, and what the driver
-is asked to do for it."""
+"""The library's device memory on the host: who gets a freed block, what the driver
+is asked to do for it, and that nobody waits for another thread's driver call."""
 import ctypes
 import os
 import subprocess
@@ -163,14 +163,31 @@ def test_capturing_streams_are_refused(mem, use):
     assert mem.alloc(use, SIDE) is not None
 
 
+def test_no_lock_is_held_while_the_driver_works(mem):
+    p = mem.alloc(ANY, NULL)
+    mem.lib.handle_free(p, UNUSED)
+    mem.lib.hold(1)
+    with ThreadPoolExecutor(2) as ex:
+        try:
+            slow = ex.submit(mem.alloc, KEPT, SIDE, 50 * N)  # stops inside the driver
+            assert mem.lib.wait_held()
+            quick = ex.submit(lambda: (mem.alloc(ANY, NULL), mem.lib.handle_free(p, UNUSED)))
+            assert quick.result(timeout=20)[0] == p
+        finally:
+            mem.lib.hold(0)
+        assert slow.result(timeout=20)
+
+
 @pytest.mark.parametrize("bits", [UNUSED, ON_NULL, ELSEWHERE])
 def test_kept_memory_is_bounded(mem, bits):
-    """1/64 of the device (1 MB here)."""
+    """1/64 of the device (1 MB here); past it a few larger trims, not one a free."""
     live = [mem.alloc(KEPT, SIDE, 30000 + 17000 * i) for i in range(24)]
     mem.log()
     for p in live:
         mem.lib.handle_free(p, bits)
     assert 0.5 * MB <= mem.lib.used() <= MB
+    waits = mem.log().count("malloc")
+    assert waits == (0 if bits != ELSEWHERE else waits) and waits <= 12
 
 
 def test_temporaries_past_the_bound(mem):
