@@ -234,7 +234,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC == 4
     const int32_t *__restrict__ rowid, const int32_t *__restrict__ col, const double *__restrict__ coef,
     int64_t nnz, const double *__restrict__ dst_cells, int dst_nv, const int32_t *__restrict__ dst_vi,
     const double *__restrict__ src_cells, int src_nv, const int32_t *__restrict__ src_vi, int clip_is_dst, int window,
-    int private_v, AreaTerm area, double *__restrict__ g_dst, double *__restrict__ g_src, int32_t *__restrict__ list,
+    AreaTerm area, double *__restrict__ g_dst, double *__restrict__ g_src, int32_t *__restrict__ list,
     uint32_t *__restrict__ count) {
     // a lane's arcs of subject edges (M_p, M_q), then its source vertices' gradients
     __shared__ double own[64 * kOwn<M>];
@@ -449,14 +449,13 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC == 4
         rows[3 * i + 2] = g[t].z;
     }
     __syncthreads();
-    // cells that own their vertices: only the first and last row can be another wave's too
-    const int lo = private_v ? dst_nv * 3 : 3 * n, hi = private_v ? (int)(last - 1) * dst_nv * 3 : 0;
+    // atomics for cells that own their vertices, too: the buffer may be g_src as
+    // well, or another call's on another stream (plain adds to a wave's inner rows
+    // took 1.81 ms instead of 1.87 for the whole reverse mode of quarter degree ->
+    // HEALPix 256, and lost updates there)
     for (int i = lane; i < 3 * n; i += 64) {
         const double v = rows[i];
-        if (v == 0.0) continue;
-        double *to = g_dst + 3 * (int64_t)dst_vi[r0 * dst_nv + i / 3] + i % 3;
-        if (i >= lo && i < hi) *to += v;
-        else atomicAdd(to, v);
+        if (v != 0.0) atomicAdd(g_dst + 3 * (int64_t)dst_vi[r0 * dst_nv + i / 3] + i % 3, v);
     }
 }
 
@@ -518,14 +517,14 @@ __global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
 // Workgroups of the list pass (the waves stride over the declined pairs).
 constexpr unsigned kListBlocks = 2048;
 
-// d(area of each destination cell)/dV times dL/da_u.  private_v: no vertex
-// index is shared by two cells, so each thread owns its cell's entries of g
-// and adds without atomics (the kernels before it on the stream have finished).
+// d(area of each destination cell)/dV times dL/da_u.  (Like all of the reverse
+// mode it adds to g by atomics, whoever owns a vertex: other calls may be adding
+// to the same buffer.)
 __global__ void k_area_grad(const double *__restrict__ cells, int nv, const int32_t *__restrict__ vi,
                             int64_t ncells, double kappa, const double *__restrict__ a_to, int64_t nf,
                             const double *__restrict__ y, int64_t yc, int64_t yf,
                             const double *__restrict__ gy, int64_t gc, int64_t gf,
-                            double *__restrict__ g, int private_v) {
+                            double *__restrict__ g) {
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ncells || a_to[t] == 0.0) return;  // zero-area (ghost) cells have no area term
     double s = 0.0;
@@ -535,19 +534,13 @@ __global__ void k_area_grad(const double *__restrict__ cells, int nv, const int3
     const int32_t *v = vi + (int64_t)nv * t;
     ring_area_backward(cells + 3 * (int64_t)nv * t, nv, c, [&](int slot, const d3 &d) {
         double *gv = g + 3 * (int64_t)v[slot];
-        if (private_v) {
-            gv[0] += d.x;
-            gv[1] += d.y;
-            gv[2] += d.z;
-        } else {
-            atomicAdd(gv, d.x);
-            atomicAdd(gv + 1, d.y);
-            atomicAdd(gv + 2, d.z);
-        }
+        atomicAdd(gv, d.x);
+        atomicAdd(gv + 1, d.y);
+        atomicAdd(gv + 2, d.z);
     });
 }
 
-// The same for grids whose cells own their vertices (private_v) with at most
+// The same for grids whose cells own their vertices, with at most
 // kStagedNv vertices per cell: a workgroup's 64 cells are one contiguous run of
 // vertex data and of g (each cell's caller vertices are its own slots, in some
 // order), so both are staged through LDS with coalesced loads and stores
@@ -569,7 +562,7 @@ __global__ void __launch_bounds__(64) k_area_grad_private(const double *__restri
     double *gb = g + 3 * (int64_t)nv * c0;
     for (int i = threadIdx.x; i < n; i += 64) {
         vin[i] = src[i];
-        gout[i] = gb[i];
+        gout[i] = 0.0;
     }
     __syncthreads();
     const int t = threadIdx.x;
@@ -590,7 +583,8 @@ __global__ void __launch_bounds__(64) k_area_grad_private(const double *__restri
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += 64) gb[i] = gout[i];
+    for (int i = threadIdx.x; i < n; i += 64)
+        if (gout[i] != 0.0) atomicAdd(gb + i, gout[i]);
 }
 
 // The same for tables of NV-vertex cells whose slot -> vertex map is the
@@ -659,7 +653,8 @@ __global__ void __launch_bounds__(128) k_area_grad_table(const double *__restric
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += 128) gb[i] += stage[i];
+    for (int i = threadIdx.x; i < n; i += 128)
+        if (stage[i] != 0.0) atomicAdd(gb + i, stage[i]);
 }
 
 __global__ void k_div_rows(const double *__restrict__ gy, int64_t gc, int64_t gf, int64_t n, int64_t nf,
@@ -773,7 +768,7 @@ static void backward(const cr_regridder *R, const cr_grid *dst, const cr_grid *s
             constexpr int NC = decltype(nc)::value;
             hipLaunchKernelGGL((k_clip_grad_arcs<NC, decltype(mask)>), dim3(grid_for(F.nnz, 64)), dim3(64), arcs_lds, s,
                                rowid, F.col.p, coef, F.nnz, dst->cells.p, dst->nv, dst->vidx.p, src->cells.p, src->nv,
-                               src->vidx.p, (int)cd, window, dst->private_vertices, area, g_dst_verts, g_src_verts,
+                               src->vidx.p, (int)cd, window, area, g_dst_verts, g_src_verts,
                                list, count);
             hipLaunchKernelGGL(k_clip_grad_list<NC>, dim3(kListBlocks), dim3(64), lds, s, rowid, F.col.p, coef,
                                dst->cells.p, dst->nv, dst->vidx.p, src->cells.p, src->nv, src->vidx.p,
@@ -811,8 +806,7 @@ static void backward(const cr_regridder *R, const cr_grid *dst, const cr_grid *s
                                gto->vidx.p, n_to, kappa, a_to, nfields, y, yc, yf, gy, gc, gf, g_to);
         else
             hipLaunchKernelGGL(k_area_grad, dim3(grid_for(n_to, B)), dim3(B), 0, s, gto->cells.p, gto->nv,
-                               gto->vidx.p, n_to, kappa, a_to, nfields, y, yc, yf, gy, gc, gf, g_to,
-                               gto->private_vertices);
+                               gto->vidx.p, n_to, kappa, a_to, nfields, y, yc, yf, gy, gc, gf, g_to);
     }
     CR_HIP(hipGetLastError());
     release(coef_b, rowid_b);
