@@ -22,6 +22,44 @@
 
 namespace cr {
 
+// Gradients of one line's two vertices into caller vertices.
+__device__ __forceinline__ void add_line(double *g, const int32_t *vi, int j, int j1, const d3 &p, const d3 &q,
+                                         double w, const LineSum &S) {
+    if (!g) return;
+    d3 gp, gq;
+    line_grad(p, q, LineSum{w * S.p, w * S.q}, gp, gq);
+    atomicAdd(g + 3 * (int64_t)vi[j], gp.x);
+    atomicAdd(g + 3 * (int64_t)vi[j] + 1, gp.y);
+    atomicAdd(g + 3 * (int64_t)vi[j] + 2, gp.z);
+    atomicAdd(g + 3 * (int64_t)vi[j1], gq.x);
+    atomicAdd(g + 3 * (int64_t)vi[j1] + 1, gq.y);
+    atomicAdd(g + 3 * (int64_t)vi[j1] + 2, gq.z);
+}
+
+// The destination cells' area term: cell i's area has dL/da_i = -kappa / a_i
+// sum_f gy_if y_if (y null: no term).
+struct AreaTerm {
+    const double *y, *gy, *a_to;
+    const int64_t *rowptr;
+    int64_t yc, yf, gc, gf, nf;
+    double kappa;
+};
+__device__ __forceinline__ double area_coef(const AreaTerm &A, int64_t i) {
+    if (A.a_to[i] == 0.0) return 0.0;  // zero-area (ghost) cells have no area term
+    double s = 0.0;
+    for (int64_t f = 0; f < A.nf; ++f) s += A.gy[i * A.gc + f * A.gf] * A.y[i * A.yc + f * A.yf];
+    return -A.kappa * s / A.a_to[i];
+}
+// ... of a cell by itself, as lines that are boundary all along.
+__device__ __forceinline__ void add_area(const double *cell, int nv, const int32_t *vi, double c, double *g) {
+    for (int v = 0; v < nv; ++v) {
+        const int v1 = v + 1 == nv ? 0 : v + 1;
+        const d3 p = load3(cell + 3 * v), q = load3(cell + 3 * v1);
+        const double h = whole_sum(p, q);
+        add_line(g, vi, v, v1, p, q, c, LineSum{h, h});
+    }
+}
+
 // Per non-zero of CSR(A) (rows = dst, cols = src), one thread each: the
 // coefficient dL/dA_u,ij (unit-sphere areas).
 __global__ void k_pair_coef(const int32_t *__restrict__ rowid, const int32_t *__restrict__ col, int64_t nnz,
@@ -172,37 +210,8 @@ __device__ __forceinline__ void flush_rows(const double *lacc, int64_t r0, int64
     }
 }
 
-// Gradients of one line's two vertices into caller vertices.
-__device__ __forceinline__ void add_line(double *g, const int32_t *vi, int j, int j1, const d3 &p, const d3 &q,
-                                         double w, const LineSum &S) {
-    if (!g) return;
-    d3 gp, gq;
-    line_grad(p, q, LineSum{w * S.p, w * S.q}, gp, gq);
-    atomicAdd(g + 3 * (int64_t)vi[j], gp.x);
-    atomicAdd(g + 3 * (int64_t)vi[j] + 1, gp.y);
-    atomicAdd(g + 3 * (int64_t)vi[j] + 2, gp.z);
-    atomicAdd(g + 3 * (int64_t)vi[j1], gq.x);
-    atomicAdd(g + 3 * (int64_t)vi[j1] + 1, gq.y);
-    atomicAdd(g + 3 * (int64_t)vi[j1] + 2, gq.z);
-}
-
 // Destination rows of a wave summed in LDS: at most 256 lines of three doubles.
 inline int arc_rows(int dst_nv) { return std::max(1, std::min(64, 256 / dst_nv)); }
-
-// The destination cells' area term: cell i's area has dL/da_i = -kappa / a_i
-// sum_f gy_if y_if (y null: no term).
-struct AreaTerm {
-    const double *y, *gy, *a_to;
-    const int64_t *rowptr;
-    int64_t yc, yf, gc, gf, nf;
-    double kappa;
-};
-__device__ __forceinline__ double area_coef(const AreaTerm &A, int64_t i) {
-    if (A.a_to[i] == 0.0) return 0.0;  // zero-area (ghost) cells have no area term
-    double s = 0.0;
-    for (int64_t f = 0; f < A.nf; ++f) s += A.gy[i * A.gc + f * A.gf] * A.y[i * A.yc + f * A.yf];
-    return -A.kappa * s / A.a_to[i];
-}
 
 // Subject edges a pair may have inside the clip polygon in part (more: declined),
 // kept in LDS; a quad's are at most 4, a 16-gon's rarely more than 8.
@@ -257,17 +266,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC == 4
     if (area.y && g_dst) {
         for (int64_t r = lane; r < last; r += 64) {
             const double c = area.rowptr[r0 + r] >= k0 ? area_coef(area, r0 + r) : 0.0;
-            if (r < window) {
+            if (r < window)
                 acoef[r] = c;
-            } else if (c != 0.0) {
-                const double *cell = dst_cells + 3 * (int64_t)dst_nv * (r0 + r);
-                for (int v = 0; v < dst_nv; ++v) {
-                    const int v1 = v + 1 == dst_nv ? 0 : v + 1;
-                    const d3 p = load3(cell + 3 * v), q = load3(cell + 3 * v1);
-                    const double h = whole_sum(p, q);
-                    add_line(g_dst, dst_vi + (r0 + r) * dst_nv, v, v1, p, q, c, LineSum{h, h});
-                }
-            }
+            else if (c != 0.0)
+                add_area(dst_cells + 3 * (int64_t)dst_nv * (r0 + r), dst_nv, dst_vi + (r0 + r) * dst_nv, c, g_dst);
         }
     }
     if (w != 0.0) {
@@ -512,7 +514,21 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
     }
 }
 
-__global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
+// Before the vertex pass: its list's count, and the area term of the destination rows
+// that no wave of the pass has -- rows without a non-zero that do not lie between two
+// non-zeros of one wave.  (The term is 0 there, but for an upstream gradient that is
+// not finite, or a y that is not the forward's.)
+__global__ void k_vertex_start(uint32_t *__restrict__ count, AreaTerm area, int64_t n_rows, int64_t nnz,
+                               const double *__restrict__ dst_cells, int dst_nv, const int32_t *__restrict__ dst_vi,
+                               double *__restrict__ g_dst) {
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r == 0) *count = 0u;
+    if (r >= n_rows || !area.y || !g_dst) return;
+    const int64_t k = area.rowptr[r];
+    if (k != area.rowptr[r + 1] || (k % 64 != 0 && k != nnz)) return;
+    const double c = area_coef(area, r);
+    if (c != 0.0) add_area(dst_cells + 3 * (int64_t)dst_nv * r, dst_nv, dst_vi + r * dst_nv, c, g_dst);
+}
 
 // Workgroups of the list pass (the waves stride over the declined pairs).
 constexpr unsigned kListBlocks = 2048;
@@ -745,25 +761,25 @@ static void backward(const cr_regridder *R, const cr_grid *dst, const cr_grid *s
         hipLaunchKernelGGL(k_pair_coef, dim3(grid_for(F.nnz, B)), dim3(B), 0, s, rowid, F.col.p, F.nnz,
                            (int)(transpose != 0), (int)(normalize != 0), kappa, a_to, nfields, x, xc, xf, gy, gc,
                            gf, coef);
+    DevBuf<int32_t> list_b;
+    DevBuf<uint32_t> count_b;
+    int32_t *list = ws ? ws->list : nullptr;
+    uint32_t *count = ws ? ws->count : nullptr;
+    if (!ws) {
+        list_b.alloc_async(F.nnz, s);
+        count_b.alloc_async(1, s);
+        list = list_b.p;
+        count = count_b.p;
+    }
+    const AreaTerm area{normalize && !transpose ? y : nullptr, gy, a_to, F.rowptr.p, yc, yf, gc, gf, nfields, kappa};
+    hipLaunchKernelGGL(k_vertex_start, dim3(grid_for(area.y ? F.nrows : 1, B)), dim3(B), 0, s, count, area, F.nrows,
+                       F.nnz, dst->cells.p, dst->nv, dst->vidx.p, g_dst_verts);
     if (F.nnz) {
         // most pairs by boundary arcs; the pairs that declines through the clip pipeline
-        DevBuf<int32_t> list_b;
-        DevBuf<uint32_t> count_b;
-        int32_t *list = ws ? ws->list : nullptr;
-        uint32_t *count = ws ? ws->count : nullptr;
-        if (!ws) {
-            list_b.alloc_async(F.nnz, s);
-            count_b.alloc_async(1, s);
-            list = list_b.p;
-            count = count_b.p;
-        }
-        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, count);  // a kernel: no memset node in a graph
         const size_t lds = (size_t)kGradRows * dst->nv * 3 * sizeof(double);
         const bool cd = R->stats.clip_with_dst != 0;
         const int window = arc_rows(dst->nv);
         const size_t arcs_lds = (size_t)window * dst->nv * 3 * sizeof(double);
-        const AreaTerm area{normalize && !transpose ? y : nullptr, gy, a_to, F.rowptr.p, yc, yf, gc, gf, nfields,
-                            kappa};
         auto vertex_pass = [&](auto nc, auto mask) {
             constexpr int NC = decltype(nc)::value;
             hipLaunchKernelGGL((k_clip_grad_arcs<NC, decltype(mask)>), dim3(grid_for(F.nnz, 64)), dim3(64), arcs_lds, s,
@@ -809,7 +825,7 @@ static void backward(const cr_regridder *R, const cr_grid *dst, const cr_grid *s
                                gto->vidx.p, n_to, kappa, a_to, nfields, y, yc, yf, gy, gc, gf, g_to);
     }
     CR_HIP(hipGetLastError());
-    release(coef_b, rowid_b);
+    release(coef_b, rowid_b, list_b, count_b);
     if (!ws) synchronise(s);
 }
 
