@@ -394,7 +394,7 @@ static bool levels_layout(const Csr &A, int dtype, int64_t nf, int64_t sf, int64
     if (sf != 1 || df != 1) return false;
     const int64_t mean = A.nnz / std::max<int64_t>(1, A.nrows);
     if (dtype == CR_F64) return A.f64_variant < 0 && nf >= std::max<int64_t>(6, std::min<int64_t>(16, mean / 4));
-    return nf >= 64 || (A.tuned_variant < 0 && nf >= (mean <= 8 ? 6 : 16));
+    return nf >= 64 || (!A.pinned && nf >= (mean <= 8 ? 6 : 16));
 }
 
 // Kernel choice: fields side by side -> levels.hip; other FP64 layouts -> the
@@ -627,6 +627,7 @@ cr_status cr_regrid_tune(cr_regridder *R, int32_t transpose, int64_t nfields, co
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         A.tuned_variant = best;
+        A.pinned = false;
         if (chosen) *chosen = best;
         if (best_ms) *best_ms = best_t;
     });
@@ -643,8 +644,12 @@ cr_status cr_regrid_set_variant(cr_regridder *R, int32_t transpose, int32_t dtyp
         const int n = dtype == CR_F32 ? kNumVariants : kNumF64Variants;
         CR_REQUIRE(variant >= -1 && variant < n, CR_INVALID_ARGUMENT, "cr_regrid_set_variant: no such variant");
         Csr &A = transpose ? R->bwd : R->fwd;
-        if (dtype == CR_F32) A.tuned_variant = variant;
-        else A.f64_variant = variant;
+        if (dtype == CR_F32) {
+            A.tuned_variant = variant;
+            A.pinned = variant >= 0;
+        } else {
+            A.f64_variant = variant;
+        }
     });
 }
 

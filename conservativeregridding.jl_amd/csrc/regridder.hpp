@@ -55,6 +55,7 @@ struct Csr {
     // the transposed matrix, each of whose rows has its columns ascending; null: none
     const Csr *transposed = nullptr;
     int tuned_variant = -1;    // FP32 kernel variant (cr_regrid_tune / set_variant); -1: default
+    bool pinned = false;       // by set_variant: fields side by side use it, too
     mutable std::atomic<int> default_variant{-1};  // the default FP32 variant chosen for this matrix; -1: not yet
     int f64_variant = -1;      // FP64 kernel variant; -1: default
     // Kernel plans, made on first use (guarded: handles are shared by callers):

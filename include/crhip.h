@@ -347,7 +347,8 @@ cr_status cr_regrid_backward_noalloc(const cr_regridder *R, const cr_grid *dst, 
  * variant with the default's numerics (products and sums in FP64 from the FP64
  * A: variants 8-17, 25 and 28) on the given device fields (dst is overwritten
  * with the regridded result) and stores the fastest in the handle for that
- * direction; later cr_regrid calls of that direction use it.  Variants that
+ * direction; later cr_regrid calls of that direction use it (but for fields side
+ * by side, which have a kernel of their own, see below).  Variants that
  * round A to FP32 or sum in FP32 are used only when pinned
  * (cr_regrid_set_variant).  Synchronises the stream.
  */
@@ -383,7 +384,7 @@ cr_status cr_regrid_tune(cr_regridder *R, int32_t transpose, int64_t nfields, co
  *           apply).  Fields side by side (unit field strides) have a kernel
  *           of their own: FP32 with >= 64 fields always, with fewer (>= 6, or
  *           16 where rows have more than 8 non-zeros on average) unless a
- *           variant is pinned or tuned; FP64 sums of the FP64 A, no plan.
+ *           variant is pinned; FP64 sums of the FP64 A, no plan.
  *   CR_F64: 0 row kernel, 1 staged tile kernel (default; unit field strides
  *           and >= 6 fields, more for long rows: the side-by-side kernel, with
  *           the tile kernel's plan and results).
