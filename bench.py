@@ -875,8 +875,9 @@ def main():
         # clip stage's time.  The vertex-gradient pass (k_clip_grad_arcs, which
         # carries the area term, and the declined pairs' k_clip_grad_list)
         # differentiates the clip of every kept pair: 2x the clip's operations is
-        # counted over the whole pass, a pipeline's work that the pass by boundary
-        # arcs does with less, so the rate is that of equivalent operations.
+        # counted over the whole pass.  That is a pipeline's work, which the pass by
+        # boundary arcs does with less: a rate of equivalent operations, comparable
+        # between versions and no share of the peak.
         peak64 = 78.6e12
         clip_flops = flops_per_cand * ncand
         grad_flops = 2.0 * flops_per_kept * nnz
@@ -889,13 +890,12 @@ def main():
                                "frac": round(clip_flops / (st["ms_clip"] * 1e-3) / peak64, 4),
                                "flops_per_candidate": round(flops_per_cand, 1)},
             "vertex_pass": {"kernels": "k_clip_grad_arcs (with the area term) + k_clip_grad_list",
-                            "flops_lower_bound": grad_flops, "ms_vertex_pass": round(ms_vert, 4),
-                            "achieved_TFLOPs_lower_bound": round(grad_flops / (ms_vert * 1e-3) / 1e12, 3),
-                            "frac_lower_bound": round(grad_flops / (ms_vert * 1e-3) / peak64, 4),
+                            "equivalent_flops": grad_flops, "ms_vertex_pass": round(ms_vert, 4),
+                            "equivalent_TFLOPs": round(grad_flops / (ms_vert * 1e-3) / 1e12, 3),
                             "clip_flops_per_kept_pair": round(flops_per_kept, 1)}}
         log(f"[bench] FP64 rooflines: k_clip_compact {fp64_kernels['k_clip_compact']['achieved_TFLOPs']:.2f} "
-            f"TFLOP/s ({fp64_kernels['k_clip_compact']['frac']:.1%} of 78.6), vertex pass >= "
-            f"{fp64_kernels['vertex_pass']['achieved_TFLOPs_lower_bound']:.2f} TFLOP/s")
+            f"TFLOP/s ({fp64_kernels['k_clip_compact']['frac']:.1%} of 78.6), vertex pass "
+            f"the equivalent of {fp64_kernels['vertex_pass']['equivalent_TFLOPs']:.2f} TFLOP/s")
 
     out = {
         "metric": METRIC,
