@@ -76,6 +76,7 @@ struct CallScope {
     CallScope();
     ~CallScope();
     CallScope(const CallScope &) = delete;
+    bool failed = false;  // it may have left its handles' work pending
 };
 // Wait for stream s: what this call has freed in order on it so far is free for anyone.
 void synchronise(hipStream_t s);
@@ -157,12 +158,15 @@ cr_status guard(F &&f) {
         f();
         return CR_OK;
     } catch (const Error &e) {
+        call.failed = true;
         set_error(e.msg);
         return e.status;
     } catch (const std::bad_alloc &) {
+        call.failed = true;
         set_error("host allocation failed");
         return CR_OUT_OF_MEMORY;
     } catch (const std::exception &e) {
+        call.failed = true;
         set_error(e.what());
         return CR_INTERNAL;
     }

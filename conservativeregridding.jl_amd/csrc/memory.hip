@@ -200,13 +200,14 @@ void freed_by_call(Cache &c, F f) {
             if (b.second.state == kCall && b.second.call == t_call.id) f(b.second);
 }
 
-// The call is over: synchronise the streams it freed temporaries on.
-void end_call() {
+// The call is over: synchronise the streams it freed temporaries on -- after a failure
+// the null stream, too, for the sake of the handles it was reading.
+void end_call(bool failed) {
     Cache &c = cache();
     std::vector<hipStream_t> pending;
     Lock lock(c.mu);
     freed_by_call(c, [&](Free &f) {
-        if (!f.stream) f.state = kNull;
+        if (!f.stream && !failed) f.state = kNull;
         else if (std::find(pending.begin(), pending.end(), f.stream) == pending.end()) pending.push_back(f.stream);
     });
     for (hipStream_t s : pending) {
@@ -228,7 +229,7 @@ CallScope::CallScope() { ++t_call.depth; }
 CallScope::~CallScope() {
     if (--t_call.depth) return;
     try {
-        if (t_call.id && !g_child) end_call();
+        if (t_call.id && !g_child) end_call(failed);
     } catch (const std::exception &) {  // no host memory: the call's blocks stay its own
     }
     t_call = Call{};

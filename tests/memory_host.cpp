@@ -63,6 +63,7 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *st) {
 }
 
 void call_begin(void) { t_scope.reset(new cr::CallScope); }
+void call_fail(void) { t_scope->failed = true; }
 void call_end(void) { t_scope.reset(); }
 // use: 0 temporary, 1 kept, 2 any stream; null: refused or out of memory
 void *mem_alloc(size_t n, int use, void *s) {

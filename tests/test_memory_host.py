@@ -79,6 +79,16 @@ def test_null_stream_temporaries_need_no_synchronisation(mem):
     assert "sync@0" not in mem.log()
 
 
+@pytest.mark.parametrize("stream", [NULL, SIDE])
+def test_a_failed_call_leaves_nothing_pending(mem, stream):
+    """Its grids and regridders may be destroyed next, and count as unused."""
+    mem.lib.call_begin()
+    mem.lib.mem_free(mem.alloc(TEMP, stream), stream)
+    mem.lib.call_fail()
+    mem.lib.call_end()
+    assert mem.log()[-1] == "sync@%d" % stream
+
+
 @pytest.mark.parametrize("stream", [PER_THREAD, SIDE])
 def test_running_calls_keep_their_temporaries(mem, stream):
     """One stream handle on two threads (hipStreamPerThread: two streams)."""
