@@ -234,7 +234,7 @@ constexpr int kOwn = 2 * kArcs<M> + 1;  // a lane's doubles in LDS (odd: lanes o
 // Differentiating every crossing and fan triangle instead, with the crossings
 // queued in LDS, took 15 600 VALU instructions a wave against 5 000 here: the whole
 // vertex pass on quarter degree -> HEALPix 256 (16-gons, nnz 4.35 M), with the
-// declined pairs and the area term, 4.39 -> 1.62 ms; C96 -> 1 degree 276 -> 100 us.
+// declined pairs and the area term, 4.39 -> 1.68 ms; C96 -> 1 degree 276 -> 100 us.
 // The lane-to-double mapping of the atomics matters as much: with a lane per pair
 // and vertex this kernel ran 2.55 ms.  Three waves a SIMD (168 registers, a few
 // spilled) against two: 1.88 and 2.11 ms for the whole reverse mode.
