@@ -298,7 +298,9 @@ void launch(const Csr &A, const TilePlan *P, const T *x, int64_t xc, T *y, int64
     const int64_t chunk = (int64_t)lpr * V;
     const int64_t gy = (nf + chunk - 1) / chunk;
     CR_REQUIRE(gy <= 65535, CR_UNSUPPORTED, "too many fields for one launch");
-    // two rows a thread group where their entries fit the stage
+    // two rows a thread group where their entries fit the stage (FP32: one where two
+    // would leave fewer than 1024 blocks: 37 fields of 360 x 180 -> C48 14.7 -> 9.1
+    // us, of 2592 rows 3.9 -> 3.3)
     const int groups = kLevelThreads / lpr;
     const int64_t mean = (A.nnz + A.nrows - 1) / A.nrows;
     int run, parts = 1, wide_blocks = 0;
@@ -309,14 +311,18 @@ void launch(const Csr &A, const TilePlan *P, const T *x, int64_t xc, T *y, int64
     if (EVEN) {
         // every part's block reads its tile's row starts (4 KB), so runs are long
         // where that leaves enough blocks: 33 fields of 786 k rows take 201 us
-        // with runs of 128, 163 with 256, 151 with 512
-        const int64_t even = std::min<int64_t>(512, std::max<int64_t>(128, A.nnz / 4096));
+        // with runs of 128, 163 with 256, 151 with 512.  Where 128 leaves few
+        // blocks they are shorter, down to two rows a thread group: 64 fields of
+        // 2592 rows take 21.5 us with runs of 128, 10.6 with 8; 100 fields of C24
+        // -> 180 x 90 23.5 with 128, 14.1 with 36
+        const int64_t even =
+            std::min<int64_t>(512, std::max<int64_t>(std::min<int64_t>(128, A.nnz * gy / 1024), A.nnz / 4096));
         run = (int)std::min<int64_t>(kStageEven / 4 * 3, std::max<int64_t>(even, 2 * groups * mean));
         parts = (int)((A.nnz / P->ntiles + run - 1) / run);  // of a tile with the mean number of non-zeros
         parts = std::max(1, parts);
         units = P->ntiles * parts;
     } else {
-        run = (int)std::min<int64_t>(2 * groups, kLevelThreads);
+        run = (int)std::min<int64_t>(A.nrows < 2048 * (int64_t)groups ? groups : 2 * groups, kLevelThreads);
         if (run * mean > kStage / 4 * 3) run = std::max<int>(std::min<int64_t>(groups, kStage / 4 * 3 / mean), 1);
         units = (A.nrows + run - 1) / run;
         wide_blocks = (int)std::min<int64_t>(8192, (A.wide_cap + 7) / 8 * 8);  // 0 when no row can be wide
