@@ -397,6 +397,16 @@ static bool levels_layout(const Csr &A, int dtype, int64_t nf, int64_t sf, int64
     return nf >= 64 || (!A.pinned && nf >= (mean <= 8 ? 6 : 16));
 }
 
+// FP64 fields, once the plan is there: in a small matrix with wide rows (a pole's)
+// the thread groups that run through them take longer than all the rest, whatever
+// the number of fields, and the tile kernel is ahead for more of them.  180 x 90 ->
+// C24 (36 k non-zeros), k = 6: 17.1 / 8.8, 12: 17.3 / 14.4, 16: 16.3 / 18.2; 360 x
+// 180 -> C48 (145 k), k = 6: 19.8 / 11.2, 10: 19.8 / 16.5, 12: 19.5 / 19.0; 720 x
+// 361 -> C90 (520 k), k = 6: 25.0 / 27.7.
+static bool levels_ahead(const Csr &A, const TilePlan &P, int64_t nf) {
+    return P.nwide == 0 || nf >= 16 || A.nnz >= (1 << 18) || (A.nnz >= (1 << 17) && nf >= 13);
+}
+
 // Kernel choice: fields side by side -> levels.hip; other FP64 layouts -> the
 // tile kernel (1 or 2 fields per stage) unless the row kernel is pinned; other
 // FP32 layouts -> the autotuned (or pinned, or default: 1024-row tiles, 4
@@ -412,10 +422,10 @@ void apply(const cr_regridder *R, bool transpose, int dtype, int64_t nf, const v
         double *y = (double *)dst;
         const double *ar = normalize ? area : nullptr;
         const int v = A.f64_variant >= 0 ? A.f64_variant : kDefaultF64Variant;
-        if (levels_layout(A, dtype, nf, sf, df)) {
-            const TilePlan &P = tile_plan(A, kEven, kGeomS, s, false);
-            launch_levels(A, P, x, sc, y, dc, nf, ar, s);
-            launch_huge<double>(A, P, x, sc, sf, y, dc, df, nf, ar, nullptr, s);
+        const TilePlan *P = levels_layout(A, dtype, nf, sf, df) ? &tile_plan(A, kEven, kGeomS, s, false) : nullptr;
+        if (P && levels_ahead(A, *P, nf)) {
+            launch_levels(A, *P, x, sc, y, dc, nf, ar, s);
+            launch_huge<double>(A, *P, x, sc, sf, y, dc, df, nf, ar, nullptr, s);
         } else if (v == 1)
             launch_tiled<double>(A, kGeomS, nf >= 2 ? 2 : 1, false, 0, 0, x, sc, sf, y, dc, df, nf, ar, nullptr,
                                  s);

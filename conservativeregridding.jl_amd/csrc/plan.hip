@@ -367,6 +367,7 @@ template <class G>
 __global__ void __launch_bounds__(kPlanThreads) k_plan_emit(int64_t nrows, const int4 *__restrict__ table,
                                                             const int4 *__restrict__ exits,
                                                             const int2 *__restrict__ sub, TileRec *__restrict__ recs,
+                                                            const int32_t *__restrict__ nwide,
                                                             int64_t *__restrict__ totals) {
     __shared__ int4 e[kChunk];
     const int64_t nA = (nrows + kRowAlign - 1) / kRowAlign, base = (int64_t)blockIdx.x * kChunk;
@@ -407,6 +408,7 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan_emit(int64_t nrows, const
         totals[0] = t;
         totals[1] = ent_total;
         totals[2] = col_total;
+        totals[3] = nwide ? *nwide : 0;
     }
 }
 
@@ -791,25 +793,26 @@ void make_plan(const Csr &A, TilePlan &P, hipStream_t s) {
     DevBuf<int4> table(nA, s), exits(nA, s);
     DevBuf<int2> sub(nA * kRowAlign, s);
     DevBuf<TileRec> recs(nrows > 0 ? nrows : 1, s);
-    DevBuf<int64_t> totals(3, s);
+    DevBuf<int64_t> totals(4, s);
     DevBuf<int64_t> hflag(nrows + 1, s), hpos(nrows + 1, s);
     hipLaunchKernelGGL((k_plan_table<G, STYLE>), dim3((unsigned)nA), dim3(kPlanThreads), 0, s, nrows, A.rowptr.p,
                        prev.p, table.p, sub.p);
     hipLaunchKernelGGL(k_plan_chunk, dim3((unsigned)nC), dim3(kPlanThreads), 0, s, nrows, table.p, exits.p);
     hipLaunchKernelGGL(k_plan_emit<G>, dim3((unsigned)nC), dim3(kPlanThreads), 0, s, nrows, table.p, exits.p, sub.p,
-                       recs.p, totals.p);
+                       recs.p, A.nwide, totals.p);
     CR_HIP(hipMemsetAsync(hflag.p + nrows, 0, sizeof(int64_t), s));
     hipLaunchKernelGGL(k_huge_flags, dim3(grid_for(nrows, 256)), dim3(256), 0, s, nrows, A.rowptr.p,
                        (int64_t)G::kCols, hflag.p);
     exclusive_sum<int64_t *, int64_t *>(T, hflag.p, hpos.p, nrows + 1, s);
     CR_HIP(hipGetLastError());
-    int64_t h[3], nh = 0;
+    int64_t h[4], nh = 0;
     CR_HIP(hipMemcpyAsync(h, totals.p, sizeof(h), hipMemcpyDeviceToHost, s));
     CR_HIP(hipMemcpyAsync(&nh, hpos.p + nrows, sizeof(nh), hipMemcpyDeviceToHost, s));
     synchronise(s);
     P.ntiles = h[0];
     P.nslots = h[1];
     P.nhuge = nh;
+    P.nwide = h[3];
     P.tiles.alloc_kept(P.ntiles, s);
     P.key.alloc_kept(P.nslots, s);
     P.val32.alloc_kept(P.nslots, s);

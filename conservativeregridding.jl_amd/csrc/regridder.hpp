@@ -33,6 +33,7 @@ struct TilePlan {
     // plan's rows are 32-row blocks of the matrix in an order of their own
     DevBuf<int32_t> rowmap;
     int64_t nhuge = 0;
+    int64_t nwide = 0;       // rows with more than kWideRow non-zeros (plans in the matrix's row order)
     int64_t nslots = 0;
     // the tiles' distinct columns and the 32-column lines (128 bytes of an FP32
     // field) they touch, summed over tiles: lines * 32 / cols is the plan's
