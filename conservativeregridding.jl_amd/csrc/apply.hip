@@ -177,9 +177,24 @@ __global__ void __launch_bounds__(256) k_row_ids(const int64_t *__restrict__ row
     }
 }
 
+// The same for long rows, a wave each.
+__global__ void __launch_bounds__(256) k_row_ids_long(const int64_t *__restrict__ rowptr, int64_t nrows,
+                                                      int32_t *__restrict__ row) {
+    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= nrows) return;
+    const int64_t end = rowptr[r + 1];
+    for (int64_t k = rowptr[r] + (threadIdx.x & 63); k < end; k += 64) row[k] = (int32_t)r;
+}
+
+// A block of 256 rows has 256 times the mean row's non-zeros to write: a matrix onto
+// a few cells would leave all of them to a block or two (1440 x 720 onto 18 x 9, 162
+// rows of 6500: 2134 us, by waves 5; onto 240 x 120, 42 a row: 27 and 5).
 void row_ids(const Csr &A, int32_t *row, hipStream_t s) {
     if (A.nrows == 0 || A.nnz == 0) return;
-    hipLaunchKernelGGL(k_row_ids, dim3(grid_for(A.nrows, 256)), dim3(256), 0, s, A.rowptr.p, A.nrows, row);
+    if (A.nnz > 32 * A.nrows)
+        hipLaunchKernelGGL(k_row_ids_long, dim3(grid_for(A.nrows, 4)), dim3(256), 0, s, A.rowptr.p, A.nrows, row);
+    else
+        hipLaunchKernelGGL(k_row_ids, dim3(grid_for(A.nrows, 256)), dim3(256), 0, s, A.rowptr.p, A.nrows, row);
 }
 
 // Reciprocal areas and the list of wide rows of both directions; thread i takes
