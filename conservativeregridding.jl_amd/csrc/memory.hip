@@ -95,7 +95,8 @@ Cache &cache() {
 // The library call of this thread, and how a handle's buffers are released.
 struct Call {
     int depth = 0;
-    uint64_t id = 0;  // 0: no temporaries yet
+    uint64_t id = 0;     // 0: no temporaries yet
+    size_t pending = 0;  // its free blocks in state kCall
     bool checked = false;
     hipStream_t checked_stream = nullptr;  // not capturing
 };
@@ -154,6 +155,7 @@ void trim(Device &d, size_t most, uint64_t before, bool own, Lock &lock) {
     for (auto it : order) {
         if (d.kept <= most && it->second.stamp >= before) break;
         d.kept -= it->first;
+        if (it->second.state == kCall) --t_call.pending;
         out.push_back(*it);
         d.free.erase(it);
     }
@@ -192,12 +194,16 @@ void bound(Device &d, int index, Lock &lock) {
     if (dev != index) (void)hipSetDevice(dev);
 }
 
-// Each block this call freed in order on its streams.
+// Each block this call freed in order on its streams; f may give it another state.
 template <class F>
 void freed_by_call(Cache &c, F f) {
+    if (!t_call.pending) return;
     for (auto &dev : c.devices)
         for (auto &b : dev.second.free)
-            if (b.second.state == kCall && b.second.call == t_call.id) f(b.second);
+            if (b.second.state == kCall && b.second.call == t_call.id) {
+                f(b.second);
+                if (b.second.state != kCall) --t_call.pending;
+            }
 }
 
 // The call is over: synchronise the streams it freed temporaries on -- after a failure
@@ -237,7 +243,7 @@ CallScope::~CallScope() {
 
 void synchronise(hipStream_t s) {
     CR_HIP(hipStreamSynchronize(s));
-    if (!t_call.id) return;
+    if (!t_call.pending) return;
     Cache &c = cache();
     Lock lock(c.mu);
     freed_by_call(c, [&](Free &f) {
@@ -288,6 +294,7 @@ void *device_alloc(size_t bytes, Memory use, hipStream_t s) {
     }
     if (it != d.free.end()) {
         void *p = it->second.p;
+        if (it->second.state == kCall) --t_call.pending;
         c.live[p] = {it->first, dev, it->second.pool};
         d.kept -= it->first;
         d.free.erase(it);
@@ -324,6 +331,7 @@ void device_free(void *p, bool ordered, hipStream_t s) {
         State st = t_release;
         if (ordered) st = t_call.id ? kCall : s ? kUnknown : kNull;
         d.free.insert({b.bytes, Free{p, st, st == kCall ? t_call.id : 0, s, b.pool, d.frees}});
+        if (st == kCall) ++t_call.pending;
         c.live.erase(l);
         d.frees++;
         d.kept += b.bytes;
