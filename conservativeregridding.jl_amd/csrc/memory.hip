@@ -26,7 +26,9 @@
 //     wait, so calls that only need those stay ordered by their own stream;
 //   * kClean: nobody.
 //
-// No lock is held while the driver works.  The kept blocks are bounded (1/64 of the
+// The driver's allocations and frees are asked for in the relaxed capture mode: a
+// handle may be released (by a garbage collector) while some stream, its thread's own
+// too, is being captured.  No lock is held while the driver works.  The kept blocks are bounded (1/64 of the
 // device's memory: 4.5 GB): past that the oldest go back to the driver until a quarter
 // of the bound is free, and so do blocks that no allocation took over the last kKeep
 // frees, and all of them when an allocation fails.
@@ -112,8 +114,16 @@ size_t rounded(size_t bytes) {
     return (bytes + step - 1) / step * step;
 }
 
+// In its lifetime this thread's hipMalloc and hipFree disturb no capture.
+struct Relaxed {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // Wait for the device's pending work (the caller has made it current).  No lock held.
 bool device_wait() {
+    Relaxed r;
     void *p = nullptr;
     if (hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess) return true;
     (void)hipGetLastError();
@@ -165,6 +175,7 @@ void trim(Device &d, size_t most, uint64_t before, bool own, Lock &lock) {
         if (f.pool) (void)hipFreeAsync(f.p, f.state == kCall ? f.stream : nullptr);
         else (void)hipFree(f.p);
     };
+    Relaxed r;
     std::vector<std::pair<size_t, Free>> back;
     for (auto &b : out) {
         if (b.second.state == kUnknown) back.push_back(b);
@@ -301,7 +312,10 @@ void *device_alloc(size_t bytes, Memory use, hipStream_t s) {
         return p;
     }
     lock.unlock();
-    auto fresh = [&](void **p) { return ordered ? hipMallocAsync(p, want, s) : hipMalloc(p, want); };
+    auto fresh = [&](void **p) {
+        Relaxed r;
+        return ordered ? hipMallocAsync(p, want, s) : hipMalloc(p, want);
+    };
     void *p = nullptr;
     hipError_t e = fresh(&p);
     if (e == hipErrorOutOfMemory) {

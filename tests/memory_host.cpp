@@ -18,6 +18,7 @@ void note(const std::string &s) {
     std::lock_guard<std::mutex> l(g_mu);
     g_log += s + ";";
 }
+thread_local hipStreamCaptureMode t_mode = hipStreamCaptureModeGlobal;
 hipError_t get(void **p, size_t n) {
     std::unique_lock<std::mutex> l(g_mu);
     if (g_hold) {
@@ -51,9 +52,13 @@ const char *hipGetErrorString(hipError_t) { return "error"; }
 hipError_t hipMemGetInfo(size_t *a, size_t *t) { return *a = *t = g_total, hipSuccess; }
 hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t *, int) { return hipErrorUnknown; }
 hipError_t hipMemPoolSetAttribute(hipMemPool_t, hipMemPoolAttr, void *) { return hipSuccess; }
-hipError_t hipMalloc(void **p, size_t n) { return note("malloc"), get(p, n); }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *m) { return std::swap(*m, t_mode), hipSuccess; }
+void strict(const char *call) {  // these break captures of other modes
+    if (t_mode != hipStreamCaptureModeRelaxed) note(std::string(call) + " in another mode than relaxed");
+}
+hipError_t hipMalloc(void **p, size_t n) { return strict("malloc"), note("malloc"), get(p, n); }
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t s) { return note("malloc@" + name(s)), get(p, n); }
-hipError_t hipFree(void *p) { return note("free"), put(p); }
+hipError_t hipFree(void *p) { return strict("free"), note("free"), put(p); }
 hipError_t hipFreeAsync(void *p, hipStream_t s) { return note("free@" + name(s)), put(p); }
 hipError_t hipDeviceSynchronize(void) { return note("devicesync"), hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { return note("sync@" + name(s)), hipSuccess; }
